@@ -230,10 +230,11 @@ int rq_create(rq_ctx** out, int device, size_t budget) {
                               (trace_max_stack(v) - depth));
   }
   // counter slots (eager, then capture) + one trailing word of traversal error bits
-  const size_t cbytes = ((COUNTER_SLOTS + CAPTURE_SLOTS) * 2 + 1) * sizeof(uint32_t);
+  const size_t cwords = (size_t)(COUNTER_SLOTS + CAPTURE_SLOTS) * SLOT_WORDS;
+  const size_t cbytes = cwords * sizeof(uint64_t) + sizeof(uint32_t);
   int rc = ctx_alloc(c, cbytes, (void**)&c->counters);
   if (rc == RQ_OK) {
-    c->errword = c->counters + (COUNTER_SLOTS + CAPTURE_SLOTS) * 2;
+    c->errword = reinterpret_cast<uint32_t*>(c->counters + cwords);
     hipMemset(c->counters, 0, cbytes);
     c->gstack_bytes = gmax * 2 * sizeof(int32_t);
     rc = ctx_alloc(c, c->gstack_bytes, (void**)&c->gstack);
@@ -603,7 +604,6 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
     if (blocks == 0) return set_err(c, RQ_E_UNSUPPORTED, "variant too large for the scratch");
     a.gstack = reinterpret_cast<int32_t*>(c->scratch + NOALLOC_COUNTER_BYTES);
     a.counter = reinterpret_cast<unsigned long long*>(c->scratch);
-    a.ctr_base = 0ull;
     a.err = c->errword;
     a.grid = std::max(1u, std::min({c->trace_grid[variant], (uint32_t)blocks,
                                      (n + (uint32_t)blk - 1) / (uint32_t)blk}));
@@ -611,6 +611,7 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
     const SliceSchedule sched = slice_schedule(
         n, trace_chunk(n, a.grid * (uint32_t)blk / 64u, c->slice_closest));
     a.chunk = sched.chunk, a.chunk_small = sched.small, a.big_slices = sched.big;
+    a.segs = trace_segs(sched.total, a.grid * (uint32_t)blk / 64u, a.grid);
     a.sphere = b->scene && b->scene->kind == RQ_PRIM_SPHERE ? 1 : 0;
     const LaunchCtx lc{(hipStream_t)stream, nullptr};
     e = launch_counter_reset(lc, a.counter);
@@ -625,8 +626,8 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
   // takes a capture slot of its own, zeroed in the graph before the trace.
   const uint32_t slot = own_zero ? COUNTER_SLOTS + (c->capture_seq++ % CAPTURE_SLOTS)
                                  : next_counter_slot(c);
-  a.counter = reinterpret_cast<unsigned long long*>(c->counters) + slot;
-  a.ctr_base = own_zero ? 0ull : c->counter_base[slot];
+  a.counter = c->counters + (size_t)slot * SLOT_WORDS;
+  if (!own_zero) std::copy_n(c->counter_base[slot], TRACE_SEGS, a.ctr_base);
   a.err = c->errword;
   // the launch grid (launch_trace takes the same), its waves and slice size
   const uint32_t full_grid = any ? c->trace_grid_any[variant] : c->trace_grid[variant];
@@ -637,6 +638,7 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
       slice_schedule(n, trace_chunk(n, full_grid * (uint32_t)blk / 64u,
                                     any ? c->slice_any : c->slice_closest));
   a.chunk = sched.chunk, a.chunk_small = sched.small, a.big_slices = sched.big;
+  a.segs = trace_segs(sched.total, waves, a.grid);
   if (count_dev) a.chunk = any ? c->slice_any : c->slice_closest;  // the largest slice
   a.sphere = b->scene && b->scene->kind == RQ_PRIM_SPHERE ? 1 : 0;
   if (own_zero) {
@@ -645,9 +647,12 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
   }
   e = launch_trace(launch_ctx(c, stream), a, any, counted, variant);
   if (e != hipSuccess) return hip_err(c, e, "trace launch");
-  // the launch moves its slot's counter by its number of slices, or not at
-  // all when the waves' first slices cover it (RayStream)
-  if (!own_zero && sched.total > waves) c->counter_base[slot] += sched.total;
+  // the launch moves each of its slot's counters by the segment's number of
+  // slices, or not at all when its waves' first slices cover it (RayStream)
+  for (uint32_t q = 0; !own_zero && q < a.segs; ++q) {
+    const uint32_t tq = seg_total(q, a.segs, sched.total);
+    if (tq > seg_blocks(q, a.segs, a.grid) * ((uint32_t)blk / 64u)) c->counter_base[slot][q] += tq;
+  }
   return RQ_OK;
 }
 

@@ -23,10 +23,11 @@ struct rq_ctx {
   uint32_t refill_closest = 64, refill_any = 64;
   // largest wave slice of the ray stream, per query kind (trace_chunk)
   uint32_t slice_closest = rq::TRACE_RAY_CHUNK, slice_any = rq::TRACE_RAY_CHUNK;
-  // COUNTER_SLOTS 64-bit ray-stream counters (never reset), their values
-  // after the launches enqueued so far, and one word of traversal error bits
-  uint32_t* counters = nullptr;
-  uint64_t counter_base[rq::COUNTER_SLOTS] = {};
+  // counter slots: TRACE_SEGS 64-bit ray-stream counters each (SLOT_WORDS
+  // apart, never reset), their values after the launches enqueued so far, and
+  // one word of traversal error bits
+  unsigned long long* counters = nullptr;
+  uint64_t counter_base[rq::COUNTER_SLOTS][rq::TRACE_SEGS] = {};
   uint32_t* errword = nullptr;   // traversal error bits (stack deeper than provided)
   uint32_t counter_seq = 0;
   uint32_t capture_seq = 0;      // next capture slot (after the COUNTER_SLOTS eager ones)
@@ -86,8 +87,8 @@ void ctx_free(rq_ctx* c, void* p);
 LaunchCtx launch_ctx(rq_ctx* c, void* stream);
 // The next ray-stream counter slot (round robin over COUNTER_SLOTS). A launch
 // passes counter_base[slot] to its kernel and then adds the number of slices
-// its waves take from the counter (RayStream), so the slot's next launch
-// starts from the counter's value after this one.
+// its waves take from each counter (RayStream), so the slot's next launch
+// starts from the counters' values after this one.
 uint32_t next_counter_slot(rq_ctx* c);
 // The stack overflow area of launches on `stream`, allocated on a stream's
 // first traversal launch (not under graph capture: `may_alloc` false then);

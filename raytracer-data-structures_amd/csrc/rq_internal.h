@@ -124,6 +124,46 @@ __host__ __device__ inline SliceSchedule slice_schedule(uint32_t n, uint32_t chu
   return q;
 }
 
+// A launch whose slices outnumber its waves hands them out from TRACE_SEGS
+// counters, not one: device atomics on one word are served one after another,
+// 12.3 ns each (8.3 M rays that miss at the root, in 28,000 slices: 0.374 ms
+// from one counter, 0.101 ms from eight), so one counter sets the pace of the
+// small slices at the end of a launch (8.3 M shadow rays 1.01 -> 0.84 ms,
+// 8.4 M uniform rays 0.73 -> 0.66 ms). SLICE_GROUP consecutive slices at a
+// time are dealt to the segments in turn (each segment gets the same share of
+// an image's hard and easy parts, and the waves of one segment, which run on
+// one XCD when the blocks are dealt round robin, walk neighbouring rays); a
+// wave takes slices of its block's segment only (block b: segment b mod 8),
+// so no wave goes through the other counters at the end. A launch of fewer
+// slices than waves touches no counter: wave w traces slice w.
+constexpr uint32_t TRACE_SEGS = 8;
+constexpr uint32_t SLICE_GROUP = 8;
+constexpr uint32_t COUNTER_STRIDE = 32;  // 64-bit words between counters (256 bytes)
+constexpr uint32_t SLOT_WORDS = TRACE_SEGS * COUNTER_STRIDE;  // 64-bit words of a counter slot
+__host__ __device__ inline uint32_t trace_segs(uint32_t total, uint32_t waves, uint32_t grid) {
+  return total > waves && grid >= TRACE_SEGS ? TRACE_SEGS : 1u;
+}
+// Segment q's k-th slice among all.
+__host__ __device__ inline uint64_t seg_slice(uint32_t q, uint32_t segs, uint64_t k) {
+  return segs == 1u ? k : (k / SLICE_GROUP * TRACE_SEGS + q) * SLICE_GROUP + k % SLICE_GROUP;
+}
+// Slices of segment q among `total`.
+inline uint32_t seg_total(uint32_t q, uint32_t segs, uint32_t total) {
+  if (segs == 1u) return total;
+  const uint32_t round = TRACE_SEGS * SLICE_GROUP, rem = total % round, at = q * SLICE_GROUP;
+  return total / round * SLICE_GROUP + (rem > at ? (rem - at < SLICE_GROUP ? rem - at : SLICE_GROUP) : 0u);
+}
+// Blocks of segment q in a grid, and block b's segment and index in it.
+__host__ __device__ inline uint32_t seg_blocks(uint32_t q, uint32_t segs, uint32_t grid) {
+  return segs == 1u ? grid : (grid + TRACE_SEGS - 1u - q) / TRACE_SEGS;
+}
+__host__ __device__ inline uint32_t seg_of(uint32_t b, uint32_t segs) {
+  return segs == 1u ? 0u : b % TRACE_SEGS;
+}
+__host__ __device__ inline uint32_t seg_index(uint32_t b, uint32_t segs) {
+  return segs == 1u ? b : b / TRACE_SEGS;
+}
+
 // Build workspace (device), all sized for n primitives.
 struct BuildBuffers {
   uint32_t* codes = nullptr;      // n, primitive order
@@ -205,14 +245,17 @@ struct TraceArgs {
   uint32_t* tests;
   int32_t* gstack;
   uint32_t gdepth;      // overflow entries per thread
-  unsigned long long* counter;  // ray-stream counter of this launch's slot (never reset)
-  uint64_t ctr_base;    // its value when this launch starts
+  // ray-stream counters of this launch's slot (one per segment, never reset)
+  // and their values when this launch starts
+  unsigned long long* counter;
+  uint64_t ctr_base[TRACE_SEGS];
   uint32_t* err;        // set to 1 if a ray needed a deeper stack than provided
   uint32_t grid;        // blocks (persistent grid of the chosen variant)
   uint32_t refill_idle; // idle lanes in a wave before it refills from its slice
   uint32_t chunk;       // rays per slice taken from the global counter (the large slices)
   uint32_t chunk_small; // rays per slice after the first big_slices (standalone kernels)
   uint32_t big_slices;  // slices of `chunk` rays before the small ones
+  uint32_t segs;        // segments the slices are dealt to (trace_segs)
   int32_t sphere;       // leaves are spheres (centre, r, r*r) instead of triangles
   // Set when the ray count is known on the device only: the launch traces rays
   // [0, min(nrays, *nrays_dev)) and computes its slice schedule from that
@@ -230,15 +273,15 @@ void trace_variant_info(int v, int* block, int* depth, int* tstack, int* wide = 
 int trace_max_stack(int variant);  // total stack entries per lane (LDS + overflow)
 uint32_t trace_grid_blocks(int device, int variant, bool any);
 hipError_t launch_copy16(const LaunchCtx& lc, const void* src, void* dst, uint64_t bytes);
-// Zeroes one ray-stream counter with a one-thread kernel (a memset node would
-// not be safe to replay in a captured graph).
+// Zeroes a slot's ray-stream counters with a kernel (a memset node would not
+// be safe to replay in a captured graph).
 hipError_t launch_counter_reset(const LaunchCtx& lc, unsigned long long* counter);
 // Scratch of the allocation-free closest-hit entry: NOALLOC_SCRATCH_BYTES per
 // device (a static device array), its first NOALLOC_COUNTER_BYTES the
-// counter, the rest the overflow area; the launch grid is capped so that the
+// counters, the rest the overflow area; the launch grid is capped so that the
 // overflow area of every thread fits.
 constexpr size_t NOALLOC_SCRATCH_BYTES = 64ull << 20;
-constexpr size_t NOALLOC_COUNTER_BYTES = 256;
+constexpr size_t NOALLOC_COUNTER_BYTES = SLOT_WORDS * sizeof(uint64_t);
 // The device address of the scratch on the current device.
 hipError_t noalloc_scratch_address(void** ptr);
 

@@ -15,30 +15,32 @@ namespace rq {
 
 // Where a wave takes its slices of the ray stream from. The standalone kernels
 // number the slices (a.chunk rays each for the first a.big_slices, then
-// a.chunk_small): wave w starts on slice w (no atomic), and takes slice
-// waves + k from the k-th add to a 64-bit counter that is never reset
-// (k = counter add - base). When the waves' first slices cover the launch no
-// wave touches the counter; otherwise each wave makes exactly one failing add
-// and every later slice is one add, so the launch moves the counter by
-// exactly its number of slices, which the host adds to the base of the
-// slot's next launch. The batch kernel counts rays from 0 in LDS.
+// a.chunk_small) and deal them to segments (seg_slice): the w-th wave of a
+// segment starts on the segment's slice w (no atomic), and takes its slice
+// waves + k from the k-th add to the segment's 64-bit counter that is never
+// reset (k = counter add - TraceArgs::ctr_base). When the waves' first slices cover the
+// segment no wave touches the counter; otherwise each wave makes exactly one
+// failing add and every later slice is one add, so the launch moves the
+// counter by exactly the segment's number of slices, which the host adds to
+// the base of the slot's next launch. The batch kernel counts rays from 0 in
+// LDS.
 struct RayStream {
   uint32_t* ctr32 = nullptr;            // counter of rays from 0 (batch, LDS), or
-  unsigned long long* ctr64 = nullptr;  // the slot's monotonic slice counter
-  uint64_t base = 0;                    // ctr64 at launch
-  uint32_t wave = 0, waves = 0;         // this wave's index, waves in the grid
+  unsigned long long* ctr64 = nullptr;  // the segment's monotonic slice counter
+  uint32_t seg = 0, segs = 1;           // this wave's segment, segments of the launch
+  uint32_t wave = 0, waves = 0;         // this wave's index, waves in the segment
 };
-// The launch's ray count and slice sizes, in scalar registers: from the
-// kernel arguments, or computed here from a count read from device memory
+// The launch's ray count, slice sizes and segments, in scalar registers: from
+// the kernel arguments, or computed here from a count read from device memory
 // (TraceArgs::nrays_dev).
 struct Schedule {
-  uint32_t n, chunk, small, big;
+  uint32_t n, chunk, small, big, segs;
 };
-__device__ inline Schedule schedule_of(const TraceArgs& a, uint32_t waves) {
-  if (!a.nrays_dev) return Schedule{a.nrays, a.chunk, a.chunk_small, a.big_slices};
+__device__ inline Schedule schedule_of(const TraceArgs& a, uint32_t waves, uint32_t grid) {
+  if (!a.nrays_dev) return Schedule{a.nrays, a.chunk, a.chunk_small, a.big_slices, a.segs};
   const uint32_t n = min(a.nrays, __builtin_amdgcn_readfirstlane(*a.nrays_dev));
   const SliceSchedule q = slice_schedule(n, trace_chunk(n, waves, a.chunk));
-  return Schedule{n, q.chunk, q.small, q.big};
+  return Schedule{n, q.chunk, q.small, q.big, trace_segs(q.total, waves, grid)};
 }
 __device__ inline uint32_t slice_begin(const Schedule& a, uint64_t s) {
   return s <= a.big ? (uint32_t)min(s * a.chunk, (uint64_t)a.n)
@@ -206,14 +208,14 @@ __device__ inline int4 link_load(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
 constexpr int ROWS_SMALL = 0, ROWS_BIG = 1, ROWS_ANY = 2;
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
           int ROWS, class Src>
-__device__ inline void trace_loop_impl(const TraceArgs& a, const RayStream& rs, int32_t* s_node,
-                                       float* s_tn, uint32_t gtid, uint32_t gstride, Src* src) {
+__device__ inline void trace_loop_impl(const TraceArgs& a, const Schedule& sc, const RayStream& rs,
+                                       int32_t* s_node, float* s_tn, uint32_t gtid,
+                                       uint32_t gstride, Src* src) {
   static_assert(!(WIDE && COUNT), "counted traversal walks the binary nodes");
   const bool big = ROWS == ROWS_ANY ? a.nprims > WIDE_UNIFORM_MAX_NODES : ROWS == ROWS_BIG;
   const int tid = threadIdx.x, lane = tid & 63;
   const uint64_t lt = (1ull << lane) - 1ull;
   const int max_sp = DEPTH + (int)a.gdepth;
-  const Schedule sc = schedule_of(a, (uint32_t)rs.waves);
   const float slack = (SPHERES && a.sphere) ? SPHERE_SLACK : SLAB_SLACK;
 
   RayState r{};  // lanes that never take a ray still read their (unused) octant
@@ -223,7 +225,8 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const RayStream& rs, 
   uint32_t cnext = 0, cend = 0;
   bool wave_out = false;  // the global stream is exhausted for this wave
   if (rs.ctr64) {
-    cnext = slice_begin(sc, rs.wave), cend = slice_begin(sc, rs.wave + 1ull);
+    const uint64_t s = seg_slice(rs.seg, rs.segs, rs.wave);
+    cnext = slice_begin(sc, s), cend = slice_begin(sc, s + 1);
     wave_out = cnext >= sc.n;
   }
   uint32_t ray = 0;
@@ -294,15 +297,17 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const RayStream& rs, 
         }
         cnext = b, cend = e;
       } else if (cnext >= cend) {
-        if (rs.ctr64 && slice_begin(sc, rs.waves) >= sc.n) {  // first slices cover all
+        if (rs.ctr64 && slice_begin(sc, seg_slice(rs.seg, rs.segs, rs.waves)) >= sc.n) {
+          // first slices cover all
           wave_out = true;
           break;
         }
         uint64_t s = 0;
         if (lane == 0)
-          s = rs.ctr64 ? atomicAdd(rs.ctr64, 1ull) - rs.base + rs.waves
+          s = rs.ctr64 ? atomicAdd(rs.ctr64, 1ull) - a.ctr_base[rs.seg] + rs.waves
                        : atomicAdd(rs.ctr32, sc.chunk);
         s = __shfl(s, 0, 64);
+        if (rs.ctr64) s = seg_slice(rs.seg, rs.segs, s);
         const uint32_t b = rs.ctr64 ? slice_begin(sc, s) : (uint32_t)min(s, (uint64_t)sc.n);
         if (b >= sc.n) {
           wave_out = true;
@@ -502,8 +507,9 @@ template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES 
 __device__ inline void trace_loop(const TraceArgs& a, const RayStream& rs, int32_t* s_node,
                                   float* s_tn, uint32_t gtid, uint32_t gstride,
                                   Src* src = nullptr) {
+  const Schedule sc{a.nrays, a.chunk, 0u, 0u, 1u};
   trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_ANY, Src>(
-      a, rs, s_node, s_tn, gtid, gstride, src);
+      a, sc, rs, s_node, s_tn, gtid, gstride, src);
 }
 // A path per row form, chosen once per launch (the query kernels: one tree).
 // Below 2^25 nodes every row, the link row included, is a load at a 32-bit
@@ -511,14 +517,15 @@ __device__ inline void trace_loop(const TraceArgs& a, const RayStream& rs, int32
 // hit kernels also drop their register spills.
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES = true,
           bool WIDE = false>
-__device__ inline void trace_loop_split(const TraceArgs& a, const RayStream& rs, int32_t* s_node,
-                                        float* s_tn, uint32_t gtid, uint32_t gstride) {
+__device__ inline void trace_loop_split(const TraceArgs& a, const Schedule& sc,
+                                        const RayStream& rs, int32_t* s_node, float* s_tn,
+                                        uint32_t gtid, uint32_t gstride) {
   if (WIDE && a.nprims > WIDE_UNIFORM_MAX_NODES)
     trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_BIG, NoSlices>(
-        a, rs, s_node, s_tn, gtid, gstride, nullptr);
+        a, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
   else
     trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_SMALL, NoSlices>(
-        a, rs, s_node, s_tn, gtid, gstride, nullptr);
+        a, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
 }
 
 }  // namespace rq

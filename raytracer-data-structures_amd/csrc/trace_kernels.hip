@@ -2,8 +2,8 @@
 // running trace_loop (trace_device.h), a table of kernel variants for the
 // autotuner, and the launcher.
 //
-// Kernel shape: persistent waves take slices of the ray stream from a global
-// counter; when enough lanes have finished (wave ballot), the wave refills the
+// Kernel shape: persistent waves take slices of the ray stream from their
+// segment's counter; when enough lanes have finished (wave ballot), the wave refills the
 // idle lanes from its slice (ray compaction), so long rays do not hold a wave
 // of finished lanes. The per-lane stack lives in LDS ([depth][lane],
 // conflict-free) and spills to a global [depth][thread] area past the LDS
@@ -21,18 +21,21 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES > 0
 void k_trace(TraceArgs a) {
   __shared__ int32_t s_node[DEPTH * BLOCK];
   __shared__ float s_tn[TSTACK ? DEPTH * BLOCK : 1];
+  constexpr uint32_t WPB = BLOCK / 64;
+  const Schedule sc = schedule_of(a, gridDim.x * WPB, gridDim.x);
   RayStream rs;
-  rs.ctr64 = a.counter;
-  rs.base = a.ctr_base;
-  rs.wave = (blockIdx.x * BLOCK + threadIdx.x) >> 6;
-  rs.waves = gridDim.x * (BLOCK / 64);
+  rs.segs = sc.segs;
+  rs.seg = seg_of(blockIdx.x, sc.segs);
+  rs.ctr64 = a.counter + rs.seg * COUNTER_STRIDE;
+  rs.wave = seg_index(blockIdx.x, sc.segs) * WPB + (threadIdx.x >> 6);
+  rs.waves = seg_blocks(rs.seg, sc.segs, gridDim.x) * WPB;
   trace_loop_split<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE>(
-      a, rs, s_node, s_tn, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK);
+      a, sc, rs, s_node, s_tn, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK);
 }
 
 // Device scratch of the allocation-free closest-hit entry
-// (rq_closest_hit_noalloc): the launch's ray-stream counter in the first 256
-// bytes, then the traversal stack overflow area ([depth][thread] pairs). One
+// (rq_closest_hit_noalloc): the launch's ray-stream counters in the first
+// NOALLOC_COUNTER_BYTES, then the traversal stack overflow area ([depth][thread] pairs). One
 // copy per device, held from module load until the process ends; its address
 // comes from hipGetSymbolAddress (noalloc_scratch_address), never from the
 // array's name in host code. Calls that overlap on one device share it and
@@ -40,7 +43,7 @@ void k_trace(TraceArgs a) {
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 __global__ __launch_bounds__(64) void k_counter_reset(unsigned long long* ctr) {
-  if (threadIdx.x == 0) *ctr = 0ull;
+  if (threadIdx.x < TRACE_SEGS) ctr[threadIdx.x * COUNTER_STRIDE] = 0ull;
 }
 
 typedef void (*TraceFn)(TraceArgs);
