@@ -229,10 +229,10 @@ int rq_any_hit_counted(rq_ctx* ctx, const rq_bvh* b, const rq_rays* rays, uint32
  * stack entries carry their entry distance (closest hit skips entries
  * beyond the best hit when popped), and the node format walked: binary
  * (64-byte nodes, two children) or wide (the binary tree collapsed into
- * 128-byte 4-child nodes, written by every rq_build_lbvh / rq_rebuild_lbvh /
+ * 64-byte 4-child nodes, written by every rq_build_lbvh / rq_rebuild_lbvh /
  * rq_bvh_load), and the waves per SIMD the closest-hit and any-hit kernels
- * are compiled for (0: as many as their registers allow; 6: registers
- * capped for six, which hides more of the dependent node fetches). Results
+ * promise (6: their registers and LDS stack leave room for six or more,
+ * which hides more of the dependent node fetches; 0: no promise). Results
  * are identical for all. A new context uses wide variants (9 for closest
  * hit, 14 for any hit, refill 64, slices of 1024). */
 typedef struct {

@@ -299,8 +299,8 @@ constexpr int batch_lds_words(bool build, int depth, bool tstack) {
 // batch run (WIDE: walking the 4-wide nodes of the widen phase), or as the
 // continuous-batching step of the serving loop (binary nodes). WAVES waves
 // per SIMD cap the registers: the build phases are written to fit 8 (lean
-// 8-key sort tiles, descriptors loaded per phase); the 4-wide walk fits 6
-// (79 VGPRs) where its LDS stack allows, the binary walk 7-8.
+// 8-key sort tiles, descriptors loaded per phase); the 4-wide walk fits 8
+// (63 VGPRs) where its LDS stack allows, the binary walk 7-8.
 enum KernelMode { KM_BUILD, KM_TRACE };
 template <int DEPTH, bool TSTACK, int WAVES, KernelMode MODE, bool WIDE, bool WAVE_ITEMS = WIDE>
 __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_batch(
@@ -485,7 +485,7 @@ constexpr int kNumBuildVariants = sizeof(kBuild) / sizeof(kBuild[0]);
 // Trace kernels of a batch run (4-wide walk): the batch configurations.
 const BatchVariant kBatchVariants[] = {
     {24, false, k_batch<24, false, 6, KM_TRACE, true>},
-    {16, false, k_batch<16, false, 6, KM_TRACE, true>},
+    {16, false, k_batch<16, false, 8, KM_TRACE, true>},
     {32, false, k_batch<32, false, 4, KM_TRACE, true>},
     {12, true, k_batch<12, true, 6, KM_TRACE, true>},
     {28, false, k_batch<28, false, 5, KM_TRACE, true>},
@@ -497,7 +497,7 @@ const BatchVariant kServeVariants[] = {
     {8, true, k_batch<8, true, 7, KM_TRACE, false>},     {10, true, k_batch<10, true, 7, KM_TRACE, false>},
     {16, false, k_batch<16, false, 8, KM_TRACE, false>}, {8, true, k_batch<8, true, 8, KM_TRACE, false>},
     {16, false, k_batch<16, false, 5, KM_TRACE, true, false>},
-    {16, false, k_batch<16, false, 6, KM_TRACE, true, false>}};
+    {16, false, k_batch<16, false, 8, KM_TRACE, true, false>}};
 constexpr int kServeWideFirst = 6;
 constexpr int kNumBatchVariants = sizeof(kBatchVariants) / sizeof(kBatchVariants[0]);
 constexpr int kNumServeVariants = sizeof(kServeVariants) / sizeof(kServeVariants[0]);

@@ -538,10 +538,8 @@ __device__ inline void leaf_record(const BuildView& v, uint32_t k, TriRec& tr, f
 // ---- 4-wide collapse ------------------------------------------------------------
 // The wide node of binary internal node i holds, in binary order, for each
 // child c of i: c's box if c is a leaf (one slot, the next one unused), else
-// the boxes of c's two children (two slots). Boxes are copied exactly, so a
-// slab test against a wide slot is the test the binary traversal makes
-// against the same subtree. Every internal node gets its wide node (only the
-// root and even-depth nodes are reached from the root).
+// the boxes of c's two children (two slots). Every internal node gets its
+// wide node (only the root and even-depth nodes are reached from the root).
 struct WideSlots {
   float lo[4][3], hi[4][3];
   int32_t link[4];
@@ -551,15 +549,50 @@ __device__ inline void wide_empty(WideSlots& w, int k) {
   w.hi[k][0] = w.hi[k][1] = w.hi[k][2] = -INFINITY;
   w.link[k] = 0;
 }
+// One axis of the record's grid: the slots' planes on base + (1024 + q) * step.
+// The step is the slots' extent over 252 (two steps to spare on a byte), at
+// least 2^-21 of the largest coordinate, so that the rounding of the base
+// (2^-24 of a magnitude of at most 2^21 + 1024 steps) stays within an eighth
+// of a step, and 2^-60. The base lies one step further down, so no lo plane
+// needs a negative q. The quotient (1024 + q) is computed with an error below
+// 2^-12 of a step and rounded outward by 2^-9 more, so the plane the walk
+// computes contains the exact one by over 2^-10 of a step: the walk's own
+// rounding is below that for an origin within the grid, and relative to the
+// distance (covered by its slack) for one further away. An extent or a
+// coordinate of 2^100 or more (or one that is not finite) makes the step NaN,
+// and the walk reads a NaN plane as a box that reaches everywhere.
+__device__ inline void wide_axis(const float* lo, const float* hi, float* base, float* step,
+                                 uint32_t* qlo, uint32_t* qhi) {
+  const float l = fminf(fminf(lo[0], lo[1]), fminf(lo[2], lo[3]));
+  const float h = fmaxf(fmaxf(hi[0], hi[1]), fmaxf(hi[2], hi[3]));
+  const float ext = h - l, mag = fmaxf(fabsf(l), fabsf(h));
+  const bool sane = ext < 0x1p100f && mag < 0x1p100f;
+  const float s =
+      sane ? fmaxf(fmaxf(ext * (1.0f / 252.0f), mag * 0x1p-21f), 0x1p-60f) : NAN;
+  const float b = sane ? l - (WIDE_Q0 + 1.0f) * s : 0.0f;
+  const float rs = 1.0f / s;
+  uint32_t ql = 0u, qh = 0u;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float a = floorf((lo[k] - b) * rs - (WIDE_Q0 + 0x1p-9f));
+    const float c = ceilf((hi[k] - b) * rs - (WIDE_Q0 - 0x1p-9f));
+    ql |= (uint32_t)fminf(fmaxf(a, 0.0f), 255.0f) << (8 * k);
+    qh |= (uint32_t)fminf(fmaxf(c, 0.0f), 255.0f) << (8 * k);
+  }
+  *base = b, *step = s, *qlo = ql, *qhi = qh;
+}
 __device__ inline void wide_store(WideNode* W, const WideSlots& w) {
-  W->lox = make_float4(w.lo[0][0], w.lo[1][0], w.lo[2][0], w.lo[3][0]);
-  W->hix = make_float4(w.hi[0][0], w.hi[1][0], w.hi[2][0], w.hi[3][0]);
-  W->loy = make_float4(w.lo[0][1], w.lo[1][1], w.lo[2][1], w.lo[3][1]);
-  W->hiy = make_float4(w.hi[0][1], w.hi[1][1], w.hi[2][1], w.hi[3][1]);
-  W->loz = make_float4(w.lo[0][2], w.lo[1][2], w.lo[2][2], w.lo[3][2]);
-  W->hiz = make_float4(w.hi[0][2], w.hi[1][2], w.hi[2][2], w.hi[3][2]);
-  W->link = make_int4(w.link[0], w.link[1], w.link[2], w.link[3]);
-  W->pad = make_int4(0, 0, 0, 0);
+  float lo[3][4], hi[3][4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int x = 0; x < 3; ++x) lo[x][k] = w.lo[k][x], hi[x][k] = w.hi[k][x];
+  WideNode n;
+  wide_axis(lo[0], hi[0], &n.base.x, &n.base.w, &n.lox, &n.hix);
+  wide_axis(lo[1], hi[1], &n.base.y, &n.step_y, &n.loy, &n.hiy);
+  wide_axis(lo[2], hi[2], &n.base.z, &n.step_z, &n.loz, &n.hiz);
+  n.link = make_int4(w.link[0], w.link[1], w.link[2], w.link[3]);
+  *W = n;
 }
 // From the finished binary node records in global memory.
 __device__ inline void widen_global(const BuildBuffers& B, uint32_t i) {

@@ -7,6 +7,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 #include <map>
 #include <set>
 #include <mutex>
@@ -172,7 +173,7 @@ int bvh_alloc(rq_ctx* c, rq_bvh* b, uint32_t n) {
                  64 * ni,
                  48 * nn,
                  4 * nn,
-                 128 * ni,
+                 sizeof(WideNode) * ni,
                  24 * nn,
                  24 * nn,
                  24 * (size_t)((nn + REFIT_CHUNK_MIN - 1) / REFIT_CHUNK_MIN)};
@@ -534,17 +535,57 @@ int rq_bvh_export_wide(rq_ctx* c, const rq_bvh* b, float* boxes, int32_t* links)
   if (b->n < 2) return RQ_OK;
   const size_t ni = b->n - 1;
   std::vector<WideNode> w(ni);
+  std::vector<NodeRec> nodes(ni);
   hipError_t e = hipDeviceSynchronize();
   if (e == hipSuccess) e = hipMemcpy(w.data(), b->B.wide, ni * sizeof(WideNode), hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpy(nodes.data(), b->B.nodes, ni * sizeof(NodeRec), hipMemcpyDeviceToHost);
   if (e != hipSuccess) return hip_err(c, e, "wide export");
+  // The records hold the links and the boxes on a grid; the boxes handed out
+  // are the exact ones they stand for (the binary records'), once each
+  // record's box is found to contain its own.
+  const float inf = std::numeric_limits<float>::infinity();
   for (size_t i = 0; i < ni; ++i) {
-    const float* q = &w[i].lox.x;  // lox, hix, loy, hiy, loz, hiz (4 slots each)
-    for (int k = 0; k < 4 && boxes; ++k) {
-      float* o = boxes + 24 * i + 6 * k;
-      o[0] = q[k], o[1] = q[8 + k], o[2] = q[16 + k];
-      o[3] = q[4 + k], o[4] = q[12 + k], o[5] = q[20 + k];
+    float ex[4][6];
+    int32_t want[4] = {0, 0, 0, 0};
+    for (int s = 0; s < 4; ++s)
+      for (int x = 0; x < 3; ++x) ex[s][x] = inf, ex[s][3 + x] = -inf;
+    auto slot = [&](const NodeRec& q, int side, float* o) {
+      const float4 &lo = side ? q.lo1 : q.lo0, &hi = side ? q.hi1 : q.hi0;
+      o[0] = lo.x, o[1] = lo.y, o[2] = lo.z, o[3] = hi.x, o[4] = hi.y, o[5] = hi.z;
+    };
+    auto link = [](const NodeRec& q, int side) {
+      int32_t l;
+      std::memcpy(&l, side ? &q.hi0.w : &q.lo0.w, 4);
+      return l;
+    };
+    for (int side = 0; side < 2; ++side) {
+      const int32_t ch = link(nodes[i], side);
+      if (ch < 0) {
+        want[2 * side] = ch;
+        slot(nodes[i], side, ex[2 * side]);
+      } else if ((size_t)ch < ni) {
+        for (int g = 0; g < 2; ++g) {
+          want[2 * side + g] = link(nodes[ch], g);
+          slot(nodes[ch], g, ex[2 * side + g]);
+        }
+      }
     }
-    if (links) std::memcpy(links + 4 * i, &w[i].link, 16);
+    const WideNode& q = w[i];
+    const int32_t got[4] = {q.link.x, q.link.y, q.link.z, q.link.w};
+    const double base[3] = {q.base.x, q.base.y, q.base.z}, step[3] = {q.base.w, q.step_y, q.step_z};
+    const uint32_t ql[3] = {q.lox, q.loy, q.loz}, qh[3] = {q.hix, q.hiy, q.hiz};
+    for (int s = 0; s < 4; ++s) {
+      if (got[s] != want[s])
+        return set_err(c, RQ_E_HIP, "wide node %zu slot %d: link %d, not %d", i, s, got[s], want[s]);
+      for (int x = 0; x < 3 && want[s]; ++x) {
+        const double l = base[x] + (WIDE_Q0 + (ql[x] >> (8 * s) & 255u)) * step[x];
+        const double h = base[x] + (WIDE_Q0 + (qh[x] >> (8 * s) & 255u)) * step[x];
+        if (l > ex[s][x] || h < ex[s][3 + x])  // (a NaN step is a box everywhere)
+          return set_err(c, RQ_E_HIP, "wide node %zu slot %d: its box does not hold the exact one", i, s);
+      }
+      if (boxes) std::memcpy(boxes + 24 * i + 6 * s, ex[s], sizeof ex[s]);
+    }
+    if (links) std::memcpy(links + 4 * i, got, sizeof got);
   }
   return RQ_OK;
 }

@@ -35,16 +35,30 @@ static_assert(sizeof(TriRec) == 48, "triangle record is 48 bytes");
 // 4-wide node: the binary LBVH collapsed two levels at a time. The wide node
 // of a binary internal node i (kept at index i; every internal node has one,
 // the walk reaches the root and the nodes at even depth) holds the boxes of
-// i's grandchildren, or of a child that is a leaf, as four child slots in SoA
-// order, one 128-byte record per visit. Links follow the binary convention
-// (>= 0 wide node = binary index, < 0 leaf ~k); an unused slot has link 0
-// (the root is never a child) and an empty box (lo +inf, hi -inf).
-struct alignas(128) WideNode {
-  float4 lox, hix, loy, hiy, loz, hiz;
+// i's grandchildren, or of a child that is a leaf, in four child slots, one
+// 64-byte record per visit. Links follow the binary convention (>= 0 wide
+// node = binary index, < 0 leaf ~k); an unused slot has link 0 (the root is
+// never a child).
+// The boxes are kept on a grid of the node's own, a byte per plane (one byte
+// of lo / hi per slot): plane = base + (1024 + q) * step per axis, every lo
+// plane at or below the exact one and every hi plane at or above it, by at
+// least 2^-10 of a step (wide_store). They only cull, so answers do not
+// depend on them. A visit is bound by the vector memory path as much as by
+// arithmetic: with the exact boxes (seven 16-byte loads of a 128-byte record)
+// the loads of the camera rays' walk held the L1's return path 77 % of the
+// time and their 28 registers kept the kernels at six waves per SIMD; a grid
+// record is four loads and sixteen registers. (1024 + q is the half-precision
+// number whose low byte is q: a byte permute makes two planes at a time, and
+// the mixed-precision multiply-add reads them without a conversion.)
+struct alignas(64) WideNode {
+  float4 base;  // base x, y, z, step x
+  float step_y, step_z;
+  uint32_t lox, hix;  // byte s: slot s's plane
+  uint32_t loy, hiy, loz, hiz;
   int4 link;
-  int4 pad;
 };
-static_assert(sizeof(WideNode) == 128, "wide node record is 128 bytes");
+static_assert(sizeof(WideNode) == 64, "wide node record is 64 bytes");
+constexpr float WIDE_Q0 = 1024.0f;
 
 // Radix sort tiling (onesweep): WAVES*64 threads, ITEMS keys per thread.
 // The standalone build sorts 16 keys per thread; the batch kernel, whose
@@ -82,9 +96,9 @@ constexpr int TRACE_MAX_STACK = 64;
 constexpr int TRACE_MAX_STACK_WIDE = 96;
 constexpr int TRACE_MIN_LDS_DEPTH = 12;
 constexpr int TRACE_MAX_VARIANTS = 24;
-// Variants a new context uses: the 4-wide walk, 128 threads and 24 LDS entries
-// for closest hit, 256 threads and 16 entries for any hit (the fastest or
-// within a few per cent on camera, shadow, bounce and uniform random rays).
+// Variants a new context uses: the 4-wide walk with 16 LDS entries, 128
+// threads for closest hit and 256 for any hit (eight waves per SIMD; the
+// fastest on camera, shadow, bounce and uniform random rays).
 constexpr int TRACE_DEFAULT_CLOSEST = 9;
 constexpr int TRACE_DEFAULT_ANY = 14;
 constexpr int COUNTER_SLOTS = 64;
@@ -98,14 +112,17 @@ constexpr uint32_t TRACE_RAY_CHUNK = 1024;      // default largest wave slice of
 constexpr uint32_t TRACE_RAY_CHUNK_MAX = 4096;  // largest that may be configured
 
 // Rays per wave slice for a launch of n rays over `waves` persistent waves:
-// `largest` (a power of two, 64..4096) when every wave gets at least two full
-// slices, halved down to one ray per lane (64) for smaller launches, so that
-// a small batch still spreads over as many waves as it can fill (each slice
-// after a wave's first costs one device atomic on the launch's counter).
+// `largest` (a power of two, 64..4096) when every wave gets at least eight
+// full slices, halved down to one ray per lane (64) for smaller launches. A
+// slice of hard rays (an object's silhouette: 90 node visits a ray where 20
+// are usual) can hold a wave past the end of all others: at two slices a wave
+// (512 rays) 1 % of the waves ended 1.5 times later than the rest on 8.3 M
+// camera rays (1.06 ms against 0.75 at 128 rays). Each slice after a wave's
+// first costs one device atomic.
 __host__ __device__ inline uint32_t trace_chunk(uint32_t n, uint32_t waves,
                                                 uint32_t largest = TRACE_RAY_CHUNK) {
   uint32_t c = largest;
-  while (c > 64 && (uint64_t)n < 2ull * c * waves) c >>= 1;
+  while (c > 64 && (uint64_t)n < 8ull * c * waves) c >>= 1;
   return c;
 }
 // Slice schedule of a standalone launch: slices of `chunk` rays over the

@@ -179,7 +179,7 @@ struct rq_server {
   int32_t* gstack = nullptr;
   uint32_t gdepth = 0, grid = 0;
   // trace kernel of the steps (serve_variant_info): the 4-wide walk, LDS
-  // stack depth 16, 6 waves per SIMD (against the binary walk, serving 64
+  // stack depth 16, 8 waves per SIMD (at 6, against the binary walk, serving 64
   // meshes of 10k-2M triangles at 2000 requests/s: p50 1.40 -> 1.15 ms,
   // saturation 2.90 -> 3.16 Grays/s)
   int variant = 7;

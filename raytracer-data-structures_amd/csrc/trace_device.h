@@ -48,6 +48,11 @@ __device__ inline uint32_t slice_begin(const Schedule& a, uint64_t s) {
                                     (uint64_t)a.n);
 }
 
+// This lane's rank among the lanes of a wave mask.
+__device__ inline uint32_t rank_in(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 // A wave takes its slices from the RayStream unless the caller gives a slice
 // source: Src::next(b, e) returns the wave's next slice [b, e) of a.rays, or
 // false when the wave is to finish its rays and return. It is called with
@@ -59,9 +64,9 @@ struct NoSlices {
 
 struct RayState {
   float ox, oy, oz, dx, dy, dz;
-  float ix, iy, iz;  // 1/d
+  float ix, iy, iz;  // 1/d (the wide walk: of at most 2^100, wide_inv)
   bool sx, sy, sz;   // sign bit of 1/d: the near plane of that axis is hi
-  float tmin, tmax;
+  float tmin;
 };
 
 // Relative slack on the far bound: a triangle's rounded Möller–Trumbore t can
@@ -75,11 +80,10 @@ constexpr float SLAB_SLACK = 1.000030517578125f;
 // hit with a 2^-9 relative slack keeps every box whose sphere's computed t
 // can still beat the best hit.
 constexpr float SPHERE_SLACK = 1.001953125f;
-// Wide walk: the near / far rows are loaded at byte offsets node * 128 + row
-// held in 32 bits (a scalar base plus one vector offset; the row is scalar
-// when the wave's octant is uniform, per lane otherwise), so the node count
-// must stay below 2^25; larger trees select the rows per value.
-constexpr uint32_t WIDE_UNIFORM_MAX_NODES = 1u << 25;
+// Wide walk: a record is loaded at a byte offset node * 64 held in 32 bits (a
+// scalar base plus one vector offset) while the node count stays at or below
+// this; larger trees take 64-bit addresses.
+constexpr uint32_t WIDE_SMALL_MAX_NODES = 1u << 25;
 
 // Slab test (same operations and order as the oracle): near/far planes by
 // the sign of 1/d, t = (plane - o) * (1/d). A zero direction component gives
@@ -95,16 +99,29 @@ __device__ inline bool slab(const float4& lo, const float4& hi, const RayState& 
   return tn <= tf * slack;
 }
 
-// Slot test of a wide node on pre-selected near / far planes: the same
-// operations as slab(), so a slot culls exactly where the binary walk culls
-// the same box.
-__device__ inline bool slab_w(float nx, float ny, float nz, float fx, float fy, float fz,
-                              const RayState& r, float thi, float slack, float& tn) {
-  const float an = (nx - r.ox) * r.ix, bn = (ny - r.oy) * r.iy, cn = (nz - r.oz) * r.iz;
-  const float af = (fx - r.ox) * r.ix, bf = (fy - r.oy) * r.iy, cf = (fz - r.oz) * r.iz;
-  tn = fmaxf(fmaxf(an, bn), fmaxf(cn, r.tmin));
-  const float tf = fminf(fminf(af, bf), fminf(cf, thi));
-  return tn <= tf * slack;
+// The wide walk's 1/d: finite, so that a plane on the grid is never inf - inf
+// for a ray parallel to an axis. At 2^100 a plane of the grid, which lies
+// outside the exact box by over 2^-10 of a step of at least 2^-60, is still
+// further than 2^30 on its side of an origin on or inside the exact box.
+__device__ inline float wide_inv(float d) {
+  return copysignf(fminf(fabsf(1.0f / d), 0x1p100f), d);
+}
+// Four planes of a wide node on one axis, a byte each in q: distances
+// (base + (1024 + q) * step - o) / d as (1024 + q) * si + bi with
+// si = step / d and bi = (base - o) / d.
+typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
+__device__ inline float4 wide_planes(uint32_t q, float si, float bi) {
+  // 0x6400 | q is the half-precision 1024 + q
+  const Half2 a = __builtin_bit_cast(Half2, __builtin_amdgcn_perm(0x64646464u, q, 0x04010400u));
+  const Half2 b = __builtin_bit_cast(Half2, __builtin_amdgcn_perm(0x64646464u, q, 0x04030402u));
+  return make_float4(__builtin_fmaf((float)a[0], si, bi), __builtin_fmaf((float)a[1], si, bi),
+                     __builtin_fmaf((float)b[0], si, bi), __builtin_fmaf((float)b[1], si, bi));
+}
+// Slot test of a wide node: the last axis joins the interval [tn, tf] of the
+// others; eps is the relative slack on the far bound.
+__device__ inline bool slot_hit(float n, float f, float eps, float& tn, float tf) {
+  tn = fmaxf(tn, n), tf = fminf(tf, f);
+  return tn <= __builtin_fmaf(fabsf(tf), eps, tf);
 }
 
 __device__ inline void cas_pair(uint32_t& ka, int32_t& ca, uint32_t& kb, int32_t& cb) {
@@ -123,8 +140,10 @@ __device__ inline void cas_hit(bool& ha, int32_t& ca, bool& hb, int32_t& cb) {
 }
 
 // Möller–Trumbore, main.cpp:137-162 (v_0 read as v0), t restricted to
-// (tmin, tmax). Dot products (x*x' + y*y') + z*z', no contraction.
-__device__ inline bool mt(const TriRec& T, const RayState& r, float& t, float& u, float& v) {
+// (tmin, tmax], tmax the ray's or the best hit so far (the caller tells a tie
+// from an end). Dot products (x*x' + y*y') + z*z', no contraction.
+__device__ inline bool mt(const TriRec& T, const RayState& r, float tmax, float& t, float& u,
+                          float& v) {
   const float px = r.dy * T.e2.z - r.dz * T.e2.y;
   const float py = r.dz * T.e2.x - r.dx * T.e2.z;
   const float pz = r.dx * T.e2.y - r.dy * T.e2.x;
@@ -140,7 +159,7 @@ __device__ inline bool mt(const TriRec& T, const RayState& r, float& t, float& u
   const float vv = ((r.dx * qx + r.dy * qy) + r.dz * qz) * inv;
   if (vv < 0.0f || uu + vv > 1.0f) return false;
   const float tt = ((T.e2.x * qx + T.e2.y * qy) + T.e2.z * qz) * inv;
-  if (!(tt > r.tmin && tt < r.tmax)) return false;
+  if (!(tt > r.tmin && tt <= tmax)) return false;
   t = tt, u = uu, v = vv;
   return true;
 }
@@ -149,8 +168,8 @@ __device__ inline bool mt(const TriRec& T, const RayState& r, float& t, float& u
 // behind the origin (tca < 0) or a miss distance beyond the radius rejects;
 // otherwise t0 = tca - thc, t1 = tca + thc, and castRay takes t1 when t0 < 0
 // (main.cpp:349-353). The reference accepts that t whatever its value (it is
-// >= 0 once tca >= 0); here it must lie in [tmin, tmax).
-__device__ inline bool sphere_hit(const TriRec& S, const RayState& r, float& t) {
+// >= 0 once tca >= 0); here it must lie in [tmin, tmax], as above.
+__device__ inline bool sphere_hit(const TriRec& S, const RayState& r, float tmax, float& t) {
   const float lx = S.v0.x - r.ox, ly = S.v0.y - r.oy, lz = S.v0.z - r.oz;
   const float tca = (lx * r.dx + ly * r.dy) + lz * r.dz;
   if (tca < 0.0f) return false;
@@ -160,9 +179,73 @@ __device__ inline bool sphere_hit(const TriRec& S, const RayState& r, float& t) 
   const float thc = sqrtf(r2 - d2);
   const float t0 = tca - thc, t1 = tca + thc;
   const float tt = t0 < 0.0f ? t1 : t0;
-  if (!(tt >= r.tmin && tt < r.tmax)) return false;
+  if (!(tt >= r.tmin && tt <= tmax)) return false;
   t = tt;
   return true;
+}
+
+// The primitive tests accept a few rays that miss the primitive's box: the
+// sphere test by the cancellation above, the triangle test by its rounding
+// when the triangle is small for its distance (some rays in ten thousand at
+// 10^6 times its size). The walks answer for the rays that hit the box; a wide
+// node's box on the grid is larger than the exact one, so the wide walk tests
+// the exact one where the primitive test leaves a doubt.
+__device__ inline bool leaf_box(const float lo[3], const float hi[3], const RayState& r,
+                                float slack) {
+  const float o[3] = {r.ox, r.oy, r.oz}, d[3] = {r.ix, r.iy, r.iz};
+  float tn = r.tmin, tf = INFINITY;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    // an axis without direction, the origin on a plane: inside, as 0 * inf
+    const float i = fabsf(d[k]) < 0x1p100f ? d[k] : copysignf(INFINITY, d[k]);
+    const bool s = signbit(i);
+    tn = fmaxf(((s ? hi[k] : lo[k]) - o[k]) * i, tn);
+    tf = fminf(((s ? lo[k] : hi[k]) - o[k]) * i, tf);
+  }
+  return tn <= tf * slack;
+}
+// A triangle hit at t is doubtful at 2^12 times the triangle's size (the
+// rounding of u and v, about 2^-22 of that ratio, is then a thousandth).
+__device__ inline bool tri_doubt(const TriRec& T, float t) {
+  const float m = fmaxf(fmaxf(fmaxf(fabsf(T.e1.x), fabsf(T.e1.y)), fmaxf(fabsf(T.e1.z), fabsf(T.e2.x))),
+                        fmaxf(fabsf(T.e2.y), fabsf(T.e2.z)));
+  return t > 0x1p12f * m;
+}
+// Its box, from the record (within a rounding of the build's, far less than
+// a doubtful hit's error).
+__device__ inline bool tri_box(const TriRec& T, const RayState& r) {
+  const float v[3] = {T.v0.x, T.v0.y, T.v0.z}, e[3] = {T.e1.x, T.e1.y, T.e1.z},
+              f[3] = {T.e2.x, T.e2.y, T.e2.z};
+  float lo[3], hi[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    lo[k] = v[k] + fminf(fminf(e[k], f[k]), 0.0f);
+    hi[k] = v[k] + fmaxf(fmaxf(e[k], f[k]), 0.0f);
+  }
+  return leaf_box(lo, hi, r, SLAB_SLACK);
+}
+// A sphere leaf's box, as the build gives it (leaf_record).
+__device__ inline bool sphere_box(const TriRec& S, const RayState& r) {
+  const float c[3] = {S.v0.x, S.v0.y, S.v0.z};
+  float lo[3], hi[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) lo[k] = (c[k] - S.e1.x) + 0.0f, hi[k] = (c[k] + S.e1.x) + 0.0f;
+  return leaf_box(lo, hi, r, SPHERE_SLACK);
+}
+
+// The wide records as a raw buffer resource (scalar registers): loads at a
+// 32-bit offset from it need no 64-bit address arithmetic. Dword 3 selects
+// the 32-bit data format that gfx9 buffer instructions require.
+__device__ inline __amdgpu_buffer_rsrc_t wide_rsrc(const TraceArgs& a) {
+  const uint64_t bytes = (uint64_t)a.nprims * sizeof(WideNode);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<WideNode*>(a.wide), (short)0,
+                                           (int)(uint32_t)min(bytes, (uint64_t)0xFFFFFFFFu),
+                                           0x00020000);
+}
+typedef uint32_t Row __attribute__((ext_vector_type(4)));
+template <int AT>
+__device__ inline Row row_load(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
+  return __builtin_bit_cast(Row, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, AT, 0));
 }
 
 // Persistent traversal loop of one wave. BLOCK threads per block; DEPTH stack entries
@@ -177,46 +260,30 @@ __device__ inline bool sphere_hit(const TriRec& S, const RayState& r, float& t) 
 // SPHERES: the leaves may be spheres (a.sphere); false compiles triangles only.
 // WIDE: walk the 4-wide nodes (a.wide) instead of the binary ones: the slots
 // a ray's box test accepts are visited nearest first (closest hit; any hit in
-// slot order), the others pushed farthest first. The same boxes are tested
-// with the same slack, so culling is as conservative as the binary walk and
-// the result (the lexicographic minimum) is the same; visit order differs.
-// The wide records as a raw buffer resource (scalar registers): row loads at
-// a 32-bit offset from it, with the row's fixed part as a scalar or immediate
-// offset, need no 64-bit address arithmetic. Dword 3 selects the 32-bit data
-// format that gfx9 buffer instructions require.
-__device__ inline __amdgpu_buffer_rsrc_t wide_rsrc(const TraceArgs& a) {
-  const uint64_t bytes = (uint64_t)a.nprims * sizeof(WideNode);
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<WideNode*>(a.wide), (short)0,
-                                           (int)(uint32_t)min(bytes, (uint64_t)0xFFFFFFFFu),
-                                           0x00020000);
-}
-__device__ inline float4 row_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0);
-  return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
-                     __uint_as_float(v[3]));
-}
-__device__ inline int4 link_load(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
-  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, 96, 0);
-  return make_int4((int)v[0], (int)v[1], (int)v[2], (int)v[3]);
-}
-
-// ROWS, how the wide walk addresses a node's rows: a tree of
-// WIDE_UNIFORM_MAX_NODES nodes or more has rows beyond a 32-bit byte offset,
-// addressed in 64 bits with the near / far rows selected per value (ROWS_BIG);
-// smaller trees address them by 32-bit offsets from the array's base
-// (ROWS_SMALL); ROWS_ANY decides per launch inside one code path.
+// slot order), the others pushed farthest first. Their boxes contain the
+// binary nodes' and are tested with the same slack, so culling is at least as
+// conservative as the binary walk and the result (the lexicographic minimum)
+// is the same; visit order differs.
+// ROWS, how the wide walk addresses a record: a tree of more than
+// WIDE_SMALL_MAX_NODES nodes in 64 bits (ROWS_BIG), smaller ones by 32-bit
+// offsets from the array's base (ROWS_SMALL); ROWS_ANY decides per launch
+// inside one code path.
+// cold() points at the arguments a ray needs only when it starts or ends. The
+// query kernels read them again from the kernel's argument memory each time:
+// as hoisted scalars they crowded out the walk's own (33 of them spilled to
+// vector lanes, which held two registers and cost reads in the loop).
 constexpr int ROWS_SMALL = 0, ROWS_BIG = 1, ROWS_ANY = 2;
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
-          int ROWS, class Src>
-__device__ inline void trace_loop_impl(const TraceArgs& a, const Schedule& sc, const RayStream& rs,
-                                       int32_t* s_node, float* s_tn, uint32_t gtid,
-                                       uint32_t gstride, Src* src) {
+          int ROWS, class Src, class Cold>
+__device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, const Schedule& sc,
+                                       const RayStream& rs, int32_t* s_node, float* s_tn,
+                                       uint32_t gtid, uint32_t gstride, Src* src) {
   static_assert(!(WIDE && COUNT), "counted traversal walks the binary nodes");
-  const bool big = ROWS == ROWS_ANY ? a.nprims > WIDE_UNIFORM_MAX_NODES : ROWS == ROWS_BIG;
+  const bool big = ROWS == ROWS_ANY ? a.nprims > WIDE_SMALL_MAX_NODES : ROWS == ROWS_BIG;
   const int tid = threadIdx.x, lane = tid & 63;
-  const uint64_t lt = (1ull << lane) - 1ull;
   const int max_sp = DEPTH + (int)a.gdepth;
   const float slack = (SPHERES && a.sphere) ? SPHERE_SLACK : SLAB_SLACK;
+  const float eps = slack - 1.0f;
 
   RayState r{};  // lanes that never take a ray still read their (unused) octant
   bool active = false;
@@ -236,18 +303,19 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Schedule& sc, c
   uint32_t vis = 0, tst = 0;
 
   auto finish = [&]() {
-    const uint32_t oi = a.out_index ? a.out_index[ray] : ray;
+    const auto* c = cold();
+    const uint32_t oi = c->out_index ? c->out_index[ray] : ray;
     if (ANY) {
-      a.occ[oi] = best >= 0 ? 1 : 0;
+      c->occ[oi] = best >= 0 ? 1 : 0;
     } else {
-      a.prim[oi] = best;
-      if (a.t) a.t[oi] = best >= 0 ? bt : INFINITY;
-      if (a.u) a.u[oi] = bu;
-      if (a.v) a.v[oi] = bv;
+      c->prim[oi] = best;
+      if (c->t) c->t[oi] = best >= 0 ? bt : INFINITY;
+      if (c->u) c->u[oi] = bu;
+      if (c->v) c->v[oi] = bv;
     }
     if (COUNT) {
-      a.visits[oi] = vis;
-      a.tests[oi] = tst;
+      c->visits[oi] = vis;
+      c->tests[oi] = tst;
     }
     active = false;
   };
@@ -304,9 +372,10 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Schedule& sc, c
         }
         uint64_t s = 0;
         if (lane == 0)
-          s = rs.ctr64 ? atomicAdd(rs.ctr64, 1ull) - a.ctr_base[rs.seg] + rs.waves
+          s = rs.ctr64 ? atomicAdd(rs.ctr64, 1ull) - cold()->ctr_base[rs.seg] + rs.waves
                        : atomicAdd(rs.ctr32, sc.chunk);
-        s = __shfl(s, 0, 64);
+        s = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(s >> 32)) << 32 |
+            __builtin_amdgcn_readfirstlane((uint32_t)s);
         if (rs.ctr64) s = seg_slice(rs.seg, rs.segs, s);
         const uint32_t b = rs.ctr64 ? slice_begin(sc, s) : (uint32_t)min(s, (uint64_t)sc.n);
         if (b >= sc.n) {
@@ -317,96 +386,69 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Schedule& sc, c
         cend = rs.ctr64 ? slice_begin(sc, s + 1) : min(b + sc.chunk, sc.n);
       }
       const uint32_t take = min((uint32_t)__popcll(m), cend - cnext);
-      const uint32_t rank = (uint32_t)__popcll(m & lt);
+      const uint32_t rank = rank_in(m);
       if (!active && rank < take) {
         const uint32_t rr = cnext + rank;
+        const auto* c = cold();
         ray = rr;
-        r.ox = a.rays.ox[rr], r.oy = a.rays.oy[rr], r.oz = a.rays.oz[rr];
-        r.dx = a.rays.dx[rr], r.dy = a.rays.dy[rr], r.dz = a.rays.dz[rr];
-        r.tmin = a.rays.tmin[rr], r.tmax = a.rays.tmax[rr];
-        r.ix = 1.0f / r.dx, r.iy = 1.0f / r.dy, r.iz = 1.0f / r.dz;
+        r.ox = c->rays.ox[rr], r.oy = c->rays.oy[rr], r.oz = c->rays.oz[rr];
+        r.dx = c->rays.dx[rr], r.dy = c->rays.dy[rr], r.dz = c->rays.dz[rr];
+        r.tmin = c->rays.tmin[rr], bt = c->rays.tmax[rr];
+        if (WIDE)
+          r.ix = wide_inv(r.dx), r.iy = wide_inv(r.dy), r.iz = wide_inv(r.dz);
+        else
+          r.ix = 1.0f / r.dx, r.iy = 1.0f / r.dy, r.iz = 1.0f / r.dz;
         r.sx = signbit(r.ix), r.sy = signbit(r.iy), r.sz = signbit(r.iz);
-        best = -1, bt = r.tmax, bu = 0.0f, bv = 0.0f, vis = 0, tst = 0, sp = 0;
+        best = -1, bu = 0.0f, bv = 0.0f, vis = 0, tst = 0, sp = 0;
         node = a.nprims == 1 ? ~0 : 0;
         active = true;
-        if (!(r.tmin < r.tmax) || a.nprims == 0) finish();
+        if (!(r.tmin < bt) || a.nprims == 0) finish();
       }
       cnext += take;
       m = __ballot(!active);
     }
     if (__ballot(active) == 0ull && wave_out) break;
 
-    // Wide walk: when every active lane's direction has the same signs (an
-    // octant), the near / far rows are picked by scalar byte offsets instead
-    // of a select per value. Lanes that finish keep it so; a refill
-    // recomputes it.
-    uint32_t uni_rows = 0u, s_oct = 0u;
-    uint64_t mx = 0, my = 0, mz = 0;  // lanes whose 1/d has that sign bit set
     const __amdgpu_buffer_rsrc_t wrs = wide_rsrc(a);
-    if (WIDE) {
-      const uint32_t oct = (uint32_t)r.sx | ((uint32_t)r.sy << 1) | ((uint32_t)r.sz << 2);
-      const uint64_t am = __ballot(active);
-      const int first = am ? __ffsll((long long)am) - 1 : 0;
-      const uint32_t oref = (uint32_t)__shfl((int)oct, first, 64);
-      const bool uni = __ballot(active && oct != oref) == 0ull && !big;
-      uni_rows = __builtin_amdgcn_readfirstlane((uint32_t)uni);
-      s_oct = __builtin_amdgcn_readfirstlane(oref);
-      mx = __ballot(r.sx), my = __ballot(r.sy), mz = __ballot(r.sz);
-    }
 
     // ---- traverse until enough lanes are idle to be worth a refill -------
     for (;;) {
       if (WIDE && active && node >= 0) {
-        float4 nx, fx, ny, fy, nz, fz;
-        const WideNode* w = a.wide + node;
-        // the node's row offset, shared by both offset paths (computed here, a
-        // path that only issues loads needs no wait behind the other's loads)
-        const uint32_t base = (uint32_t)node << 7;
-        int4 ln;
-        if (!big && !uni_rows) {
-          // mixed octants: the same rows at per-lane byte offsets (an OR into
-          // the node's 128-byte row, cheaper than a select per value). The
-          // offsets are formed from the wave's sign masks at each visit
-          // (volatile: not hoisted out of the loop, where they would hold
-          // three registers across it; the closest-hit kernel would reach 91
-          // and leave less room beside a concurrent any-hit launch).
-          uint32_t qx, qy, qz;
-          asm volatile("v_cndmask_b32_e64 %0, 0, 16, %1" : "=v"(qx) : "s"(mx));
-          asm volatile("v_cndmask_b32_e64 %0, 0, 16, %1" : "=v"(qy) : "s"(my));
-          asm volatile("v_cndmask_b32_e64 %0, 0, 16, %1" : "=v"(qz) : "s"(mz));
-          nx = row_load(wrs, base | qx, 0u), fx = row_load(wrs, base | (qx ^ 16u), 0u);
-          ny = row_load(wrs, base | qy, 32u), fy = row_load(wrs, base | (qy ^ 16u), 32u);
-          nz = row_load(wrs, base | qz, 64u), fz = row_load(wrs, base | (qz ^ 16u), 64u);
-          if (ROWS == ROWS_ANY) ln = link_load(wrs, base);
-        } else if (ROWS == ROWS_ANY ? uni_rows != 0u : !big) {
-          // rows at byte offsets lox 0, hix 16, loy 32, hiy 48, loz 64, hiz 80;
-          // the near row of an axis is hi when its sign bit is set
-          const uint32_t ox = (s_oct & 1u) << 4, oy = 32u + ((s_oct & 2u) << 3),
-                         oz = 64u + ((s_oct & 4u) << 2);
-          nx = row_load(wrs, base, ox), fx = row_load(wrs, base, ox ^ 16u);
-          ny = row_load(wrs, base, oy), fy = row_load(wrs, base, oy ^ 16u);
-          nz = row_load(wrs, base, oz), fz = row_load(wrs, base, oz ^ 16u);
-          if (ROWS == ROWS_ANY) ln = link_load(wrs, base);
+        Row r0, r1, r2, r3;
+        if (!big) {
+          const uint32_t off = (uint32_t)node * (uint32_t)sizeof(WideNode);
+          r0 = row_load<0>(wrs, off), r1 = row_load<16>(wrs, off);
+          r2 = row_load<32>(wrs, off), r3 = row_load<48>(wrs, off);
         } else {
-          const float4 lx = w->lox, hx = w->hix, ly = w->loy, hy = w->hiy, lz = w->loz,
-                       hz = w->hiz;
-          // near / far rows by the direction's sign (hi is near when 1/d < 0)
-          nx = r.sx ? hx : lx, fx = r.sx ? lx : hx;
-          ny = r.sy ? hy : ly, fy = r.sy ? ly : hy;
-          nz = r.sz ? hz : lz, fz = r.sz ? lz : hz;
-          if (ROWS != ROWS_SMALL) ln = w->link;
+          const Row* w = reinterpret_cast<const Row*>(a.wide + node);
+          r0 = w[0], r1 = w[1], r2 = w[2], r3 = w[3];
         }
-        // the link row after the rows: the uniform path, which statically
-        // follows the per-lane path's loads, then starts with nothing in
-        // flight to wait on. (A walk that decides the row form per launch
-        // loads it in each branch instead: one load after them would be a
-        // select between a buffer and a 64-bit load.)
-        if (ROWS == ROWS_SMALL) ln = link_load(wrs, base);
-        float t0, t1, t2, t3;
-        const bool h0 = slab_w(nx.x, ny.x, nz.x, fx.x, fy.x, fz.x, r, bt, slack, t0) & (ln.x != 0);
-        const bool h1 = slab_w(nx.y, ny.y, nz.y, fx.y, fy.y, fz.y, r, bt, slack, t1) & (ln.y != 0);
-        const bool h2 = slab_w(nx.z, ny.z, nz.z, fx.z, fy.z, fz.z, r, bt, slack, t2) & (ln.z != 0);
-        const bool h3 = slab_w(nx.w, ny.w, nz.w, fx.w, fy.w, fz.w, r, bt, slack, t3) & (ln.w != 0);
+        const int4 ln = make_int4((int)r3[0], (int)r3[1], (int)r3[2], (int)r3[3]);
+        // near / far planes by the direction's sign (hi is near when 1/d < 0),
+        // two axes and then the third: the planes of all three at once would
+        // hold eight registers more
+        float t0, t1, t2, t3, f0, f1, f2, f3;
+        {
+          const float sx = __uint_as_float(r0[3]) * r.ix, sy = __uint_as_float(r1[0]) * r.iy;
+          const float bx = (__uint_as_float(r0[0]) - r.ox) * r.ix,
+                      by = (__uint_as_float(r0[1]) - r.oy) * r.iy;
+          const float4 nx = wide_planes(r.sx ? r1[3] : r1[2], sx, bx),
+                       fx = wide_planes(r.sx ? r1[2] : r1[3], sx, bx),
+                       ny = wide_planes(r.sy ? r2[1] : r2[0], sy, by),
+                       fy = wide_planes(r.sy ? r2[0] : r2[1], sy, by);
+          t0 = fmaxf(fmaxf(nx.x, ny.x), r.tmin), f0 = fminf(fminf(fx.x, fy.x), bt);
+          t1 = fmaxf(fmaxf(nx.y, ny.y), r.tmin), f1 = fminf(fminf(fx.y, fy.y), bt);
+          t2 = fmaxf(fmaxf(nx.z, ny.z), r.tmin), f2 = fminf(fminf(fx.z, fy.z), bt);
+          t3 = fmaxf(fmaxf(nx.w, ny.w), r.tmin), f3 = fminf(fminf(fx.w, fy.w), bt);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const float sz = __uint_as_float(r1[1]) * r.iz, bz = (__uint_as_float(r0[2]) - r.oz) * r.iz;
+        const float4 nz = wide_planes(r.sz ? r2[3] : r2[2], sz, bz),
+                     fz = wide_planes(r.sz ? r2[2] : r2[3], sz, bz);
+        const bool h0 = slot_hit(nz.x, fz.x, eps, t0, f0) & (ln.x != 0);
+        const bool h1 = slot_hit(nz.y, fz.y, eps, t1, f1) & (ln.y != 0);
+        const bool h2 = slot_hit(nz.z, fz.z, eps, t2, f2) & (ln.z != 0);
+        const bool h3 = slot_hit(nz.w, fz.w, eps, t3, f3) & (ln.w != 0);
         const int k = (int)h0 + (int)h1 + (int)h2 + (int)h3;
         // sort the slots by entry distance, misses last: a hit's key is its
         // distance's bits (ordered for tn >= +0, i.e. tmin >= 0; otherwise
@@ -481,23 +523,28 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Schedule& sc, c
         const TriRec T = a.tris[~node];
         if (COUNT) ++tst;
         float t, u = 0.0f, v = 0.0f;
-        bool done = false;
-        if ((SPHERES && a.sphere) ? sphere_hit(T, r, t) : mt(T, r, t, u, v)) {
+        bool done = false, hit;
+        if (SPHERES && a.sphere) {
+          hit = sphere_hit(T, r, bt, t) && (!WIDE || sphere_box(T, r));
+        } else {
+          hit = mt(T, r, bt, t, u, v);
+          if (WIDE && hit && tri_doubt(T, t)) hit = a.nprims < 2u || tri_box(T, r);
+        }
+        if (hit) {
           const int32_t prim = __float_as_int(T.v0.w);
+          // t <= bt, which is the ray's open end until there is a hit
           if (ANY) {
-            best = prim, bt = t;
-            done = true;
-          } else if (best < 0 || t < bt || (t == bt && prim < best)) {
+            if (t < bt) best = prim, done = true;
+          } else if (t < bt || (best >= 0 && prim < best)) {
             best = prim, bt = t, bu = u, bv = v;
           }
         }
         if (done || !pop()) finish();
       }
-      const uint64_t idle = __ballot(!active);
-      if (__ballot(active) == 0ull || (!wave_out && __popcll(idle) >= a.refill_idle)) break;
+      const uint32_t idle = (uint32_t)__popcll(__ballot(!active));
+      if (idle == 64u || (!wave_out && idle >= a.refill_idle)) break;
     }
   }
-
 }
 
 // One code path for trees of any size (the batch and serving kernels, whose
@@ -509,23 +556,21 @@ __device__ inline void trace_loop(const TraceArgs& a, const RayStream& rs, int32
                                   Src* src = nullptr) {
   const Schedule sc{a.nrays, a.chunk, 0u, 0u, 1u};
   trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_ANY, Src>(
-      a, sc, rs, s_node, s_tn, gtid, gstride, src);
+      a, [&] { return &a; }, sc, rs, s_node, s_tn, gtid, gstride, src);
 }
-// A path per row form, chosen once per launch (the query kernels: one tree).
-// Below 2^25 nodes every row, the link row included, is a load at a 32-bit
-// offset from the scalar base, with no 64-bit address arithmetic; the closest-
-// hit kernels also drop their register spills.
+// A path per record addressing, chosen once per launch (the query kernels:
+// one tree).
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES = true,
-          bool WIDE = false>
-__device__ inline void trace_loop_split(const TraceArgs& a, const Schedule& sc,
+          bool WIDE = false, class Cold>
+__device__ inline void trace_loop_split(const TraceArgs& a, const Cold& cold, const Schedule& sc,
                                         const RayStream& rs, int32_t* s_node, float* s_tn,
                                         uint32_t gtid, uint32_t gstride) {
-  if (WIDE && a.nprims > WIDE_UNIFORM_MAX_NODES)
+  if (WIDE && a.nprims > WIDE_SMALL_MAX_NODES)
     trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_BIG, NoSlices>(
-        a, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
+        a, cold, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
   else
     trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_SMALL, NoSlices>(
-        a, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
+        a, cold, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
 }
 
 }  // namespace rq

@@ -15,7 +15,18 @@
 namespace rq {
 namespace {
 
-// WAVES > 0: registers capped for that many waves per SIMD.
+// The kernel's arguments, read from its argument memory anew at each call
+// (the empty asm hides that the address never changes).
+typedef __attribute__((address_space(4))) const TraceArgs* ArgsPtr;
+struct KernelArgs {
+  __device__ ArgsPtr operator()() const {
+    ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+  }
+};
+
+// WAVES > 0: registers capped so that this many waves fit a SIMD.
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool WIDE = false, int WAVES = 0>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1)))
 void k_trace(TraceArgs a) {
@@ -27,19 +38,19 @@ void k_trace(TraceArgs a) {
   rs.segs = sc.segs;
   rs.seg = seg_of(blockIdx.x, sc.segs);
   rs.ctr64 = a.counter + rs.seg * COUNTER_STRIDE;
-  rs.wave = seg_index(blockIdx.x, sc.segs) * WPB + (threadIdx.x >> 6);
+  rs.wave = seg_index(blockIdx.x, sc.segs) * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   rs.waves = seg_blocks(rs.seg, sc.segs, gridDim.x) * WPB;
   trace_loop_split<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE>(
-      a, sc, rs, s_node, s_tn, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK);
+      a, KernelArgs{}, sc, rs, s_node, s_tn, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK);
 }
 
 // Device scratch of the allocation-free closest-hit entry
 // (rq_closest_hit_noalloc): the launch's ray-stream counters in the first
-// NOALLOC_COUNTER_BYTES, then the traversal stack overflow area ([depth][thread] pairs). One
-// copy per device, held from module load until the process ends; its address
-// comes from hipGetSymbolAddress (noalloc_scratch_address), never from the
-// array's name in host code. Calls that overlap on one device share it and
-// race.
+// NOALLOC_COUNTER_BYTES, then the traversal stack overflow area
+// ([depth][thread] pairs). One copy per device, held from module load until
+// the process ends; its address comes from hipGetSymbolAddress
+// (noalloc_scratch_address), never from the array's name in host code. Calls
+// that overlap on one device share it and race.
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 __global__ __launch_bounds__(64) void k_counter_reset(unsigned long long* ctr) {
@@ -50,51 +61,50 @@ typedef void (*TraceFn)(TraceArgs);
 struct Variant {
   int block, depth;
   bool tstack, wide;
-  int closest_waves, any_waves;  // waves per SIMD the kernels are capped for (0: none)
+  int closest_waves, any_waves;  // waves per SIMD that are promised (0: none)
   TraceFn closest, any;
 };
 
 // Variant 0 is the canonical binary configuration (the counted kernels run
-// it); the wide variants need the BVH's 4-wide nodes. A wide any-hit kernel
-// whose LDS stack leaves room for 6 waves per SIMD (6 x 4 waves x 64 lanes x
-// DEPTH x 4 B <= 160 KB: DEPTH <= 26) is compiled for 6 (80 VGPRs, no spills;
-// left to itself the compiler takes 81 and gets 5): it waits on dependent
-// node fetches more than it issues, and the sixth wave hides more of that
-// wait (shadow rays of a 1.31 M-triangle frame 11 %, uniform rays over 5.24 M
-// triangles 6 % faster). The closest-hit walk issues at ~0.8 of the peak and
-// spills at that cap, so it keeps its 5 waves. The launch grid follows each
-// kernel's own occupancy.
-constexpr int any_waves(bool wide, int depth) { return wide && depth <= 26 ? 6 : 0; }
-#define RQ_VARIANT(B, D, T, W)                                              \
-  {                                                                         \
-    B, D, T, W, 0, any_waves(W, D), k_trace<false, false, B, D, T, W>,      \
-        k_trace<true, false, B, D, false, W, any_waves(W, D)>               \
+// it); the wide variants need the BVH's 4-wide nodes. A wide walk waits on
+// dependent record fetches, so its kernels are compiled for as many waves per
+// SIMD as their LDS stack leaves room for: eight (64 VGPRs) with 16 entries,
+// six with 24. Left to itself the compiler takes 70 VGPRs and over 96 SGPRs,
+// six waves. 8.3 M camera rays over 1.31 M triangles 0.78 ms at six, 0.73 at
+// seven, 0.68 at eight; 8.3 M uniform rays over 5.24 M triangles 0.60, 0.55,
+// 0.54 ms closest and 0.53, 0.48, 0.45 ms any hit. The launch grid follows
+// each kernel's own occupancy.
+constexpr int wide_waves(int depth, bool tstack) {
+  int w = 8;
+  while (w > 1 && w * 4 * 64 * depth * (tstack ? 8 : 4) > 160 * 1024) --w;
+  return w;
+}
+// What rq_trace_variant_get promises: six waves or more for the any-hit
+// kernels with that much LDS, and for the closest-hit kernels of the last two
+// variants.
+constexpr int promised(bool wide, int depth) { return wide && depth <= 26 ? 6 : 0; }
+#define RQ_WIDE(B, D, T, C)                                                  \
+  {                                                                          \
+    B, D, T, true, C, promised(true, D),                                     \
+        k_trace<false, false, B, D, T, true, wide_waves(D, T)>,              \
+        k_trace<true, false, B, D, false, true, wide_waves(D, false)>        \
   }
-// Variants whose closest-hit kernel is capped at six waves per SIMD as well
-// (80 VGPRs, 2 spilled). In a 1920x1080x4 frame of a 1.31 M-triangle mesh
-// its launches take the same time alone, but beside the concurrent any-hit
-// launch (also at six) the two share the CUs better: 3.26 -> 3.21 ms per
-// frame.
-#define RQ_VARIANT6(B, D)                                                   \
-  {                                                                         \
-    B, D, false, true, 6, any_waves(true, D),                               \
-        k_trace<false, false, B, D, false, true, 6>,                        \
-        k_trace<true, false, B, D, false, true, any_waves(true, D)>         \
+#define RQ_BINARY(B, D, T)                                                   \
+  {                                                                          \
+    B, D, T, false, 0, 0, k_trace<false, false, B, D, T>,                    \
+        k_trace<true, false, B, D, false>                                    \
   }
 const Variant kVariants[] = {
-    RQ_VARIANT(128, 24, false, false), RQ_VARIANT(128, 16, false, false),
-    RQ_VARIANT(64, 24, false, false),  RQ_VARIANT(256, 16, false, false),
-    RQ_VARIANT(128, 24, true, false),  RQ_VARIANT(128, 16, true, false),
-    RQ_VARIANT(64, 16, true, false),   RQ_VARIANT(64, 32, false, false),
-    RQ_VARIANT(64, 12, true, false),   RQ_VARIANT(128, 24, false, true),
-    RQ_VARIANT(128, 32, false, true), RQ_VARIANT(64, 32, false, true),
-    RQ_VARIANT(128, 24, true, true),  RQ_VARIANT(64, 24, true, true),
-    RQ_VARIANT(256, 16, false, true),  RQ_VARIANT(256, 24, false, true),
-    RQ_VARIANT(256, 28, false, true),  RQ_VARIANT6(256, 16),
-    RQ_VARIANT6(128, 24),
+    RQ_BINARY(128, 24, false),   RQ_BINARY(128, 16, false),   RQ_BINARY(64, 24, false),
+    RQ_BINARY(256, 16, false),   RQ_BINARY(128, 24, true),    RQ_BINARY(128, 16, true),
+    RQ_BINARY(64, 16, true),     RQ_BINARY(64, 32, false),    RQ_BINARY(64, 12, true),
+    RQ_WIDE(128, 16, false, 0),  RQ_WIDE(128, 32, false, 0),  RQ_WIDE(64, 32, false, 0),
+    RQ_WIDE(128, 24, true, 0),   RQ_WIDE(64, 24, true, 0),    RQ_WIDE(256, 16, false, 0),
+    RQ_WIDE(256, 24, false, 0),  RQ_WIDE(256, 28, false, 0),  RQ_WIDE(256, 16, false, 6),
+    RQ_WIDE(128, 24, false, 6),
 };
-#undef RQ_VARIANT
-#undef RQ_VARIANT6
+#undef RQ_WIDE
+#undef RQ_BINARY
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 static_assert(TRACE_DEFAULT_CLOSEST < kNumVariants && TRACE_DEFAULT_ANY < kNumVariants,
               "default variants in the table");
