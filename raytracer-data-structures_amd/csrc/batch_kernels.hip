@@ -161,7 +161,6 @@ __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* er
   t.gdepth = gdepth;
   t.err = err;
   t.refill_idle = refill_idle;
-  t.chunk = 64;
   t.sphere = 0;  // batch meshes are triangle scenes
   if (WAVE_ITEM) {
     // lane 0 resets the counter and is the lane that takes from it (trace_loop)
@@ -172,21 +171,16 @@ __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* er
   }
   int32_t* s_node = reinterpret_cast<int32_t*>(lds);
   float* s_tn = reinterpret_cast<float*>(lds + DEPTH * BUILD_BLOCK);
-  const uint32_t gtid = blockIdx.x * BUILD_BLOCK + threadIdx.x;
-  const uint32_t gstride = gridDim.x * BUILD_BLOCK;
-  RayStream stream;
-  stream.ctr32 = s_ctr;
+  ItemRays src{s_ctr, nr};
   if (any) {
     t.occ = m.occ + r0;
-    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE>(t, stream, s_node, s_tn,
-                                                                    gtid, gstride);
+    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE>(t, src, s_node, s_tn);
   } else {
     t.prim = m.prim + r0;
     t.t = m.t ? m.t + r0 : nullptr;
     t.u = m.u ? m.u + r0 : nullptr;
     t.v = m.v_ ? m.v_ + r0 : nullptr;
-    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE>(t, stream, s_node, s_tn,
-                                                                      gtid, gstride);
+    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE>(t, src, s_node, s_tn);
   }
   if (!WAVE_ITEM) __syncthreads();
 }
@@ -199,7 +193,6 @@ __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* er
 // rather than once per tile; the first item of another mesh or kind ends the
 // walk and starts the next one.
 struct ItemSlices {
-  static constexpr bool kActive = true;
   const BatchArgs& args;
   uint32_t xcd, k;  // segment cursor: segment (xcd + k) % BATCH_XCDS
   uint32_t mesh, kind, nrays;
@@ -255,24 +248,18 @@ __device__ inline void trace_mesh(const BatchArgs& a, const BatchMeshDev& m, uin
   t.gdepth = a.gdepth;
   t.err = a.ctl + BATCH_CTL_TRACE_ERR;
   t.refill_idle = a.refill_idle;
-  t.chunk = 64;
   t.sphere = 0;  // batch meshes are triangle scenes
   int32_t* s_node = reinterpret_cast<int32_t*>(lds);
   float* s_tn = reinterpret_cast<float*>(lds + DEPTH * BUILD_BLOCK);
-  const uint32_t gtid = blockIdx.x * BUILD_BLOCK + threadIdx.x;
-  const uint32_t gstride = gridDim.x * BUILD_BLOCK;
-  const RayStream stream;  // unused: the slices come from src
   if (src->kind) {
     t.occ = m.occ;
-    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE>(t, stream, s_node, s_tn, gtid,
-                                                                    gstride, src);
+    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE>(t, *src, s_node, s_tn);
   } else {
     t.prim = m.prim;
     t.t = m.t;
     t.u = m.u;
     t.v = m.v_;
-    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE>(t, stream, s_node, s_tn,
-                                                                      gtid, gstride, src);
+    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE>(t, *src, s_node, s_tn);
   }
 }
 

@@ -670,14 +670,17 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
   a.counter = c->counters + (size_t)slot * SLOT_WORDS;
   if (!own_zero) std::copy_n(c->counter_base[slot], TRACE_SEGS, a.ctr_base);
   a.err = c->errword;
-  // the launch grid (launch_trace takes the same), its waves and slice size
+  // the launch grid, its waves and slice size
   const uint32_t full_grid = any ? c->trace_grid_any[variant] : c->trace_grid[variant];
-  a.grid = std::max(1u, std::min(full_grid, (n + (uint32_t)blk - 1) / (uint32_t)blk));
+  const uint32_t wpb = (uint32_t)blk / 64u, full_waves = full_grid * wpb;
+  const uint32_t spread = wide && !count_dev ? spread_chunk(n, full_waves) : 64u;
+  const uint32_t chunk = spread < 64u ? spread
+                                      : trace_chunk(n, full_waves, any ? c->slice_any : c->slice_closest);
+  a.grid = std::max<uint32_t>(1u, (uint32_t)std::min<uint64_t>(
+                                       full_grid, (n + (uint64_t)spread * wpb - 1) / (spread * wpb)));
   a.refill_idle = any ? c->refill_any : c->refill_closest;
-  const uint32_t waves = a.grid * (uint32_t)blk / 64u;
-  const SliceSchedule sched =
-      slice_schedule(n, trace_chunk(n, full_grid * (uint32_t)blk / 64u,
-                                    any ? c->slice_any : c->slice_closest));
+  const uint32_t waves = a.grid * wpb;
+  const SliceSchedule sched = slice_schedule(n, chunk);
   a.chunk = sched.chunk, a.chunk_small = sched.small, a.big_slices = sched.big;
   a.segs = trace_segs(sched.total, waves, a.grid);
   if (count_dev) a.chunk = any ? c->slice_any : c->slice_closest;  // the largest slice

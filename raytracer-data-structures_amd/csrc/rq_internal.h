@@ -125,6 +125,19 @@ __host__ __device__ inline uint32_t trace_chunk(uint32_t n, uint32_t waves,
   while (c > 64 && (uint64_t)n < 8ull * c * waves) c >>= 1;
   return c;
 }
+// Rays per wave of a launch too small to give every wave 64 (`waves`: the
+// waves the chip holds): two, or the power of two above that at which all have
+// a wave; the idle lanes share the rays' walks (SplitSlots in trace_device.h).
+// 64: full waves. 16 k rays, 500 spheres: 295 us at 64 a wave, 255 of them
+// shared, 93 / 64 / 46 at 8 / 4 / 2; 65 k rays, 100 k triangles: 523, 464,
+// 449 / 440 / 426 at 32 / 16 / 8. One ray a wave gains nothing over two: 4 k
+// rays 139 us against 137, 7 k short ones 32 against 28 (a wave costs its
+// start).
+inline uint32_t spread_chunk(uint32_t n, uint32_t waves) {
+  uint32_t c = 2;
+  while (c < 64 && (uint64_t)c * waves < n) c <<= 1;
+  return c;
+}
 // Slice schedule of a standalone launch: slices of `chunk` rays over the
 // first three quarters of the stream, then slices of chunk / 4 (at least 64)
 // so that the waves finish together; slice s starts at slice_begin(s).
@@ -134,7 +147,7 @@ struct SliceSchedule {
 __host__ __device__ inline SliceSchedule slice_schedule(uint32_t n, uint32_t chunk) {
   SliceSchedule q;
   q.chunk = chunk;
-  q.small = chunk / 4 < 64 ? 64 : chunk / 4;
+  q.small = chunk <= 64 ? chunk : (chunk / 4 < 64 ? 64 : chunk / 4);
   q.big = (uint32_t)((3ull * n / 4) / chunk);
   const uint64_t rest = n - (uint64_t)q.big * chunk;
   q.total = q.big + (uint32_t)((rest + q.small - 1) / q.small);

@@ -9,37 +9,23 @@
 // so far. The result is the (t, primitive id) lexicographic minimum, i.e. the
 // NONE loop of main.cpp:373-387 (lowest index wins ties).
 #pragma once
+#include <type_traits>
+
 #include "rq_internal.h"
 
 namespace rq {
 
-// Where a wave takes its slices of the ray stream from. The standalone kernels
-// number the slices (a.chunk rays each for the first a.big_slices, then
-// a.chunk_small) and deal them to segments (seg_slice): the w-th wave of a
-// segment starts on the segment's slice w (no atomic), and takes its slice
-// waves + k from the k-th add to the segment's 64-bit counter that is never
-// reset (k = counter add - TraceArgs::ctr_base). When the waves' first slices cover the
-// segment no wave touches the counter; otherwise each wave makes exactly one
-// failing add and every later slice is one add, so the launch moves the
-// counter by exactly the segment's number of slices, which the host adds to
-// the base of the slot's next launch. The batch kernel counts rays from 0 in
-// LDS.
-struct RayStream {
-  uint32_t* ctr32 = nullptr;            // counter of rays from 0 (batch, LDS), or
-  unsigned long long* ctr64 = nullptr;  // the segment's monotonic slice counter
-  uint32_t seg = 0, segs = 1;           // this wave's segment, segments of the launch
-  uint32_t wave = 0, waves = 0;         // this wave's index, waves in the segment
-};
-// The launch's ray count, slice sizes and segments, in scalar registers: from
-// the kernel arguments, or computed here from a count read from device memory
+// The launch's ray count, slice sizes and segments: from the kernel arguments,
+// or computed here from a count read from device memory
 // (TraceArgs::nrays_dev).
 struct Schedule {
   uint32_t n, chunk, small, big, segs;
 };
-__device__ inline Schedule schedule_of(const TraceArgs& a, uint32_t waves, uint32_t grid) {
-  if (!a.nrays_dev) return Schedule{a.nrays, a.chunk, a.chunk_small, a.big_slices, a.segs};
-  const uint32_t n = min(a.nrays, __builtin_amdgcn_readfirstlane(*a.nrays_dev));
-  const SliceSchedule q = slice_schedule(n, trace_chunk(n, waves, a.chunk));
+template <class Args>
+__device__ inline Schedule schedule_of(const Args* a, uint32_t waves, uint32_t grid) {
+  if (!a->nrays_dev) return Schedule{a->nrays, a->chunk, a->chunk_small, a->big_slices, a->segs};
+  const uint32_t n = min(a->nrays, __builtin_amdgcn_readfirstlane(*a->nrays_dev));
+  const SliceSchedule q = slice_schedule(n, trace_chunk(n, waves, a->chunk));
   return Schedule{n, q.chunk, q.small, q.big, trace_segs(q.total, waves, grid)};
 }
 __device__ inline uint32_t slice_begin(const Schedule& a, uint64_t s) {
@@ -48,18 +34,71 @@ __device__ inline uint32_t slice_begin(const Schedule& a, uint64_t s) {
                                     (uint64_t)a.n);
 }
 
+// The lane's number, computed here and now (volatile: a value that the walk
+// would hold in a register, or spill, across all of its loops).
+__device__ inline int lane_now() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
 // This lane's rank among the lanes of a wave mask.
 __device__ inline uint32_t rank_in(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// A wave takes its slices from the RayStream unless the caller gives a slice
-// source: Src::next(b, e) returns the wave's next slice [b, e) of a.rays, or
-// false when the wave is to finish its rays and return. It is called with
-// every lane of the wave active and its result is wave-uniform.
-struct NoSlices {
-  static constexpr bool kActive = false;
-  __device__ bool next(uint32_t&, uint32_t&) { return false; }
+// Where a wave takes its slices of the ray stream from: Src::next(b, e)
+// returns the wave's next slice [b, e) of the rays, or false when there is
+// none left for it. It is called with every lane of the wave active and its
+// result is wave-uniform.
+//
+// The standalone kernels number the slices (chunk rays each for the first
+// big_slices, then chunk_small) and deal them to segments (seg_slice): the
+// w-th wave of a segment starts on the segment's slice w (no atomic), and
+// takes its slice waves + k from the k-th add to the segment's 64-bit counter
+// that is never reset (k = counter add - TraceArgs::ctr_base). When the waves'
+// first slices cover the segment no wave touches the counter; otherwise each
+// wave makes exactly one failing add and every later slice is one add, so the
+// launch moves the counter by exactly the segment's number of slices, which
+// the host adds to the base of the slot's next launch.
+template <class Cold, int WPB>
+struct QuerySlices {
+  Cold cold;
+  Schedule sc;
+  uint32_t seg, index, waves;  // the segment, this wave's index in it, its waves
+  bool first = true;
+  __device__ QuerySlices(const Cold& c, uint32_t wave_in_block)
+      : cold(c), sc(schedule_of(c(), gridDim.x * WPB, gridDim.x)), seg(seg_of(blockIdx.x, sc.segs)),
+        index(seg_index(blockIdx.x, sc.segs) * WPB + wave_in_block),
+        waves(seg_blocks(seg, sc.segs, gridDim.x) * WPB) {}
+  __device__ bool next(uint32_t& b, uint32_t& e) {
+    uint64_t s = index;
+    if (!first) {
+      if (slice_begin(sc, seg_slice(seg, sc.segs, waves)) >= sc.n) return false;  // first slices cover all
+      const auto* c = cold();
+      uint64_t k = 0;
+      if ((threadIdx.x & 63u) == 0u) k = atomicAdd(c->counter + seg * COUNTER_STRIDE, 1ull);
+      k = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(k >> 32)) << 32 |
+          __builtin_amdgcn_readfirstlane((uint32_t)k);
+      s = k - c->ctr_base[seg] + waves;
+    }
+    first = false;
+    s = seg_slice(seg, sc.segs, s);
+    b = slice_begin(sc, s), e = slice_begin(sc, s + 1);
+    return b < sc.n;
+  }
+};
+// One block's waves share the n rays of an item, 64 at a time from a counter
+// in LDS (or one wave has an item and a counter of its own).
+struct ItemRays {
+  uint32_t* ctr;
+  uint32_t n;
+  __device__ bool next(uint32_t& b, uint32_t& e) {
+    uint32_t k = 0;
+    if ((threadIdx.x & 63u) == 0u) k = atomicAdd(ctr, 64u);
+    b = __builtin_amdgcn_readfirstlane(k);
+    e = min(b + 64u, n);
+    return b < n;
+  }
 };
 
 struct RayState {
@@ -248,15 +287,55 @@ __device__ inline Row row_load(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
   return __builtin_bit_cast(Row, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, AT, 0));
 }
 
+// ---- rays walked by several lanes ---------------------------------------------
+// Once SPLIT_IDLE lanes of a wave are idle and cannot be refilled, they take
+// entries off the stacks of the lanes still walking and walk those subtrees of
+// the same rays. Such a split ray has a slot in the wave's LDS: the smallest
+// (t, primitive) found by any of its lanes as one 64-bit word (the bits of t,
+// ordered as unsigned, above the primitive), which the lanes also cull with,
+// and t, u, v of that hit. A lane's part ends when its stack is empty; the
+// results are written from the slots once the whole wave is idle. The minimum
+// does not depend on who walks what, so answers are the same.
+// A ray's walk is a chain of dependent fetches, and the longest of a wave's 64
+// (or the only one, in a small launch) sets the wave's time: 2.1 M camera
+// rays 0.31 -> 0.25 ms with their copies, 1 M uniform rays in a soup 0.48 ->
+// 0.40 ms closest and 0.38 -> 0.31 ms any hit. Rays that are short throughout
+// pay for the code's presence: 8.3 M frame rays 0.69 -> 0.71 ms. 48 idle
+// lanes: from 40 on the helpers' work costs as much as it saves, at 56 the
+// gain on camera rays is a third less; sharing only from the 4th, 7th or 10th
+// such step on loses 1 to 10 % on every kind of ray.
+constexpr uint32_t SPLIT_IDLE = 48;
+constexpr uint32_t SPLIT_SLOTS = 16;  // split rays of a wave at a time
+struct SplitSlots {
+  unsigned long long key[SPLIT_SLOTS];  // ~0: no hit; any hit: 0 once there is one
+  float tuv[SPLIT_SLOTS][3];
+  uint32_t ray[SPLIT_SLOTS];
+};
+// One wave's lanes read what others of its lanes wrote: LDS accesses of a wave
+// complete in order, volatile keeps them in the code's order.
+typedef volatile __attribute__((address_space(3))) SplitSlots* Slots;
+__device__ inline uint32_t ord_bits(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ inline float ord_float(uint32_t u) {
+  return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
+}
+// (+ 0: hits at -0 and at 0 tie)
+__device__ inline uint32_t hit_ord(float t) { return ord_bits(t + 0.0f); }
+__device__ inline unsigned long long hit_key(float t, int32_t prim) {
+  return (unsigned long long)hit_ord(t) << 32 | (uint32_t)prim;
+}
+
 // Persistent traversal loop of one wave. BLOCK threads per block; DEPTH stack entries
 // per lane in LDS ([depth][lane], conflict-free), deeper entries in the global
 // overflow area ([depth][thread]); TSTACK: entries carry their entry distance
 // and a closest-hit pop skips entries now beyond the best hit (the box test
 // redone against the current best). Leaves reached from a node are tested in
 // the same loop iteration; the order of node visits and triangle tests is the
-// canonical one unless TSTACK skips an entry. Rays are taken a.chunk at a time
-// from *ctr (global or LDS), or a slice at a time from *src; the loop returns
-// when the stream has no rays left for the wave and its lanes are idle.
+// canonical one unless TSTACK skips an entry. Rays are taken a slice at a time
+// from src; the loop returns when it has none left for the wave and its lanes
+// are idle.
 // SPHERES: the leaves may be spheres (a.sphere); false compiles triangles only.
 // WIDE: walk the 4-wide nodes (a.wide) instead of the binary ones: the slots
 // a ray's box test accepts are visited nearest first (closest hit; any hit in
@@ -275,62 +354,75 @@ __device__ inline Row row_load(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
 constexpr int ROWS_SMALL = 0, ROWS_BIG = 1, ROWS_ANY = 2;
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
           int ROWS, class Src, class Cold>
-__device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, const Schedule& sc,
-                                       const RayStream& rs, int32_t* s_node, float* s_tn,
-                                       uint32_t gtid, uint32_t gstride, Src* src) {
+__device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src& src,
+                                       int32_t* s_node, float* s_tn, SplitSlots* slots = nullptr) {
+  // (a tree past 32-bit offsets keeps the walk without it)
+  constexpr bool SPLIT = WIDE && ROWS == ROWS_SMALL;
   static_assert(!(WIDE && COUNT), "counted traversal walks the binary nodes");
   const bool big = ROWS == ROWS_ANY ? a.nprims > WIDE_SMALL_MAX_NODES : ROWS == ROWS_BIG;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int max_sp = DEPTH + (int)a.gdepth;
+  const int tid = threadIdx.x;
   const float slack = (SPHERES && a.sphere) ? SPHERE_SLACK : SLAB_SLACK;
   const float eps = slack - 1.0f;
 
   RayState r{};  // lanes that never take a ray still read their (unused) octant
   bool active = false;
-  // wave-private slice of the ray stream [cnext, cend), refilled CHUNK rays at
-  // a time from the global counter (one atomic per slice, not per refill)
-  uint32_t cnext = 0, cend = 0;
-  bool wave_out = false;  // the global stream is exhausted for this wave
-  if (rs.ctr64) {
-    const uint64_t s = seg_slice(rs.seg, rs.segs, rs.wave);
-    cnext = slice_begin(sc, s), cend = slice_begin(sc, s + 1);
-    wave_out = cnext >= sc.n;
-  }
+  uint32_t cnext = 0, cend = 0;  // what is left of the wave's slice
+  bool wave_out = false;         // there are no more slices for this wave
   uint32_t ray = 0;
   int32_t node = 0, best = -1;
   int sp = 0;
   float bt = 0.0f, bu = 0.0f, bv = 0.0f;
   uint32_t vis = 0, tst = 0;
 
-  auto finish = [&]() {
+  // the slot of a ray that several lanes walk (-1: this lane's alone; read only
+  // where lanes share), slots used
+  int own;
+  uint32_t nslots = 0;
+  const Slots ss = (Slots)slots;
+
+  auto write_hit = [&](uint32_t of, bool hit, int32_t prim, float t, float u, float v) {
     const auto* c = cold();
-    const uint32_t oi = c->out_index ? c->out_index[ray] : ray;
+    const uint32_t oi = c->out_index ? c->out_index[of] : of;
     if (ANY) {
-      c->occ[oi] = best >= 0 ? 1 : 0;
+      c->occ[oi] = hit ? 1 : 0;
     } else {
-      c->prim[oi] = best;
-      if (c->t) c->t[oi] = best >= 0 ? bt : INFINITY;
-      if (c->u) c->u[oi] = bu;
-      if (c->v) c->v[oi] = bv;
+      c->prim[oi] = hit ? prim : -1;
+      if (c->t) c->t[oi] = hit ? t : INFINITY;
+      if (c->u) c->u[oi] = u;
+      if (c->v) c->v[oi] = v;
     }
     if (COUNT) {
       c->visits[oi] = vis;
       c->tests[oi] = tst;
     }
+  };
+  // The lane's ray, or its part of a split ray, is walked to the end.
+  auto finish = [&](auto split) {
+    if (!decltype(split)::value) {
+      write_hit(ray, best >= 0, best, bt, bu, bv);
+    } else {
+      if (own < 0) write_hit(ray, best >= 0, best, bt, bu, bv);
+      own = -1;
+    }
     active = false;
+  };
+  // Entry `at` (DEPTH or deeper) of thread t's stack in the overflow area.
+  auto spilled = [&](int at, int t) -> int32_t* {
+    return cold()->gstack + 2 * ((size_t)(at - DEPTH) * (gridDim.x * BLOCK) + blockIdx.x * BLOCK + t);
   };
   auto push = [&](int32_t c, float tn) {
     if (sp < DEPTH) {
       s_node[sp * BLOCK + tid] = c;
       if (TSTACK) s_tn[sp * BLOCK + tid] = tn;
-    } else if (sp < max_sp) {
-      const size_t g = (size_t)(sp - DEPTH) * gstride + gtid;
-      a.gstack[2 * g] = c;
-      if (TSTACK) a.gstack[2 * g + 1] = __float_as_int(tn);
+    } else if (sp < DEPTH + (int)cold()->gdepth) {
+      int32_t* g = spilled(sp, tid);
+      g[0] = c;
+      if (TSTACK) g[1] = __float_as_int(tn);
     } else {
-      atomicOr(a.err, 1u);  // deeper than any LBVH of 30-bit codes: reported
+      atomicOr(cold()->err, 1u);  // deeper than any LBVH of 30-bit codes: reported
+      return;
     }
-    sp = min(sp + 1, max_sp);
+    ++sp;
   };
   // Pops the next entry into `node`; false when the stack is empty. The LDS
   // entry is read unconditionally (at a clamped depth) and replaced by the
@@ -344,9 +436,9 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, con
       node = s_node[ls * BLOCK + tid];
       float tn = TSTACK ? s_tn[ls * BLOCK + tid] : 0.0f;
       if (sp >= DEPTH) {
-        const size_t g = (size_t)(sp - DEPTH) * gstride + gtid;
-        node = a.gstack[2 * g];
-        if (TSTACK) tn = __int_as_float(a.gstack[2 * g + 1]);
+        const int32_t* g = spilled(sp, tid);
+        node = g[0];
+        if (TSTACK) tn = __int_as_float(g[1]);
       }
       if (!TSTACK || ANY || tn <= bt * slack) return true;
     }
@@ -354,36 +446,22 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, con
   };
 
   for (;;) {
+    if (SPLIT && nslots != 0u && __ballot(active) == 0ull) {
+      const int lane = lane_now();
+      if (lane < (int)nslots) {
+        const unsigned long long key = ss->key[lane];
+        write_hit(ss->ray[lane], key != ~0ull, (int32_t)(uint32_t)key, ss->tuv[lane][0],
+                  ss->tuv[lane][1], ss->tuv[lane][2]);
+      }
+      nslots = 0;
+    }
     // ---- refill idle lanes from the wave's slice of the ray stream -------
     uint64_t m = __ballot(!active);
+#pragma unroll 1
     for (int round = 0; round < 2 && m && !wave_out; ++round) {
-      if (Src::kActive && cnext >= cend) {
-        uint32_t b = 0, e = 0;
-        if (!src->next(b, e)) {
-          wave_out = true;
-          break;
-        }
-        cnext = b, cend = e;
-      } else if (cnext >= cend) {
-        if (rs.ctr64 && slice_begin(sc, seg_slice(rs.seg, rs.segs, rs.waves)) >= sc.n) {
-          // first slices cover all
-          wave_out = true;
-          break;
-        }
-        uint64_t s = 0;
-        if (lane == 0)
-          s = rs.ctr64 ? atomicAdd(rs.ctr64, 1ull) - cold()->ctr_base[rs.seg] + rs.waves
-                       : atomicAdd(rs.ctr32, sc.chunk);
-        s = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(s >> 32)) << 32 |
-            __builtin_amdgcn_readfirstlane((uint32_t)s);
-        if (rs.ctr64) s = seg_slice(rs.seg, rs.segs, s);
-        const uint32_t b = rs.ctr64 ? slice_begin(sc, s) : (uint32_t)min(s, (uint64_t)sc.n);
-        if (b >= sc.n) {
-          wave_out = true;
-          break;
-        }
-        cnext = b;
-        cend = rs.ctr64 ? slice_begin(sc, s + 1) : min(b + sc.chunk, sc.n);
+      if (cnext >= cend && !src.next(cnext, cend)) {
+        wave_out = true;
+        break;
       }
       const uint32_t take = min((uint32_t)__popcll(m), cend - cnext);
       const uint32_t rank = rank_in(m);
@@ -402,7 +480,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, con
         best = -1, bu = 0.0f, bv = 0.0f, vis = 0, tst = 0, sp = 0;
         node = a.nprims == 1 ? ~0 : 0;
         active = true;
-        if (!(r.tmin < bt) || a.nprims == 0) finish();
+        if (!(r.tmin < bt) || a.nprims == 0) finish(std::false_type{});
       }
       cnext += take;
       m = __ballot(!active);
@@ -411,166 +489,247 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, con
 
     const __amdgpu_buffer_rsrc_t wrs = wide_rsrc(a);
 
-    // ---- traverse until enough lanes are idle to be worth a refill -------
-    for (;;) {
-      if (WIDE && active && node >= 0) {
-        Row r0, r1, r2, r3;
-        if (!big) {
-          const uint32_t off = (uint32_t)node * (uint32_t)sizeof(WideNode);
-          r0 = row_load<0>(wrs, off), r1 = row_load<16>(wrs, off);
-          r2 = row_load<32>(wrs, off), r3 = row_load<48>(wrs, off);
-        } else {
-          const Row* w = reinterpret_cast<const Row*>(a.wide + node);
-          r0 = w[0], r1 = w[1], r2 = w[2], r3 = w[3];
+    // Idle lanes join the rays still walked: the k-th entry from the top of the
+    // j-th lane's stack goes to the (k * lanes + j)-th idle lane. Lanes whose
+    // rays are not split yet get a slot each while there are any.
+    auto share = [&](uint64_t idle, uint32_t nidle) {
+      const bool fresh = active && sp > 0 && own < 0;
+      const uint64_t fm = __ballot(fresh);
+      if (fresh) {
+        const uint32_t k = nslots + rank_in(fm);
+        if (k < SPLIT_SLOTS) {
+          own = (int)k;
+          ss->key[k] = best >= 0 ? hit_key(bt, best) : ~0ull;
+          ss->tuv[k][0] = bt, ss->tuv[k][1] = bu, ss->tuv[k][2] = bv;
+          ss->ray[k] = ray;
         }
-        const int4 ln = make_int4((int)r3[0], (int)r3[1], (int)r3[2], (int)r3[3]);
-        // near / far planes by the direction's sign (hi is near when 1/d < 0),
-        // two axes and then the third: the planes of all three at once would
-        // hold eight registers more
-        float t0, t1, t2, t3, f0, f1, f2, f3;
-        {
-          const float sx = __uint_as_float(r0[3]) * r.ix, sy = __uint_as_float(r1[0]) * r.iy;
-          const float bx = (__uint_as_float(r0[0]) - r.ox) * r.ix,
-                      by = (__uint_as_float(r0[1]) - r.oy) * r.iy;
-          const float4 nx = wide_planes(r.sx ? r1[3] : r1[2], sx, bx),
-                       fx = wide_planes(r.sx ? r1[2] : r1[3], sx, bx),
-                       ny = wide_planes(r.sy ? r2[1] : r2[0], sy, by),
-                       fy = wide_planes(r.sy ? r2[0] : r2[1], sy, by);
-          t0 = fmaxf(fmaxf(nx.x, ny.x), r.tmin), f0 = fminf(fminf(fx.x, fy.x), bt);
-          t1 = fmaxf(fmaxf(nx.y, ny.y), r.tmin), f1 = fminf(fminf(fx.y, fy.y), bt);
-          t2 = fmaxf(fmaxf(nx.z, ny.z), r.tmin), f2 = fminf(fminf(fx.z, fy.z), bt);
-          t3 = fmaxf(fmaxf(nx.w, ny.w), r.tmin), f3 = fminf(fminf(fx.w, fy.w), bt);
+      }
+      nslots = min(SPLIT_SLOTS, nslots + (uint32_t)__popcll(fm));
+      const bool giver = active && sp > 0 && own >= 0;
+      const uint64_t gm = __ballot(giver);
+      if (gm == 0ull) return;
+      const uint32_t givers = (uint32_t)__popcll(gm);  // < 64: some lanes are idle
+      const float inv = 1.0f / (float)givers;
+      const int lane = lane_now();
+      const uint32_t j = rank_in(gm), rank = rank_in(idle);
+      // lane j of the table: the j-th giver (lane 63 takes the rest)
+      const int table = __builtin_amdgcn_ds_permute((giver ? (int)j : 63) * 4, lane);
+      const uint32_t k = (uint32_t)(((float)rank + 0.5f) * inv);
+      const int from = __builtin_amdgcn_ds_bpermute((int)(rank - k * givers) * 4, table);
+      const int gsp = __shfl(sp, from, 64);
+      const bool help = !active && (int)k < gsp;
+      auto take = [&](auto& x) {
+        const auto y = __shfl(x, from, 64);
+        if (help) x = y;
+      };
+      take(ray), take(own), take(bt), take(r.tmin);
+      take(r.ox), take(r.oy), take(r.oz), take(r.dx), take(r.dy), take(r.dz);
+      take(r.ix), take(r.iy), take(r.iz);
+      r.sx = signbit(r.ix), r.sy = signbit(r.iy), r.sz = signbit(r.iz);
+      if (help) {
+        const int at = gsp - 1 - (int)k;
+        node = s_node[min(at, DEPTH - 1) * BLOCK + (tid - lane + from)];
+        if (at >= DEPTH) node = spilled(at, tid - lane + from)[0];
+        best = -1, sp = 0;
+        active = true;
+      } else if (giver && nidle > j) {
+        const int given = (int)(((float)(nidle - 1u - j) + 0.5f) * inv) + 1;
+        sp -= min(sp, given);
+      }
+    };
+    // ---- traverse until enough lanes are idle to be worth a refill, or, HELP,
+    // with the idle lanes' help until all are (its own copy of the loop: the
+    // slots' reads stay out of the other one) -------------------------------
+    auto walk = [&](auto split) {
+      constexpr bool HELP = decltype(split)::value;
+      for (;;) {
+        if (HELP && active && own >= 0) {  // what the ray's other lanes found
+          const uint32_t hi = (uint32_t)(ss->key[own] >> 32);
+          if (!ANY)
+            bt = fminf(bt, ord_float(hi));  // (a NaN while there is no hit)
+          else if (hi == 0u)
+            finish(split);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        const float sz = __uint_as_float(r1[1]) * r.iz, bz = (__uint_as_float(r0[2]) - r.oz) * r.iz;
-        const float4 nz = wide_planes(r.sz ? r2[3] : r2[2], sz, bz),
-                     fz = wide_planes(r.sz ? r2[2] : r2[3], sz, bz);
-        const bool h0 = slot_hit(nz.x, fz.x, eps, t0, f0) & (ln.x != 0);
-        const bool h1 = slot_hit(nz.y, fz.y, eps, t1, f1) & (ln.y != 0);
-        const bool h2 = slot_hit(nz.z, fz.z, eps, t2, f2) & (ln.z != 0);
-        const bool h3 = slot_hit(nz.w, fz.w, eps, t3, f3) & (ln.w != 0);
-        const int k = (int)h0 + (int)h1 + (int)h2 + (int)h3;
-        // sort the slots by entry distance, misses last: a hit's key is its
-        // distance's bits (ordered for tn >= +0, i.e. tmin >= 0; otherwise
-        // only the visit order suffers), a miss's 0xFFFFFFFF. Any hit: hits
-        // first, distances unused.
-        auto key = [](bool h, float t) -> uint32_t {
-          return h ? (ANY ? 0u : __float_as_uint(t)) : 0xFFFFFFFFu;
-        };
-        uint32_t k0, k1, k2, k3;
-        int32_t c0 = ln.x, c1 = ln.y, c2 = ln.z, c3 = ln.w;
-        if (ANY) {
-          // the same network on the hit flags (every pushed entry is a hit,
-          // key 0)
-          bool g0 = h0, g1 = h1, g2 = h2, g3 = h3;
-          cas_hit(g0, c0, g1, c1), cas_hit(g2, c2, g3, c3);
-          cas_hit(g0, c0, g2, c2), cas_hit(g1, c1, g3, c3);
-          cas_hit(g1, c1, g2, c2);
-          k0 = k1 = k2 = k3 = 0u;
-        } else {
-          k0 = key(h0, t0), k1 = key(h1, t1), k2 = key(h2, t2), k3 = key(h3, t3);
-          cas_pair(k0, c0, k1, c1), cas_pair(k2, c2, k3, c3);
-          cas_pair(k0, c0, k2, c2), cas_pair(k1, c1, k3, c3);
-          cas_pair(k1, c1, k2, c2);
-        }
-        if (k == 0) {
-          if (!pop()) finish();
-        } else {
-          // push the k-1 farther hits, farthest deepest: entry sp+j holds
-          // sorted slot k-1-j; with three LDS entries free all three are
-          // written (entries above the new top are dead)
-          if (k > 1 && sp + 3 <= DEPTH) {
-            const int32_t e0 = k == 4 ? c3 : (k == 3 ? c2 : c1), e1 = k == 4 ? c2 : c1;
-            s_node[sp * BLOCK + tid] = e0;
-            s_node[(sp + 1) * BLOCK + tid] = e1;
-            s_node[(sp + 2) * BLOCK + tid] = c1;
-            if (TSTACK) {
-              const uint32_t d0 = k == 4 ? k3 : (k == 3 ? k2 : k1), d1 = k == 4 ? k2 : k1;
-              s_tn[sp * BLOCK + tid] = __uint_as_float(d0);
-              s_tn[(sp + 1) * BLOCK + tid] = __uint_as_float(d1);
-              s_tn[(sp + 2) * BLOCK + tid] = __uint_as_float(k1);
-            }
-            sp += k - 1;
+        if (WIDE && active && node >= 0) {
+          Row r0, r1, r2, r3;
+          if (!big) {
+            const uint32_t off = (uint32_t)node * (uint32_t)sizeof(WideNode);
+            r0 = row_load<0>(wrs, off), r1 = row_load<16>(wrs, off);
+            r2 = row_load<32>(wrs, off), r3 = row_load<48>(wrs, off);
           } else {
-            if (k > 3) push(c3, __uint_as_float(k3));
-            if (k > 2) push(c2, __uint_as_float(k2));
-            if (k > 1) push(c1, __uint_as_float(k1));
+            const Row* w = reinterpret_cast<const Row*>(a.wide + node);
+            r0 = w[0], r1 = w[1], r2 = w[2], r3 = w[3];
           }
-          node = c0;
-        }
-      } else if (!WIDE && active && node >= 0) {
-        const float4* q = reinterpret_cast<const float4*>(a.nodes + node);
-        const float4 lo0 = q[0], hi0 = q[1], lo1 = q[2], hi1 = q[3];
-        if (COUNT) vis += 2;
-        float tn0, tn1;
-        const bool h0 = slab(lo0, hi0, r, bt, slack, tn0);
-        const bool h1 = slab(lo1, hi1, r, bt, slack, tn1);
-        const int32_t c0 = __float_as_int(lo0.w), c1 = __float_as_int(hi0.w);
-        if (h0 && h1) {
-          const bool swap = tn1 < tn0;
-          push(swap ? c0 : c1, swap ? tn0 : tn1);
-          node = swap ? c1 : c0;
-        } else if (h0) {
-          node = c0;
-        } else if (h1) {
-          node = c1;
-        } else if (!pop()) {
-          finish();
-        }
-      }
-      // leaves reached from here are tested before the next node fetch
-      while (active && node < 0) {
-        const TriRec T = a.tris[~node];
-        if (COUNT) ++tst;
-        float t, u = 0.0f, v = 0.0f;
-        bool done = false, hit;
-        if (SPHERES && a.sphere) {
-          hit = sphere_hit(T, r, bt, t) && (!WIDE || sphere_box(T, r));
-        } else {
-          hit = mt(T, r, bt, t, u, v);
-          if (WIDE && hit && tri_doubt(T, t)) hit = a.nprims < 2u || tri_box(T, r);
-        }
-        if (hit) {
-          const int32_t prim = __float_as_int(T.v0.w);
-          // t <= bt, which is the ray's open end until there is a hit
+          const int4 ln = make_int4((int)r3[0], (int)r3[1], (int)r3[2], (int)r3[3]);
+          // near / far planes by the direction's sign (hi is near when 1/d < 0),
+          // two axes and then the third: the planes of all three at once would
+          // hold eight registers more
+          float t0, t1, t2, t3, f0, f1, f2, f3;
+          {
+            const float sx = __uint_as_float(r0[3]) * r.ix, sy = __uint_as_float(r1[0]) * r.iy;
+            const float bx = (__uint_as_float(r0[0]) - r.ox) * r.ix,
+                        by = (__uint_as_float(r0[1]) - r.oy) * r.iy;
+            const float4 nx = wide_planes(r.sx ? r1[3] : r1[2], sx, bx),
+                         fx = wide_planes(r.sx ? r1[2] : r1[3], sx, bx),
+                         ny = wide_planes(r.sy ? r2[1] : r2[0], sy, by),
+                         fy = wide_planes(r.sy ? r2[0] : r2[1], sy, by);
+            t0 = fmaxf(fmaxf(nx.x, ny.x), r.tmin), f0 = fminf(fminf(fx.x, fy.x), bt);
+            t1 = fmaxf(fmaxf(nx.y, ny.y), r.tmin), f1 = fminf(fminf(fx.y, fy.y), bt);
+            t2 = fmaxf(fmaxf(nx.z, ny.z), r.tmin), f2 = fminf(fminf(fx.z, fy.z), bt);
+            t3 = fmaxf(fmaxf(nx.w, ny.w), r.tmin), f3 = fminf(fminf(fx.w, fy.w), bt);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          const float sz = __uint_as_float(r1[1]) * r.iz, bz = (__uint_as_float(r0[2]) - r.oz) * r.iz;
+          const float4 nz = wide_planes(r.sz ? r2[3] : r2[2], sz, bz),
+                       fz = wide_planes(r.sz ? r2[2] : r2[3], sz, bz);
+          const bool h0 = slot_hit(nz.x, fz.x, eps, t0, f0) & (ln.x != 0);
+          const bool h1 = slot_hit(nz.y, fz.y, eps, t1, f1) & (ln.y != 0);
+          const bool h2 = slot_hit(nz.z, fz.z, eps, t2, f2) & (ln.z != 0);
+          const bool h3 = slot_hit(nz.w, fz.w, eps, t3, f3) & (ln.w != 0);
+          const int k = (int)h0 + (int)h1 + (int)h2 + (int)h3;
+          // sort the slots by entry distance, misses last: a hit's key is its
+          // distance's bits (ordered for tn >= +0, i.e. tmin >= 0; otherwise
+          // only the visit order suffers), a miss's 0xFFFFFFFF. Any hit: hits
+          // first, distances unused.
+          auto key = [](bool h, float t) -> uint32_t {
+            return h ? (ANY ? 0u : __float_as_uint(t)) : 0xFFFFFFFFu;
+          };
+          uint32_t k0, k1, k2, k3;
+          int32_t c0 = ln.x, c1 = ln.y, c2 = ln.z, c3 = ln.w;
           if (ANY) {
-            if (t < bt) best = prim, done = true;
-          } else if (t < bt || (best >= 0 && prim < best)) {
-            best = prim, bt = t, bu = u, bv = v;
+            // the same network on the hit flags (every pushed entry is a hit,
+            // key 0)
+            bool g0 = h0, g1 = h1, g2 = h2, g3 = h3;
+            cas_hit(g0, c0, g1, c1), cas_hit(g2, c2, g3, c3);
+            cas_hit(g0, c0, g2, c2), cas_hit(g1, c1, g3, c3);
+            cas_hit(g1, c1, g2, c2);
+            k0 = k1 = k2 = k3 = 0u;
+          } else {
+            k0 = key(h0, t0), k1 = key(h1, t1), k2 = key(h2, t2), k3 = key(h3, t3);
+            cas_pair(k0, c0, k1, c1), cas_pair(k2, c2, k3, c3);
+            cas_pair(k0, c0, k2, c2), cas_pair(k1, c1, k3, c3);
+            cas_pair(k1, c1, k2, c2);
+          }
+          if (k == 0) {
+            if (!pop()) finish(split);
+          } else {
+            // push the k-1 farther hits, farthest deepest: entry sp+j holds
+            // sorted slot k-1-j; with three LDS entries free all three are
+            // written (entries above the new top are dead)
+            if (k > 1 && sp + 3 <= DEPTH) {
+              const int32_t e0 = k == 4 ? c3 : (k == 3 ? c2 : c1), e1 = k == 4 ? c2 : c1;
+              s_node[sp * BLOCK + tid] = e0;
+              s_node[(sp + 1) * BLOCK + tid] = e1;
+              s_node[(sp + 2) * BLOCK + tid] = c1;
+              if (TSTACK) {
+                const uint32_t d0 = k == 4 ? k3 : (k == 3 ? k2 : k1), d1 = k == 4 ? k2 : k1;
+                s_tn[sp * BLOCK + tid] = __uint_as_float(d0);
+                s_tn[(sp + 1) * BLOCK + tid] = __uint_as_float(d1);
+                s_tn[(sp + 2) * BLOCK + tid] = __uint_as_float(k1);
+              }
+              sp += k - 1;
+            } else {
+              if (k > 3) push(c3, __uint_as_float(k3));
+              if (k > 2) push(c2, __uint_as_float(k2));
+              if (k > 1) push(c1, __uint_as_float(k1));
+            }
+            node = c0;
+          }
+        } else if (!WIDE && active && node >= 0) {
+          const float4* q = reinterpret_cast<const float4*>(a.nodes + node);
+          const float4 lo0 = q[0], hi0 = q[1], lo1 = q[2], hi1 = q[3];
+          if (COUNT) vis += 2;
+          float tn0, tn1;
+          const bool h0 = slab(lo0, hi0, r, bt, slack, tn0);
+          const bool h1 = slab(lo1, hi1, r, bt, slack, tn1);
+          const int32_t c0 = __float_as_int(lo0.w), c1 = __float_as_int(hi0.w);
+          if (h0 && h1) {
+            const bool swap = tn1 < tn0;
+            push(swap ? c0 : c1, swap ? tn0 : tn1);
+            node = swap ? c1 : c0;
+          } else if (h0) {
+            node = c0;
+          } else if (h1) {
+            node = c1;
+          } else if (!pop()) {
+            finish(split);
           }
         }
-        if (done || !pop()) finish();
+        // leaves reached from here are tested before the next node fetch
+        while (active && node < 0) {
+          const TriRec T = a.tris[~node];
+          if (COUNT) ++tst;
+          float t, u = 0.0f, v = 0.0f;
+          bool done = false, hit;
+          if (SPHERES && a.sphere) {
+            hit = sphere_hit(T, r, bt, t) && (!WIDE || sphere_box(T, r));
+          } else {
+            hit = mt(T, r, bt, t, u, v);
+            if (WIDE && hit && tri_doubt(T, t)) hit = a.nprims < 2u || tri_box(T, r);
+          }
+          if (hit) {
+            const int32_t prim = __float_as_int(T.v0.w);
+            // t <= bt, which is the ray's open end until there is a hit
+            if (HELP && own >= 0) {
+              if (ANY) {
+                if (t < bt) ss->key[own] = 0ull, done = true;
+              } else if (t < bt || (uint32_t)(ss->key[own] >> 32) == hit_ord(t)) {
+                const unsigned long long key = hit_key(t, prim);
+                __hip_atomic_fetch_min(&slots->key[own], key, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (ss->key[own] == key)
+                  ss->tuv[own][0] = t, ss->tuv[own][1] = u, ss->tuv[own][2] = v;
+                bt = t;
+              }
+            } else if (ANY) {
+              if (t < bt) best = prim, done = true;
+            } else if (t < bt || (best >= 0 && prim < best)) {
+              best = prim, bt = t, bu = u, bv = v;
+            }
+          }
+          if (done || !pop()) finish(split);
+        }
+        const uint64_t idle = __ballot(!active);
+        const uint32_t nidle = (uint32_t)__popcll(idle);
+        if (nidle == 64u) break;
+        if (!HELP) {
+          if (!wave_out && nidle >= a.refill_idle) break;
+          if (SPLIT && nidle >= SPLIT_IDLE) break;
+        } else if (nidle >= SPLIT_IDLE) {
+          share(idle, nidle);
+        }
       }
-      const uint32_t idle = (uint32_t)__popcll(__ballot(!active));
-      if (idle == 64u || (!wave_out && idle >= a.refill_idle)) break;
+    };
+    walk(std::false_type{});
+    if (SPLIT) {
+      const uint32_t nidle = (uint32_t)__popcll(__ballot(!active));
+      if (nidle != 64u && (wave_out || nidle < a.refill_idle)) {
+        own = -1;
+        walk(std::true_type{});
+      }
     }
   }
 }
 
 // One code path for trees of any size (the batch and serving kernels, whose
 // launches walk many trees and hold their build phases in the same kernel).
-template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES = true,
-          bool WIDE = false, class Src = NoSlices>
-__device__ inline void trace_loop(const TraceArgs& a, const RayStream& rs, int32_t* s_node,
-                                  float* s_tn, uint32_t gtid, uint32_t gstride,
-                                  Src* src = nullptr) {
-  const Schedule sc{a.nrays, a.chunk, 0u, 0u, 1u};
-  trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_ANY, Src>(
-      a, [&] { return &a; }, sc, rs, s_node, s_tn, gtid, gstride, src);
+template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
+          class Src>
+__device__ inline void trace_loop(const TraceArgs& a, Src& src, int32_t* s_node, float* s_tn) {
+  trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_ANY>(
+      a, [&] { return &a; }, src, s_node, s_tn);
 }
 // A path per record addressing, chosen once per launch (the query kernels:
 // one tree).
-template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES = true,
-          bool WIDE = false, class Cold>
-__device__ inline void trace_loop_split(const TraceArgs& a, const Cold& cold, const Schedule& sc,
-                                        const RayStream& rs, int32_t* s_node, float* s_tn,
-                                        uint32_t gtid, uint32_t gstride) {
+template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool WIDE, class Src, class Cold>
+__device__ inline void trace_loop_split(const TraceArgs& a, const Cold& cold, Src& src,
+                                        int32_t* s_node, float* s_tn, SplitSlots* slots) {
   if (WIDE && a.nprims > WIDE_SMALL_MAX_NODES)
-    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_BIG, NoSlices>(
-        a, cold, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
+    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE, ROWS_BIG>(
+        a, cold, src, s_node, s_tn, slots);
   else
-    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_SMALL, NoSlices>(
-        a, cold, sc, rs, s_node, s_tn, gtid, gstride, nullptr);
+    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE, ROWS_SMALL>(
+        a, cold, src, s_node, s_tn, slots);
 }
 
 }  // namespace rq

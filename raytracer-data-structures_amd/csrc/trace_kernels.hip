@@ -33,15 +33,11 @@ void k_trace(TraceArgs a) {
   __shared__ int32_t s_node[DEPTH * BLOCK];
   __shared__ float s_tn[TSTACK ? DEPTH * BLOCK : 1];
   constexpr uint32_t WPB = BLOCK / 64;
-  const Schedule sc = schedule_of(a, gridDim.x * WPB, gridDim.x);
-  RayStream rs;
-  rs.segs = sc.segs;
-  rs.seg = seg_of(blockIdx.x, sc.segs);
-  rs.ctr64 = a.counter + rs.seg * COUNTER_STRIDE;
-  rs.wave = seg_index(blockIdx.x, sc.segs) * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  rs.waves = seg_blocks(rs.seg, sc.segs, gridDim.x) * WPB;
-  trace_loop_split<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE>(
-      a, KernelArgs{}, sc, rs, s_node, s_tn, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK);
+  __shared__ SplitSlots s_split[WIDE ? WPB : 1];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  QuerySlices<KernelArgs, (int)WPB> src(KernelArgs{}, wave);
+  trace_loop_split<ANY, COUNT, BLOCK, DEPTH, TSTACK, WIDE>(a, KernelArgs{}, src, s_node, s_tn,
+                                                           s_split + (WIDE ? wave : 0u));
 }
 
 // Device scratch of the allocation-free closest-hit entry
@@ -76,7 +72,8 @@ struct Variant {
 // each kernel's own occupancy.
 constexpr int wide_waves(int depth, bool tstack) {
   int w = 8;
-  while (w > 1 && w * 4 * 64 * depth * (tstack ? 8 : 4) > 160 * 1024) --w;
+  while (w > 1 && w * 4 * (64 * depth * (tstack ? 8 : 4) + (int)sizeof(SplitSlots)) > 160 * 1024)
+    --w;
   return w;
 }
 // What rq_trace_variant_get promises: six waves or more for the any-hit
@@ -153,9 +150,7 @@ hipError_t launch_trace(const LaunchCtx& lc, const TraceArgs& a, bool any, bool 
   // a wide variant needs the wide nodes
   if (!counted && kVariants[variant].wide && !a.wide) return hipErrorInvalidValue;
   const Variant& V = kVariants[counted ? 0 : variant];
-  uint32_t need = (uint32_t)((a.nrays + V.block - 1) / V.block);
-  uint32_t grid = std::max(1u, std::min(a.grid, need));
-  dim3 g(grid), blk(V.block);
+  dim3 g(a.grid), blk(V.block);
   hipStream_t s = lc.stream;
   if (any) {
     ProfScope ps(lc, counted ? "trace_any_counted" : "trace_any");
