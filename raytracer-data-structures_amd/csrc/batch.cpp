@@ -88,7 +88,7 @@ void push_trace(std::vector<BatchWork>& w, const rq_batch_item& it, uint32_t m, 
 // The work queue: the items of every mesh, phase after phase, tiles in order.
 // Trace items go to BATCH_XCDS segments: meshes are dealt to the segment with
 // the least ray work so far, largest first (LPT), and keep their index order
-// inside a segment.
+// inside a segment; then the segments' bounds are evened out.
 int make_work(rq_ctx* c, rq_batch* b, uint32_t ray_tile) {
   // a captured graph holds this queue's phase bounds in its kernel arguments
   drop_graph(b);
@@ -112,12 +112,12 @@ int make_work(rq_ctx* c, rq_batch* b, uint32_t ray_tile) {
         seg[m] = (uint32_t)q;
         load[q] += work[m];
       }
-      for (int q = 0; q < BATCH_XCDS; ++q) {
-        b->trace_seg[q] = (uint32_t)w.size();
+      const size_t w0 = w.size();
+      for (int q = 0; q < BATCH_XCDS; ++q)
         for (uint32_t m = 0; m < nm; ++m)
           if (seg[m] == (uint32_t)q) push_trace(w, b->items[m], m, ray_tile);
-      }
-      b->trace_seg[BATCH_XCDS] = (uint32_t)w.size();
+      for (int q = 0; q <= BATCH_XCDS; ++q)
+        b->trace_seg[q] = (uint32_t)(w0 + (w.size() - w0) * q / BATCH_XCDS);
       continue;
     }
     for (uint32_t m = 0; m < nm; ++m) {
@@ -176,9 +176,11 @@ int launch(rq_ctx* c, rq_batch* b, hipStream_t s, bool profile) {
   }
   LaunchCtx lc = launch_ctx(c, s);
   if (!profile) lc.prof = nullptr;
-  hipError_t e =
-      launch_batch(lc, batch_args(b), b->build, b->build_grid[b->build], b->variant,
-                   b->grid[b->variant]);
+  // no more trace blocks than there are items for their waves
+  const uint32_t items = b->trace_seg[BATCH_XCDS] - b->trace_seg[0];
+  const uint32_t grid = std::min(b->grid[b->variant],
+                                 std::max(1u, tiles_of(items, BATCH_XCDS * BUILD_BLOCK / 64)) * BATCH_XCDS);
+  hipError_t e = launch_batch(lc, batch_args(b), b->build, b->build_grid[b->build], b->variant, grid);
   return e == hipSuccess ? RQ_OK : hip_err(c, e, "batch launch");
 }
 

@@ -21,8 +21,9 @@ enum BatchPhase {
 };
 
 // The trace items are split into one queue segment per XCD (each XCD has its
-// own L2): a mesh's rays are traced on one XCD so its BVH stays in that L2;
-// a block drains its own XCD's segment first, then takes from the others.
+// own L2): a mesh's rays are traced on one XCD, or two, so that its BVH stays
+// in those L2s; a block drains its own XCD's segment first, then takes from
+// the others.
 constexpr int BATCH_XCDS = 8;
 
 // control words of one batch
@@ -30,22 +31,23 @@ constexpr int BATCH_CTL_TICKET = 0;                        // BATCH_PHASES queue
 constexpr int BATCH_CTL_BARRIER = BATCH_PHASES;            // grid barrier arrivals
 constexpr int BATCH_CTL_BARRIER_ERR = BATCH_PHASES + 1;    // barrier wait gave up (this run)
 constexpr int BATCH_CTL_TRACE_ERR = BATCH_PHASES + 2;      // stack deeper than provided (this run)
-constexpr int BATCH_CTL_XTICKET = BATCH_PHASES + 3;        // BATCH_XCDS trace segment tickets
-constexpr int BATCH_CTL_START = BATCH_CTL_XTICKET + BATCH_XCDS;  // blocks started (+ BATCH_CLOSED)
+constexpr int BATCH_CTL_START = BATCH_PHASES + 3;          // blocks started (+ BATCH_CLOSED)
 constexpr int BATCH_CTL_MEMBERS = BATCH_CTL_START + 1;     // blocks taking part (0 until closed)
 // BATCH_PHASES 64-bit wall-clock stamps (8-byte aligned) of the build kernel:
-// stamp 0 = the first member's start, stamp p = phase p - 1 done (the last
-// member through barrier p, or out of the kernel after the last phase)
+// stamp 0 = the first member's start, stamp p = phase p - 1 done (its last
+// member's arrival)
 constexpr int BATCH_CTL_CLOCK = (BATCH_CTL_MEMBERS + 2) & ~1;
 constexpr int BATCH_CTL_WORDS = BATCH_CTL_CLOCK + 2 * BATCH_PHASES;
 // The grid barrier's group words, after the control words: BATCH_BAR_GROUPS
 // arrival counters, then as many release words, each word on a 4 KB page of
 // its own, so that the arrivals and polls of different groups are served by
-// different memory channels rather than queueing on one word.
+// different memory channels rather than queueing on one word (12 ns an atomic).
+// The tickets of the trace segments follow, spread the same way.
 constexpr int BATCH_BAR_GROUPS = 16;
 constexpr int BATCH_BAR_STRIDE = 1024;  // words
 constexpr int BATCH_BAR_BASE = BATCH_BAR_STRIDE;
-constexpr int BATCH_CTL_ALLOC_WORDS = BATCH_BAR_BASE + 2 * BATCH_BAR_GROUPS * BATCH_BAR_STRIDE;
+constexpr int BATCH_XTICKET_BASE = BATCH_BAR_BASE + 2 * BATCH_BAR_GROUPS * BATCH_BAR_STRIDE;
+constexpr int BATCH_CTL_ALLOC_WORDS = BATCH_XTICKET_BASE + BATCH_XCDS * BATCH_BAR_STRIDE;
 static_assert(BATCH_CTL_WORDS <= BATCH_BAR_BASE, "control words before the barrier groups");
 constexpr uint32_t BATCH_CLOSED = 0x80000000u;             // start word: membership closed
 constexpr uint32_t BATCH_ANY_BIT = 0x80000000u;            // trace item tile: any-hit query

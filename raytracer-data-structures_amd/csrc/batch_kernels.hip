@@ -16,9 +16,6 @@
 namespace rq {
 namespace {
 
-// s_getreg operand of HW_REG_XCC_ID (register 20, bits [3:0]): the XCD id.
-constexpr int XCC_ID_HWREG = 20 | (0 << 6) | ((4 - 1) << 11);
-
 // About 4M polls (a few seconds): far beyond any phase of the member blocks.
 constexpr uint32_t BARRIER_SPIN_LIMIT = 1u << 22;
 // Polls the first barrier waits for the rest of the grid to start before it
@@ -57,21 +54,36 @@ __device__ inline unsigned long long* clock_stamp(uint32_t* ctl, uint32_t k) {
   return reinterpret_cast<unsigned long long*>(ctl + BATCH_CTL_CLOCK) + k;
 }
 
+// Counts the block's arrival at the end of phase `phases_done` - 1 on its
+// group's counter (group = ticket mod BATCH_BAR_GROUPS), the group's last
+// arrival on the top counter; true for the grid's last, which stamps the phase.
+// The counters are cumulative over the launch, so the last arrival of phase p
+// is the one that brings a counter to p times its members.
+__device__ inline bool arrived_last(uint32_t* ctl, uint32_t phases_done, uint32_t members,
+                                    uint32_t g, uint32_t old) {
+  constexpr uint32_t G = BATCH_BAR_GROUPS;
+  const uint32_t groups = min(members, G), in_group = (members - g + G - 1u) / G;
+  if (old + 1u != in_group * phases_done) return false;
+  __threadfence();
+  if (atomicAdd(ctl + BATCH_CTL_BARRIER, 1u) + 1u != groups * phases_done) return false;
+  *clock_stamp(ctl, phases_done) = (unsigned long long)wall_clock64();
+  return true;
+}
+
 // Grid barrier after phase `phases_done` - 1. The block's waves meet at a
 // work-group barrier, which leaves their stores in the XCD's L2; thread 0's
 // agent-scope release then writes that L2 back (one write-back per block
-// rather than one per wave), and it counts the block on its group's counter
-// (group = ticket mod BATCH_BAR_GROUPS). The group's last arrival counts the
-// group on the top counter, and the top's last arrival publishes the phase
-// on every group's release word; each block waits on its own group's word
-// and acquires. The counters are cumulative over the launch, so the last
-// arrival of phase p is the one that brings a counter to p times its
-// members. One word shared by every block, for the arrivals and for the
-// polls, had made each barrier cost ~0.15-0.3 ms on a full grid. The
-// members are running, so every wait ends; it is bounded all the same: a
+// rather than one per wave), and it counts the block's arrival. The grid's
+// last arrival publishes the phase on every group's release word; each block
+// waits on its own group's word and acquires. One word shared by every block,
+// for the arrivals and for the polls, had made each barrier cost ~0.15-0.3 ms
+// on a full grid; a time stamp of every block on one word still cost it 25 us.
+// The members are running, so every wait ends; it is bounded all the same: a
 // wait that gives up sets the sticky error word, and once it is set no later
-// barrier of the launch waits at all.
-__device__ inline void grid_barrier(uint32_t* ctl, uint32_t phases_done, uint32_t ticket) {
+// barrier of the launch waits at all. Returns the number of members (0 if the
+// wait for it gave up).
+__device__ inline uint32_t grid_barrier(uint32_t* ctl, uint32_t phases_done, uint32_t ticket,
+                                        uint32_t* s_flag) {
   __syncthreads();
   if (threadIdx.x == 0) {
     __threadfence();
@@ -98,14 +110,9 @@ __device__ inline void grid_barrier(uint32_t* ctl, uint32_t phases_done, uint32_
       }
     }
     if (members != 0u) {
-      constexpr uint32_t G = BATCH_BAR_GROUPS;
-      const uint32_t groups = min(members, G), in_group = (members - g + G - 1u) / G;
-      if (old + 1u == in_group * phases_done) {  // the group's last arrival
-        __threadfence();
-        if (atomicAdd(ctl + BATCH_CTL_BARRIER, 1u) + 1u == groups * phases_done) {
-          __threadfence();  // the grid's last arrival: release every group
-          for (uint32_t k = 0; k < G; ++k) atomicMax(bar_release(ctl, k), phases_done);
-        }
+      if (arrived_last(ctl, phases_done, members, g, old)) {
+        __threadfence();  // the grid's last arrival: release every group
+        for (uint32_t k = 0; k < BATCH_BAR_GROUPS; ++k) atomicMax(bar_release(ctl, k), phases_done);
       }
       uint32_t spins = 0;
       while (ld_agent(bar_release(ctl, g)) < phases_done) {
@@ -117,9 +124,22 @@ __device__ inline void grid_barrier(uint32_t* ctl, uint32_t phases_done, uint32_
       }
     }
     __threadfence();
-    atomicMax(clock_stamp(ctl, phases_done), (unsigned long long)wall_clock64());
+    *s_flag = members;
   }
   __syncthreads();
+  const uint32_t members = *s_flag;
+  __syncthreads();
+  return members;
+}
+
+// The next item of a queue of n items whose first `owned` are taken without a
+// ticket, by the unit (block or wave) of their number: its number, or n or
+// more. An atomic on one word takes 12 ns, and each unit used to end every
+// queue with a failed one, so the word is read first: an empty queue costs a
+// load, one whose items all have an owner nothing.
+__device__ inline uint32_t next_item(uint32_t* ticket, uint32_t owned, uint32_t n) {
+  if (owned >= n || owned + ld_agent(ticket) >= n) return n;
+  return owned + atomicAdd(ticket, 1u);
 }
 
 // Loads a block-uniform descriptor into scalar registers: every dword goes
@@ -138,11 +158,10 @@ __device__ inline T load_uniform(const T* p) {
   return t;
 }
 
-// One trace item (a tile of one mesh's rays): a ray counter in LDS hands out
-// chunks of the tile as lanes go idle. WAVE_ITEM: one wave takes the item on
-// its own (its own counter, no block barrier at either end); otherwise the
-// block's waves share it and meet at a barrier when it is done.
-template <int DEPTH, bool TSTACK, bool WIDE, bool WAVE_ITEM>
+// One trace item (a tile of one mesh's rays), shared by the block's waves: a
+// ray counter in LDS hands out chunks of the tile as lanes go idle; the waves
+// meet at a barrier when it is done.
+template <int DEPTH, bool TSTACK, bool WIDE>
 __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* err,
                                   uint32_t ray_tile, uint32_t refill_idle, const BatchMeshDev& m,
                                   uint32_t tile, uint32_t* lds, uint32_t* s_ctr) {
@@ -162,13 +181,8 @@ __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* er
   t.err = err;
   t.refill_idle = refill_idle;
   t.sphere = 0;  // batch meshes are triangle scenes
-  if (WAVE_ITEM) {
-    // lane 0 resets the counter and is the lane that takes from it (trace_loop)
-    if ((threadIdx.x & 63) == 0) *s_ctr = 0u;
-  } else {
-    if (threadIdx.x == 0) *s_ctr = 0u;
-    __syncthreads();
-  }
+  if (threadIdx.x == 0) *s_ctr = 0u;
+  __syncthreads();
   int32_t* s_node = reinterpret_cast<int32_t*>(lds);
   float* s_tn = reinterpret_cast<float*>(lds + DEPTH * BUILD_BLOCK);
   ItemRays src{s_ctr, nr};
@@ -182,8 +196,36 @@ __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* er
     t.v = m.v_ ? m.v_ + r0 : nullptr;
     trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE>(t, src, s_node, s_tn);
   }
-  if (!WAVE_ITEM) __syncthreads();
+  __syncthreads();
 }
+
+// The trace items a unit (a wave, or a block whose waves share an item) takes:
+// the item of its own number in its XCD's segment, then by ticket what has no
+// owner, its own segment first. Blocks go to the XCDs in turn. One lane's.
+constexpr uint32_t NO_ITEM = ~0u;
+template <uint32_t PER_BLOCK>
+struct SegQueue {
+  uint32_t index;   // the unit's number in its segment
+  uint32_t k = 0;   // cursor: segment (XCD + k) % BATCH_XCDS
+  bool own = true;  // its own item not taken yet
+  __device__ explicit SegQueue(uint32_t unit)
+      : index(seg_index(blockIdx.x, BATCH_XCDS) * PER_BLOCK + unit) {}
+  __device__ uint32_t take(const BatchArgs& a) {
+    for (; k < (uint32_t)BATCH_XCDS; ++k) {
+      const uint32_t q = (blockIdx.x + k) % BATCH_XCDS;
+      const uint32_t b0 = a.trace_seg[q], n = a.trace_seg[q + 1] - b0;
+      if (own) {
+        own = false;
+        if (index < n) return b0 + index;
+      }
+      const uint32_t it = next_item(a.ctl + BATCH_XTICKET_BASE + q * BATCH_BAR_STRIDE,
+                                    seg_blocks(q, BATCH_XCDS, gridDim.x) * PER_BLOCK, n);
+      if (it < n) return b0 + it;
+    }
+    return NO_ITEM;
+  }
+};
+typedef SegQueue<BUILD_BLOCK / 64> SegItems;
 
 // Slices of one wave's walk over one mesh and query kind (the batch run): the
 // tile of the item the walk starts with, then the tiles of the items the wave
@@ -194,25 +236,18 @@ __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* er
 // walk and starts the next one.
 struct ItemSlices {
   const BatchArgs& args;
-  uint32_t xcd, k;  // segment cursor: segment (xcd + k) % BATCH_XCDS
+  SegItems seg;
   uint32_t mesh, kind, nrays;
   BatchWork held;   // the walk's first item, then the item that ended it
   bool first, have_held;
-  // The wave's next item, its own XCD's segment first (every lane active).
+  // The wave's next item (every lane active).
   __device__ bool take(BatchWork& w) {
-    for (; k < (uint32_t)BATCH_XCDS; ++k) {
-      const uint32_t q = (xcd + k) % BATCH_XCDS;
-      const uint32_t b0 = args.trace_seg[q], b1 = args.trace_seg[q + 1];
-      if (b1 == b0) continue;
-      uint32_t it = 0;
-      if ((threadIdx.x & 63u) == 0) it = b0 + atomicAdd(args.ctl + BATCH_CTL_XTICKET + q, 1u);
-      it = __builtin_amdgcn_readfirstlane(it);
-      if (it < b1) {
-        w = load_uniform(args.items + it);
-        return true;
-      }
-    }
-    return false;
+    uint32_t it = 0;
+    if ((threadIdx.x & 63u) == 0) it = seg.take(args);
+    it = __builtin_amdgcn_readfirstlane(it);
+    if (it == NO_ITEM) return false;
+    w = load_uniform(args.items + it);
+    return true;
   }
   __device__ bool next(uint32_t& b, uint32_t& e) {
     BatchWork w;
@@ -263,12 +298,22 @@ __device__ inline void trace_mesh(const BatchArgs& a, const BatchMeshDev& m, uin
   }
 }
 
-// The batch build's refit chunks: one leaf per thread of a block. A work
-// item of the refit phase covers BATCH_REFIT_CHUNKS chunks, one of the
-// spanning-node phases BATCH_SPAN_TILES tiles of BUILD_BLOCK internal nodes:
-// every item costs a ticket, an atomic on one word that all blocks share,
-// and items of a single chunk or tile made the phases wait on those tickets.
+// The batch build's refit chunks: one leaf per thread of a block. The queue's
+// items are larger than that (BATCH_REFIT_CHUNKS chunks, BATCH_SPAN_TILES
+// tiles of BUILD_BLOCK internal nodes, ...); the blocks share each item of
+// phase ph in phase_parts(ph) parts, so that the last round of a phase is a
+// small part of it: 1.5 M triangles in 48 meshes are 385 to 1476 items, for
+// 1280 blocks.
 constexpr int BATCH_REFIT_CHUNK = BUILD_BLOCK;
+constexpr uint32_t BOUNDS_PARTS = 4, KARRAS_PARTS = 8, SPAN_PARTS = 4;
+__device__ inline uint32_t phase_parts(int ph) {
+  return ph == PH_BOUNDS  ? BOUNDS_PARTS
+         : ph == PH_KARRAS ? KARRAS_PARTS
+         : ph == PH_REFIT  ? BATCH_REFIT_CHUNKS
+         : ph == PH_TOP || ph == PH_WIDEN ? SPAN_PARTS
+                                          : 1u;
+}
+
 
 // LDS words of the batch kernel: the build kernel's largest phase (lean sort
 // tile, Morton histograms, refit chunk), the trace kernel's stack.
@@ -276,7 +321,7 @@ constexpr int cmax(int x, int y) { return x > y ? x : y; }
 constexpr int batch_lds_words(bool build, int depth, bool tstack) {
   return build ? cmax(cmax(cmax(sort_lds_words(SORT_ITEMS_LEAN), SORT_PASSES * 256),
                            refit_chunk_lds_words<BATCH_REFIT_CHUNK>()),
-                      karras_lds_words<NODE_TILE>())
+                      karras_lds_words<NODE_TILE / KARRAS_PARTS>())
                : depth * BUILD_BLOCK * (tstack ? 2 : 1);
 }
 
@@ -293,19 +338,17 @@ template <int DEPTH, bool TSTACK, int WAVES, KernelMode MODE, bool WIDE, bool WA
 __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_batch(
     BatchArgs a) {
   __shared__ uint32_t lds[batch_lds_words(MODE == KM_BUILD, DEPTH, TSTACK)];
-  __shared__ uint32_t s_item, s_wctr[BUILD_BLOCK / 64];
+  __shared__ uint32_t s_item, s_ctr;
   uint32_t* const ctl = a.ctl;
   const BatchWork* const items = a.items;
   const BatchMeshDev* const meshes = a.meshes;
   if constexpr (MODE == KM_TRACE) {
-    // Trace items from the XCD's segment first (the XCD comes from a hardware
-    // register; any value is safe: every segment is drained). WAVE_ITEMS
-    // (the batch run): waves take items on their own and never wait for the
-    // rest of their block; otherwise (the serving step, whose tiles are sized
-    // for a block) a block takes an item and its waves share it.
-    const uint32_t xcd = __builtin_amdgcn_s_getreg(XCC_ID_HWREG) % BATCH_XCDS;
+    // WAVE_ITEMS (the batch run): waves take items on their own and never wait
+    // for the rest of their block; otherwise (the serving step, whose tiles are
+    // sized for a block) a block takes an item and its waves share it.
     if constexpr (WAVE_ITEMS) {
-      ItemSlices src{a, xcd, 0u, 0u, 0u, 0u, BatchWork{}, false, false};
+      ItemSlices src{a, SegItems(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), 0u, 0u, 0u,
+                     BatchWork{}, false, false};
       if (!src.take(src.held)) return;
       for (;;) {
         const BatchMeshDev m = load_uniform(meshes + src.held.mesh);
@@ -314,31 +357,18 @@ __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAV
         trace_mesh<DEPTH, TSTACK, WIDE>(a, m, lds, &src);
         if (!src.have_held) return;
       }
-    }
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (int k = 0; k < BATCH_XCDS; ++k) {
-      const uint32_t q = (xcd + (uint32_t)k) % BATCH_XCDS;
-      const uint32_t b0 = a.trace_seg[q], b1 = a.trace_seg[q + 1];
-      if (b1 == b0) continue;
-      uint32_t* const ticket = ctl + BATCH_CTL_XTICKET + q;
+    } else {
+      SegQueue<1> queue(0u);
       for (;;) {
-        uint32_t it = 0;
-        if (WAVE_ITEMS) {
-          if (lane == 0) it = b0 + atomicAdd(ticket, 1u);
-          it = __builtin_amdgcn_readfirstlane(it);  // every lane is active here
-        } else {
-          if (threadIdx.x == 0) s_item = b0 + atomicAdd(ticket, 1u);
-          __syncthreads();
-          it = __builtin_amdgcn_readfirstlane(s_item);
-          __syncthreads();
-        }
-        if (it >= b1) break;
+        if (threadIdx.x == 0) s_item = queue.take(a);
+        __syncthreads();
+        const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
+        __syncthreads();
+        if (it == NO_ITEM) return;
         const BatchWork w = load_uniform(items + it);
         const BatchMeshDev m = load_uniform(meshes + w.mesh);
-        trace_item<DEPTH, TSTACK, WIDE, WAVE_ITEMS>(a.gstack, a.gdepth,
-                                                    ctl + BATCH_CTL_TRACE_ERR, a.ray_tile,
-                                                    a.refill_idle, m, w.tile, lds,
-                                                    s_wctr + (WAVE_ITEMS ? wave : 0u));
+        trace_item<DEPTH, TSTACK, WIDE>(a.gstack, a.gdepth, ctl + BATCH_CTL_TRACE_ERR, a.ray_tile,
+                                        a.refill_idle, m, w.tile, lds, &s_ctr);
       }
     }
     return;
@@ -347,22 +377,34 @@ __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAV
   // blocks the device places after the membership closed take no part
   const uint32_t ticket = join_grid(ctl, &s_item);
   if (ticket == ~0u) return;
-  if (threadIdx.x == 0) atomicMin(clock_stamp(ctl, 0), (unsigned long long)wall_clock64());
-  constexpr int first = 0, last = (int)PH_TRACE;
-  for (int ph = first; ph < last; ++ph) {
+  if (ticket == 0u && threadIdx.x == 0)
+    *clock_stamp(ctl, 0) = (unsigned long long)wall_clock64();
+  // The blocks take a phase's parts in turn: part k is block (k mod members)'s,
+  // without a ticket. (A sort tile waits on the tiles before it: every block
+  // takes its own in ascending order.) The blocks of the first phase are not
+  // counted yet: its items go by ticket.
+  uint32_t members = 0;
+  constexpr int last = (int)PH_TRACE;
+  for (int ph = 0; ph < last; ++ph) {
    {
     // kernarg words, block-uniform
-    const uint32_t b0 = a.phase_begin[ph], b1 = a.phase_begin[ph + 1];
-    uint32_t* const ticket = ctl + BATCH_CTL_TICKET + ph;
+    const uint32_t b0 = a.phase_begin[ph], parts = phase_parts(ph);
+    const uint32_t units = (a.phase_begin[ph + 1] - b0) * parts;
+    uint32_t unit = ticket - members;
     for (;;) {
-      if (b1 == b0) break;
-      if (threadIdx.x == 0) s_item = b0 + atomicAdd(ticket, 1u);
-      __syncthreads();
+      if (members != 0u) {
+        unit += members;
+      } else {
+        if (threadIdx.x == 0) s_item = next_item(ctl + BATCH_CTL_TICKET + ph, 0u, units);
+        __syncthreads();
+        unit = s_item;
+        __syncthreads();
+      }
       // block-uniform: keep the item and its mesh descriptor in scalar registers
-      const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
-      __syncthreads();
-      if (it >= b1) break;
-      const BatchWork w = load_uniform(items + it);
+      unit = __builtin_amdgcn_readfirstlane(unit);
+      if (unit >= units) break;
+      const uint32_t part = unit % parts;
+      const BatchWork w = load_uniform(items + b0 + unit / parts);
       const BatchMeshDev* const mp = meshes + w.mesh;
       // each phase loads the descriptor itself: fields it does not read are
       // never loaded and hold no scalar registers
@@ -370,16 +412,20 @@ __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAV
       switch (ph) {
         case PH_INIT: {
           VIEW;
-          build_init_part(v, threadIdx.x, BUILD_BLOCK);
+          build_init_misc(v, threadIdx.x, BUILD_BLOCK);
           break;
         }
         case PH_BOUNDS: {
           VIEW;
-          bounds_tile(v, w.tile, lds);
+          bounds_tile<BUILD_BLOCK, TRI_TILE / BOUNDS_PARTS>(v, w.tile * BOUNDS_PARTS + part, lds);
           break;
         }
         case PH_MORTON: {
           VIEW;
+          // the sort's look-back words, a part a tile (in the init phase's one
+          // item a mesh they took 0.1 ms of one block)
+          build_init_status(v, w.tile * BUILD_BLOCK + threadIdx.x,
+                            tiles_of(v.n, TRI_TILE) * BUILD_BLOCK);
           morton_tile(v, w.tile, lds);
           break;
         }
@@ -405,29 +451,25 @@ __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAV
         }
         case PH_KARRAS: {
           VIEW;
-          karras_tile(v, w.tile, lds);
+          karras_tile<NODE_TILE / KARRAS_PARTS>(v, w.tile * KARRAS_PARTS + part, lds);
           break;
         }
         case PH_REFIT: {  // chunk-union refit, pass 1 (with the chunks' wide records)
           VIEW;
-          for (uint32_t c = 0; c < (uint32_t)BATCH_REFIT_CHUNKS; ++c) {
-            const uint32_t chunk = w.tile * BATCH_REFIT_CHUNKS + c;
-            if (chunk * BATCH_REFIT_CHUNK >= v.n) break;
-            refit_chunk_tile<BATCH_REFIT_CHUNK>(v, chunk, lds);
-            __syncthreads();  // the chunk's LDS is read to the end before the next one
-          }
+          const uint32_t chunk = w.tile * BATCH_REFIT_CHUNKS + part;
+          if (chunk * BATCH_REFIT_CHUNK < v.n) refit_chunk_tile<BATCH_REFIT_CHUNK>(v, chunk, lds);
           break;
         }
         case PH_TOP: {  // pass 2: the nodes spanning chunks, a wave per 64 nodes
           VIEW;
-          for (uint32_t t = 0; t < (uint32_t)BATCH_SPAN_TILES; ++t)
+          for (uint32_t t = part; t < (uint32_t)BATCH_SPAN_TILES; t += SPAN_PARTS)
             refit_span_wave<BATCH_REFIT_CHUNK>(
                 v.B, v.n, (w.tile * BATCH_SPAN_TILES + t) * BUILD_BLOCK + threadIdx.x);
           break;
         }
         case PH_WIDEN: {  // wide records of the spanning nodes
           VIEW;
-          for (uint32_t t = 0; t < (uint32_t)BATCH_SPAN_TILES; ++t) {
+          for (uint32_t t = part; t < (uint32_t)BATCH_SPAN_TILES; t += SPAN_PARTS) {
             const uint32_t i = (w.tile * BATCH_SPAN_TILES + t) * BUILD_BLOCK + threadIdx.x;
             if (i + 1u < v.n && spans_chunks<BATCH_REFIT_CHUNK>(v.B, i)) widen_global(v.B, i);
           }
@@ -440,9 +482,12 @@ __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAV
       __syncthreads();
     }
    }
-    if (ph + 1 < last) grid_barrier(ctl, (uint32_t)(ph + 1), ticket);
+    if (ph + 1 < last) members = grid_barrier(ctl, (uint32_t)(ph + 1), ticket, &s_item);
   }
-  if (threadIdx.x == 0) atomicMax(clock_stamp(ctl, last), (unsigned long long)wall_clock64());
+  if (threadIdx.x == 0 && members != 0u) {
+    const uint32_t g = ticket % (uint32_t)BATCH_BAR_GROUPS;
+    arrived_last(ctl, (uint32_t)last, members, g, atomicAdd(bar_group(ctl, g), 1u));
+  }
 }
 
 // Clears the queue tickets, the barrier and the error words before a run (a
@@ -450,10 +495,11 @@ __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAV
 __global__ void k_batch_reset(uint32_t* ctl) {
   static_assert(BATCH_CTL_WORDS <= 64 && 2 * BATCH_BAR_GROUPS <= 64,
                 "one 64-thread block clears the control and barrier words");
-  // the start stamp is a minimum: it starts at the largest value
+  // no start stamp yet: the largest value
   const bool start = threadIdx.x == BATCH_CTL_CLOCK || threadIdx.x == BATCH_CTL_CLOCK + 1;
   if (threadIdx.x < BATCH_CTL_WORDS) ctl[threadIdx.x] = start ? 0xFFFFFFFFu : 0u;
   if (threadIdx.x < 2 * BATCH_BAR_GROUPS) *bar_group(ctl, threadIdx.x) = 0u;
+  if (threadIdx.x < BATCH_XCDS) ctl[BATCH_XTICKET_BASE + threadIdx.x * BATCH_BAR_STRIDE] = 0u;
 }
 
 typedef void (*BatchFn)(BatchArgs);

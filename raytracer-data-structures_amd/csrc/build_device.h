@@ -117,10 +117,8 @@ __host__ __device__ inline uint32_t tiles_of(uint32_t n, uint32_t tile) {
 
 // ---- phase 0: reset the build's counters, histograms and look-back words --------
 // Threads [first, first + stride) of the caller's grid share the work.
-__device__ inline void build_init_part(const BuildView& v, uint32_t first, uint32_t stride) {
+__device__ inline void build_init_misc(const BuildView& v, uint32_t first, uint32_t stride) {
   uint32_t* misc = v.B.misc;
-  const uint32_t nstatus = SORT_PASSES * tiles_of(v.n, SORT_TILE_LEAN) * 256;  // both tilings
-  for (uint32_t k = first; k < nstatus; k += stride) v.B.status[k] = 0u;
   for (uint32_t k = first; k < (uint32_t)MISC_BOUNDS; k += stride) misc[k] = 0u;  // hist, tickets
   if (first == 0) misc[MISC_ERR] = 0u, misc[MISC_HEIGHT] = HEIGHT_UNKNOWN;
   if (first < 3) {
@@ -128,18 +126,39 @@ __device__ inline void build_init_part(const BuildView& v, uint32_t first, uint3
     misc[MISC_BOUNDS + 3 + first] = 0u;        // hi (ordered max)
   }
 }
+__device__ inline void build_init_status(const BuildView& v, uint32_t first, uint32_t stride) {
+  const uint32_t nstatus = SORT_PASSES * tiles_of(v.n, SORT_TILE_LEAN) * 256;  // both tilings
+  for (uint32_t k = first; k < nstatus; k += stride) v.B.status[k] = 0u;
+}
+__device__ inline void build_init_part(const BuildView& v, uint32_t first, uint32_t stride) {
+  build_init_status(v, first, stride);
+  build_init_misc(v, first, stride);
+}
+
+// The centroids of primitives t, t + BLOCK, ... below end (the last one again
+// past it): their index and vertex fetches are in flight together.
+constexpr int CENTROIDS = 4;
+template <int BLOCK>
+__device__ inline void centroids(const BuildView& v, uint32_t t, uint32_t end, float3* c) {
+#pragma unroll
+  for (int j = 0; j < CENTROIDS; ++j) c[j] = centroid(v, min(t + j * BLOCK, end - 1u));
+}
 
 // ---- phase 1: centroid bounds of one tile (SCENE_AABB map) ------------------------
-template <int BLOCK = BUILD_BLOCK>
+template <int BLOCK = BUILD_BLOCK, int TILE = TRI_TILE>
 __device__ inline void bounds_tile(const BuildView& v, uint32_t tile, uint32_t* lds) {
   constexpr int W = BLOCK / 64;  // waves; lds holds 6 * W words
   uint32_t lo[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, hi[3] = {0u, 0u, 0u};
-  const uint32_t end = min((tile + 1) * (uint32_t)TRI_TILE, v.n);
-  for (uint32_t t = tile * TRI_TILE + threadIdx.x; t < end; t += BLOCK) {
-    const float3 c = centroid(v, t);
-    const uint32_t o[3] = {f2ord(c.x), f2ord(c.y), f2ord(c.z)};
+  const uint32_t end = min((tile + 1) * (uint32_t)TILE, v.n);
+  for (uint32_t t = tile * TILE + threadIdx.x; t < end; t += CENTROIDS * BLOCK) {
+    float3 c[CENTROIDS];
+    centroids<BLOCK>(v, t, end, c);  // (a clamped index repeats one: no harm)
 #pragma unroll
-    for (int k = 0; k < 3; ++k) lo[k] = min(lo[k], o[k]), hi[k] = max(hi[k], o[k]);
+    for (int j = 0; j < CENTROIDS; ++j) {
+      const uint32_t o[3] = {f2ord(c[j].x), f2ord(c[j].y), f2ord(c[j].z)};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) lo[k] = min(lo[k], o[k]), hi[k] = max(hi[k], o[k]);
+    }
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -155,13 +174,15 @@ __device__ inline void bounds_tile(const BuildView& v, uint32_t tile, uint32_t* 
     for (int k = 0; k < 3; ++k) lds[k * W + wave] = lo[k], lds[(3 + k) * W + wave] = hi[k];
   }
   __syncthreads();
-  if (threadIdx.x < 6) {  // one device atomic per bound per tile
+  if (threadIdx.x < 6) {  // at most one device atomic per bound per tile: they
+                          // queue on one line, so one that changes nothing is left out
     const int k = threadIdx.x;
     uint32_t m = lds[k * W];
     for (int w = 1; w < W; ++w) m = k < 3 ? min(m, lds[k * W + w]) : max(m, lds[k * W + w]);
-    if (k < 3)
+    const uint32_t now = ld_agent(&v.B.misc[MISC_BOUNDS + k]);
+    if (k < 3 && m < now)
       atomicMin(&v.B.misc[MISC_BOUNDS + k], m);
-    else
+    else if (k >= 3 && m > now)
       atomicMax(&v.B.misc[MISC_BOUNDS + k], m);
   }
   __syncthreads();
@@ -182,21 +203,26 @@ __device__ inline void morton_tile(const BuildView& v, uint32_t tile, uint32_t* 
   }
   __syncthreads();
   const uint32_t end = min((tile + 1) * (uint32_t)TRI_TILE, v.n);
-  for (uint32_t t = tile * TRI_TILE + threadIdx.x; t < end; t += BLOCK) {
-    const float3 c = centroid(v, t);
-    float q[3] = {c.x, c.y, c.z};
+  for (uint32_t t = tile * TRI_TILE + threadIdx.x; t < end; t += CENTROIDS * BLOCK) {
+    float3 c[CENTROIDS];
+    centroids<BLOCK>(v, t, end, c);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      if (v.mode == RQ_MORTON_SCENE_AABB)
-        q[k] = ext[k] > 0.0f ? (q[k] - lo[k]) / ext[k] : 0.0f;
-      else
-        q[k] = (q[k] + 30.0f) / 1000.0f;
+    for (int j = 0; j < CENTROIDS; ++j) {
+      if (t + j * BLOCK >= end) break;
+      float q[3] = {c[j].x, c[j].y, c[j].z};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        if (v.mode == RQ_MORTON_SCENE_AABB)
+          q[k] = ext[k] > 0.0f ? (q[k] - lo[k]) / ext[k] : 0.0f;
+        else
+          q[k] = (q[k] + 30.0f) / 1000.0f;
+      }
+      const uint32_t code = morton30(q[0], q[1], q[2]);
+      v.B.codes[t + j * BLOCK] = code;
+#pragma unroll
+      for (int p = 0; p < SORT_PASSES; ++p)
+        atomicAdd(&s_hist[p * 256 + ((code >> (8 * p)) & 255u)], 1u);
     }
-    const uint32_t code = morton30(q[0], q[1], q[2]);
-    v.B.codes[t] = code;
-#pragma unroll
-    for (int p = 0; p < SORT_PASSES; ++p)
-      atomicAdd(&s_hist[p * 256 + ((code >> (8 * p)) & 255u)], 1u);
   }
   __syncthreads();
   for (int i = threadIdx.x; i < SORT_PASSES * 256; i += BLOCK) {

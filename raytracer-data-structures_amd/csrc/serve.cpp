@@ -450,7 +450,6 @@ bool launch_step(rq_server* s) {
   BatchWork* it = s->host_items[buf];
   uint32_t ni = 0;
   for (int qd = 0; qd < BATCH_XCDS; ++qd) {
-    a.trace_seg[qd] = ni;
     for (uint32_t i = 0; i < ne; ++i) {
       if (seg[i] != (uint32_t)qd) continue;
       const uint32_t nt = (md[i].nrays + tile - 1) / tile;
@@ -460,7 +459,9 @@ bool launch_step(rq_server* s) {
         for (uint32_t t = 0; t < nt; ++t) it[ni++] = BatchWork{i, t | BATCH_ANY_BIT};
     }
   }
-  a.trace_seg[BATCH_XCDS] = ni;
+  // equal parts: a step of few requests is on every XCD all the same
+  for (int qd = 0; qd <= BATCH_XCDS; ++qd)
+    a.trace_seg[qd] = (uint32_t)((uint64_t)ni * qd / BATCH_XCDS);
   a.meshes = s->dev_meshes[buf];
   a.items = s->dev_items[buf];
   a.ctl = s->ctl;
@@ -474,7 +475,8 @@ bool launch_step(rq_server* s) {
     e = hipMemcpyAsync(s->dev_items[buf], it, ni * sizeof(BatchWork), hipMemcpyHostToDevice,
                        s->s_trace);
   if (e == hipSuccess) e = hipEventRecord(st->start, s->s_trace);
-  if (e == hipSuccess) e = launch_serve_trace(LaunchCtx{s->s_trace, nullptr}, a, s->variant, s->grid);
+  const uint32_t grid = std::min(s->grid, std::max(1u, tiles_of(ni, BATCH_XCDS)) * BATCH_XCDS);
+  if (e == hipSuccess) e = launch_serve_trace(LaunchCtx{s->s_trace, nullptr}, a, s->variant, grid);
   if (e == hipSuccess)
     e = hipMemcpyAsync(s->err_host[buf], s->ctl + BATCH_CTL_BARRIER_ERR, 2 * sizeof(uint32_t),
                        hipMemcpyDeviceToHost, s->s_trace);
