@@ -1,24 +1,19 @@
 /*
- * rq — batched build and traversal of many meshes in one persistent launch.
+ * rq — batched build and traversal of many meshes in one run.
  *
  * The reference builds and renders one scene per process run (main.cpp:723-853).
  * Here a batch holds many uploaded meshes of uneven sizes together with one
  * device ray batch per mesh. rq_batch_run builds every mesh's LBVH (Morton,
- * radix sort, Karras, refit) and traces every ray batch in ONE persistent
- * kernel: its blocks pull work items (mesh, phase, tile) from a device work
- * queue, phase by phase across all meshes, with grid-wide barriers between
- * phases. rq_batch_run_graph captures the launch (and its counter reset) in a
+ * radix sort, Karras, refit) and traces every ray batch from one device work
+ * queue that holds the items (mesh, tile) of all meshes, phase by phase.
+ * rq_batch_run_graph captures the run (and its counter reset) in a
  * hipGraph once and replays it. The results of every mesh are identical to
  * rq_build_lbvh + rq_closest_hit / rq_any_hit on that mesh alone.
  *
- * Co-residency: the grid is sized from the kernel's occupancy (blocks per CU
- * x CUs), but the phase barriers never assume that every block is placed:
- * they count only the blocks that have started. The first barrier waits
- * briefly for the rest of the grid, then closes the membership; blocks the
- * device places later (behind kernels of other streams that held CUs) leave
- * without work. Work items come from queues, so the members complete every
- * phase: a contended run is slower, never wrong. rq_batch_occupancy reports
- * how many blocks took part in the last run.
+ * A run is one enqueue: a launch per build phase (a block or more per work
+ * item, whatever mesh it belongs to), then one of the persistent trace kernel,
+ * which pulls its items from a queue. No block waits for one that may not have
+ * started, so a run beside other streams' kernels is slower, never wrong.
  */
 #ifndef RQ_BATCH_H
 #define RQ_BATCH_H
@@ -69,8 +64,9 @@ int rq_batch_set_config(rq_ctx* ctx, rq_batch* b, int index, uint32_t ray_tile,
                         uint32_t refill_idle);
 int rq_batch_get_config(rq_ctx* ctx, const rq_batch* b, int* index, uint32_t* ray_tile,
                         uint32_t* refill_idle);
-/* The build kernel's waves per SIMD (8, 7, 6, 5 or 4: its register cap, traded
- * against occupancy); the autotuner chooses it after the trace configuration. */
+/* The waves per SIMD of the build's sort kernels (8, 7, 6, 5 or 4: their
+ * register cap, traded against occupancy); the autotuner chooses it after the
+ * trace configuration. */
 int rq_batch_set_build_waves(rq_ctx* ctx, rq_batch* b, int waves);
 int rq_batch_get_build_waves(rq_ctx* ctx, const rq_batch* b, int* waves);
 /* Times the trace configurations, ray-tile sizes and refill thresholds on the
@@ -81,18 +77,16 @@ int rq_batch_autotune(rq_ctx* ctx, rq_batch* b, int repeats, int* best_index,
 /* Items of the work queue per phase (11 phases), for inspection. */
 int rq_batch_phase_items(rq_ctx* ctx, rq_batch* b, uint32_t* counts, int cap);
 /* Synchronises and reports the last run's build phases in ms (the first
- * `cap` of the 10 build phases, init ... widen), from wall-clock stamps the
- * build kernel takes at its grid barriers; returns the number of build
- * phases. A phase the run did not stamp reads -1. */
+ * `cap` of the 11 build phases, init ... widen), from wall-clock stamps the
+ * phases take at their starts; returns the number of build phases. Without a
+ * run they read -1. */
 int rq_batch_phase_ms(rq_ctx* ctx, rq_batch* b, double* ms, int cap);
-/* Synchronises and reports the error bits of the last run: 1 = a grid
- * barrier gave up waiting (a member block did not arrive within seconds; the
- * results of that run are invalid), 2 = a ray needed a deeper stack than
- * provided, 4 = a mesh build reported an error. */
+/* Synchronises and reports the error bits of the last run: 2 = a ray needed a
+ * deeper stack than provided, 4 = a mesh build reported an error. */
 int rq_batch_errors(rq_ctx* ctx, rq_batch* b, uint32_t* bits);
-/* Synchronises and reports the blocks that took part in the last run
- * (members) and the launch grid: members < grid when part of the grid could
- * not be placed before the first barrier (the device was busy). */
+/* Synchronises and reports the blocks of the build's sort kernels that the
+ * device holds at a time (grid), and as members the same once the batch has
+ * run: every run takes its whole grid, however busy the device. */
 int rq_batch_occupancy(rq_ctx* ctx, rq_batch* b, uint32_t* members, uint32_t* grid);
 
 #ifdef __cplusplus

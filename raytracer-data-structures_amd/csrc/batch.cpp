@@ -1,6 +1,6 @@
 // Host side of the batched build + traversal (include/rq/rq_batch.h): per-mesh
 // BVH buffers, the device work queue (items of every mesh, phase by phase),
-// the persistent launch, its hipGraph capture and the batch autotuner.
+// the launches, their hipGraph capture and the batch autotuner.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,8 +29,9 @@ struct rq_batch {
   uint32_t* ctl = nullptr;
   int32_t* gstack = nullptr;
   uint32_t gdepth = 0;
-  int build = 3;                       // build kernel: 5 waves per SIMD (batch_build_waves)
-  std::vector<uint32_t> build_grid;    // its persistent grid, per build kernel
+  int build = 3;                       // sort kernels: 5 waves per SIMD (batch_build_waves)
+  std::vector<uint32_t> build_grid;    // their blocks on the device at a time
+  bool ran = false;
   std::vector<uint32_t> grid;          // the trace kernel's, per configuration
   // the autotuned choice on 512 mixed meshes (1k-500k triangles, incoherent
   // rays): trace configuration 1 (LDS depth 16), 512-ray items, refill at 16
@@ -180,7 +181,8 @@ int launch(rq_ctx* c, rq_batch* b, hipStream_t s, bool profile) {
   const uint32_t items = b->trace_seg[BATCH_XCDS] - b->trace_seg[0];
   const uint32_t grid = std::min(b->grid[b->variant],
                                  std::max(1u, tiles_of(items, BATCH_XCDS * BUILD_BLOCK / 64)) * BATCH_XCDS);
-  hipError_t e = launch_batch(lc, batch_args(b), b->build, b->build_grid[b->build], b->variant, grid);
+  hipError_t e = launch_batch(lc, batch_args(b), b->build, b->variant, grid);
+  b->ran = b->ran || e == hipSuccess;
   return e == hipSuccess ? RQ_OK : hip_err(c, e, "batch launch");
 }
 
@@ -430,8 +432,15 @@ int rq_batch_phase_ms(rq_ctx* c, rq_batch* b, double* ms, int cap) {
   if (khz <= 0) return set_err(c, RQ_E_HIP, "no wall-clock rate");
   uint64_t st[BATCH_PHASES];
   std::memcpy(st, w + BATCH_CTL_CLOCK, sizeof st);
+  // a phase without items has no stamp and takes no time
+  uint64_t end = 0;
+  for (uint64_t s : st) end = std::max(end, s);
+  for (int ph = (int)PH_TRACE; ph >= 0; --ph) {
+    if (!st[ph]) st[ph] = end;
+    end = st[ph];
+  }
   for (int ph = 0; ph < (int)PH_TRACE && ph < cap; ++ph)
-    ms[ph] = st[ph + 1] >= st[ph] && st[0] != ~0ull ? (double)(st[ph + 1] - st[ph]) / khz : -1.0;
+    ms[ph] = st[ph + 1] >= st[ph] && st[ph] ? (double)(st[ph + 1] - st[ph]) / khz : -1.0;
   return (int)PH_TRACE;
 }
 
@@ -441,7 +450,7 @@ int rq_batch_errors(rq_ctx* c, rq_batch* b, uint32_t* bits) {
   hipError_t e = hipDeviceSynchronize();
   if (e == hipSuccess) e = hipMemcpy(w, b->ctl, sizeof w, hipMemcpyDeviceToHost);
   if (e != hipSuccess) return hip_err(c, e, "batch errors");
-  *bits = (w[BATCH_CTL_BARRIER_ERR] ? 1u : 0u) | (w[BATCH_CTL_TRACE_ERR] ? 2u : 0u);
+  *bits = w[BATCH_CTL_TRACE_ERR] ? 2u : 0u;
   for (rq_bvh* v : b->bvhs) {
     if (!v->n) continue;
     uint32_t m = 0;
@@ -477,13 +486,10 @@ int rq_batch_get_build_waves(rq_ctx* c, const rq_batch* b, int* waves) {
 
 int rq_batch_occupancy(rq_ctx* c, rq_batch* b, uint32_t* members, uint32_t* grid) {
   if (!c || !b || !members || !grid) return RQ_E_INVALID;
-  uint32_t m = 0;
-  hipError_t e = hipDeviceSynchronize();
-  if (e == hipSuccess)
-    e = hipMemcpy(&m, b->ctl + BATCH_CTL_MEMBERS, sizeof m, hipMemcpyDeviceToHost);
+  const hipError_t e = hipDeviceSynchronize();
   if (e != hipSuccess) return hip_err(c, e, "batch occupancy");
-  *members = m;
   *grid = b->build_grid[b->build];
+  *members = b->ran ? *grid : 0u;  // no launch depends on which blocks are placed
   return RQ_OK;
 }
 

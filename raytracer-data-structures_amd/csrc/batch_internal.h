@@ -1,4 +1,4 @@
-// Internal types of the persistent batch kernel (batch_kernels.hip <-> batch.cpp).
+// Internal types of the batch kernels (batch_kernels.hip <-> batch.cpp).
 #pragma once
 #include "build_device.h"
 
@@ -27,29 +27,17 @@ enum BatchPhase {
 constexpr int BATCH_XCDS = 8;
 
 // control words of one batch
-constexpr int BATCH_CTL_TICKET = 0;                        // BATCH_PHASES queue tickets
-constexpr int BATCH_CTL_BARRIER = BATCH_PHASES;            // grid barrier arrivals
-constexpr int BATCH_CTL_BARRIER_ERR = BATCH_PHASES + 1;    // barrier wait gave up (this run)
-constexpr int BATCH_CTL_TRACE_ERR = BATCH_PHASES + 2;      // stack deeper than provided (this run)
-constexpr int BATCH_CTL_START = BATCH_PHASES + 3;          // blocks started (+ BATCH_CLOSED)
-constexpr int BATCH_CTL_MEMBERS = BATCH_CTL_START + 1;     // blocks taking part (0 until closed)
-// BATCH_PHASES 64-bit wall-clock stamps (8-byte aligned) of the build kernel:
-// stamp 0 = the first member's start, stamp p = phase p - 1 done (its last
-// member's arrival)
-constexpr int BATCH_CTL_CLOCK = (BATCH_CTL_MEMBERS + 2) & ~1;
+constexpr int BATCH_CTL_TRACE_ERR = 0;  // stack deeper than provided (this run)
+// BATCH_PHASES 64-bit wall-clock stamps (8-byte aligned) of a run: stamp p =
+// the start of phase p, or the build's end (0 where the phase has no items)
+constexpr int BATCH_CTL_CLOCK = 2;
 constexpr int BATCH_CTL_WORDS = BATCH_CTL_CLOCK + 2 * BATCH_PHASES;
-// The grid barrier's group words, after the control words: BATCH_BAR_GROUPS
-// arrival counters, then as many release words, each word on a 4 KB page of
-// its own, so that the arrivals and polls of different groups are served by
-// different memory channels rather than queueing on one word (12 ns an atomic).
-// The tickets of the trace segments follow, spread the same way.
-constexpr int BATCH_BAR_GROUPS = 16;
-constexpr int BATCH_BAR_STRIDE = 1024;  // words
-constexpr int BATCH_BAR_BASE = BATCH_BAR_STRIDE;
-constexpr int BATCH_XTICKET_BASE = BATCH_BAR_BASE + 2 * BATCH_BAR_GROUPS * BATCH_BAR_STRIDE;
-constexpr int BATCH_CTL_ALLOC_WORDS = BATCH_XTICKET_BASE + BATCH_XCDS * BATCH_BAR_STRIDE;
-static_assert(BATCH_CTL_WORDS <= BATCH_BAR_BASE, "control words before the barrier groups");
-constexpr uint32_t BATCH_CLOSED = 0x80000000u;             // start word: membership closed
+// The tickets of the trace segments, after the control words, each on a 4 KB
+// page of its own: atomics on one line queue (12 ns each).
+constexpr int BATCH_XTICKET_STRIDE = 1024;  // words
+constexpr int BATCH_XTICKET_BASE = BATCH_XTICKET_STRIDE;
+constexpr int BATCH_CTL_ALLOC_WORDS = BATCH_XTICKET_BASE + BATCH_XCDS * BATCH_XTICKET_STRIDE;
+static_assert(BATCH_CTL_WORDS <= BATCH_XTICKET_BASE, "control words before the tickets");
 constexpr uint32_t BATCH_ANY_BIT = 0x80000000u;            // trace item tile: any-hit query
 // Work items of the refit phases (see batch_kernels.hip): refit chunks of
 // BUILD_BLOCK leaves, BATCH_REFIT_CHUNKS per item; spanning nodes in tiles of
@@ -86,7 +74,7 @@ struct BatchArgs {
 // Batch configurations: the trace kernels of a batch run (4-wide walk).
 int batch_num_variants();
 void batch_variant_info(int v, int* depth, int* tstack);
-// Build kernels by waves per SIMD (8, 7, 6, 5).
+// The build's sort kernels by waves per SIMD (8, 7, 6, 5, 4).
 int batch_num_build_variants();
 int batch_build_waves(int build);
 uint32_t batch_build_grid_blocks(int device, int build);
@@ -95,10 +83,10 @@ uint32_t batch_trace_grid_blocks(int device, int v);
 int serve_num_variants();
 void serve_variant_info(int v, int* depth, int* tstack, int* wide);
 uint32_t serve_grid_blocks(int device, int v);
-// A batch run: resets the control words, then the build kernel (every build
-// phase, grid barriers between them) and the trace kernel of `variant`.
-hipError_t launch_batch(const LaunchCtx& lc, const BatchArgs& a, int build, uint32_t build_grid,
-                        int variant, uint32_t trace_grid);
+// A batch run: resets the control words, then the build phases, a launch each
+// (sort kernels `build`), and the trace kernel of `variant`.
+hipError_t launch_batch(const LaunchCtx& lc, const BatchArgs& a, int build, int variant,
+                        uint32_t trace_grid);
 // The serving step: resets the control words, then the trace phase alone.
 hipError_t launch_serve_trace(const LaunchCtx& lc, const BatchArgs& a, int variant, uint32_t grid);
 

@@ -1,12 +1,16 @@
-// Persistent batch kernel: builds the LBVH of many meshes and traces their
-// ray batches in one launch. Blocks pull work items (mesh, tile) from a device
-// work queue, one queue segment per phase (init, bounds, Morton, four sort
-// passes, Karras, refit, refit top, trace) holding the items of every mesh;
-// a grid-wide barrier separates phases, so a mesh's phase k + 1 reads what
-// any block wrote in phase k. Within a phase the queue balances uneven meshes:
-// a block takes the next item as soon as it finishes one. Items of a sort pass
-// are queued mesh by mesh in tile order, so a tile's look-back only waits on
-// tiles already taken by running blocks.
+// Batch kernels: build the LBVH of many meshes and trace their ray batches.
+// One device work queue holds the items (mesh, tile) of every mesh, phase after
+// phase (init, bounds, Morton, four sort passes, Karras, refit, spanning nodes,
+// widen, trace); a phase of the build is one launch with a block or more per
+// item, whatever mesh it belongs to, and the trace phase one launch of
+// persistent waves that pull its items.
+//
+// One persistent kernel used to run all the build phases with grid barriers
+// between them. A barrier cost 33 ns a block (each block's write-back and
+// invalidation of its L2, one after another on an XCD): 42 us at 1280 blocks,
+// ten times a build, and the kernel's registers and LDS were the largest
+// phase's. Between launches the device does that once: the build of 48 meshes
+// of 64 triangles 490 -> 59 us, of 30 k triangles 1160 -> 390.
 #include <algorithm>
 
 #include "batch_internal.h"
@@ -16,120 +20,9 @@
 namespace rq {
 namespace {
 
-// About 4M polls (a few seconds): far beyond any phase of the member blocks.
-constexpr uint32_t BARRIER_SPIN_LIMIT = 1u << 22;
-// Polls the first barrier waits for the rest of the grid to start before it
-// closes the membership with the blocks that have.
-constexpr uint32_t JOIN_SPIN_LIMIT = 1u << 14;
-
-// Membership: the barriers count only the blocks that have started, so that
-// they never wait for a block the device has not placed (kernels on other
-// streams can hold CUs when the launch begins). A block joins by taking a
-// ticket from the start word at entry; a block that finds the membership
-// closed leaves at once. The first block to reach the first barrier waits
-// (bounded) until the whole grid has started, then closes the membership
-// with an atomic OR, whose returned count is the number of members: the
-// members hold tickets 0 .. members - 1. Work is pulled from queues, so any
-// number of members completes every phase: a grid that could not be placed
-// whole runs on fewer blocks, not wrongly. Returns the block's ticket, or
-// ~0u for a block that takes no part.
-__device__ inline uint32_t join_grid(uint32_t* ctl, uint32_t* s_flag) {
-  if (threadIdx.x == 0) *s_flag = atomicAdd(ctl + BATCH_CTL_START, 1u);
-  __syncthreads();
-  const uint32_t t = *s_flag;
-  __syncthreads();
-  return (t & BATCH_CLOSED) ? ~0u : t;
-}
-
-__device__ inline uint32_t* bar_group(uint32_t* ctl, uint32_t g) {
-  return ctl + BATCH_BAR_BASE + (size_t)g * BATCH_BAR_STRIDE;
-}
-__device__ inline uint32_t* bar_release(uint32_t* ctl, uint32_t g) {
-  return ctl + BATCH_BAR_BASE + (size_t)(BATCH_BAR_GROUPS + g) * BATCH_BAR_STRIDE;
-}
-
-// Phase stamps (BATCH_CTL_CLOCK): the latest (or, for the start, earliest)
-// wall-clock reading over the member blocks, one atomic per block.
+// Phase stamps (BATCH_CTL_CLOCK).
 __device__ inline unsigned long long* clock_stamp(uint32_t* ctl, uint32_t k) {
   return reinterpret_cast<unsigned long long*>(ctl + BATCH_CTL_CLOCK) + k;
-}
-
-// Counts the block's arrival at the end of phase `phases_done` - 1 on its
-// group's counter (group = ticket mod BATCH_BAR_GROUPS), the group's last
-// arrival on the top counter; true for the grid's last, which stamps the phase.
-// The counters are cumulative over the launch, so the last arrival of phase p
-// is the one that brings a counter to p times its members.
-__device__ inline bool arrived_last(uint32_t* ctl, uint32_t phases_done, uint32_t members,
-                                    uint32_t g, uint32_t old) {
-  constexpr uint32_t G = BATCH_BAR_GROUPS;
-  const uint32_t groups = min(members, G), in_group = (members - g + G - 1u) / G;
-  if (old + 1u != in_group * phases_done) return false;
-  __threadfence();
-  if (atomicAdd(ctl + BATCH_CTL_BARRIER, 1u) + 1u != groups * phases_done) return false;
-  *clock_stamp(ctl, phases_done) = (unsigned long long)wall_clock64();
-  return true;
-}
-
-// Grid barrier after phase `phases_done` - 1. The block's waves meet at a
-// work-group barrier, which leaves their stores in the XCD's L2; thread 0's
-// agent-scope release then writes that L2 back (one write-back per block
-// rather than one per wave), and it counts the block's arrival. The grid's
-// last arrival publishes the phase on every group's release word; each block
-// waits on its own group's word and acquires. One word shared by every block,
-// for the arrivals and for the polls, had made each barrier cost ~0.15-0.3 ms
-// on a full grid; a time stamp of every block on one word still cost it 25 us.
-// The members are running, so every wait ends; it is bounded all the same: a
-// wait that gives up sets the sticky error word, and once it is set no later
-// barrier of the launch waits at all. Returns the number of members (0 if the
-// wait for it gave up).
-__device__ inline uint32_t grid_barrier(uint32_t* ctl, uint32_t phases_done, uint32_t ticket,
-                                        uint32_t* s_flag) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();
-    uint32_t* const err = ctl + BATCH_CTL_BARRIER_ERR;
-    const uint32_t g = ticket % (uint32_t)BATCH_BAR_GROUPS;
-    const uint32_t old = atomicAdd(bar_group(ctl, g), 1u);
-    uint32_t members = ld_agent(ctl + BATCH_CTL_MEMBERS);
-    if (members == 0u) {  // the first barrier of the launch: close the membership
-      uint32_t spins = 0;
-      for (;;) {
-        const uint32_t st = ld_agent(ctl + BATCH_CTL_START);
-        if ((st & BATCH_CLOSED) || st >= gridDim.x || ++spins > JOIN_SPIN_LIMIT) break;
-        __builtin_amdgcn_s_sleep(2);
-      }
-      const uint32_t o = atomicOr(ctl + BATCH_CTL_START, BATCH_CLOSED);
-      if (!(o & BATCH_CLOSED)) atomicExch(ctl + BATCH_CTL_MEMBERS, o);
-      spins = 0;
-      while ((members = ld_agent(ctl + BATCH_CTL_MEMBERS)) == 0u) {
-        if (++spins > BARRIER_SPIN_LIMIT) {
-          atomicOr(err, 1u);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-      }
-    }
-    if (members != 0u) {
-      if (arrived_last(ctl, phases_done, members, g, old)) {
-        __threadfence();  // the grid's last arrival: release every group
-        for (uint32_t k = 0; k < BATCH_BAR_GROUPS; ++k) atomicMax(bar_release(ctl, k), phases_done);
-      }
-      uint32_t spins = 0;
-      while (ld_agent(bar_release(ctl, g)) < phases_done) {
-        if (++spins > BARRIER_SPIN_LIMIT || ((spins & 1023u) == 0u && ld_agent(err) != 0u)) {
-          atomicOr(err, 1u);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-      }
-    }
-    __threadfence();
-    *s_flag = members;
-  }
-  __syncthreads();
-  const uint32_t members = *s_flag;
-  __syncthreads();
-  return members;
 }
 
 // The next item of a queue of n items whose first `owned` are taken without a
@@ -218,7 +111,7 @@ struct SegQueue {
         own = false;
         if (index < n) return b0 + index;
       }
-      const uint32_t it = next_item(a.ctl + BATCH_XTICKET_BASE + q * BATCH_BAR_STRIDE,
+      const uint32_t it = next_item(a.ctl + BATCH_XTICKET_BASE + q * BATCH_XTICKET_STRIDE,
                                     seg_blocks(q, BATCH_XCDS, gridDim.x) * PER_BLOCK, n);
       if (it < n) return b0 + it;
     }
@@ -298,208 +191,138 @@ __device__ inline void trace_mesh(const BatchArgs& a, const BatchMeshDev& m, uin
   }
 }
 
-// The batch build's refit chunks: one leaf per thread of a block. The queue's
-// items are larger than that (BATCH_REFIT_CHUNKS chunks, BATCH_SPAN_TILES
-// tiles of BUILD_BLOCK internal nodes, ...); the blocks share each item of
-// phase ph in phase_parts(ph) parts, so that the last round of a phase is a
-// small part of it: 1.5 M triangles in 48 meshes are 385 to 1476 items, for
-// 1280 blocks.
-constexpr int BATCH_REFIT_CHUNK = BUILD_BLOCK;
-constexpr uint32_t BOUNDS_PARTS = 4, KARRAS_PARTS = 8, SPAN_PARTS = 4;
-__device__ inline uint32_t phase_parts(int ph) {
-  return ph == PH_BOUNDS  ? BOUNDS_PARTS
-         : ph == PH_KARRAS ? KARRAS_PARTS
-         : ph == PH_REFIT  ? BATCH_REFIT_CHUNKS
-         : ph == PH_TOP || ph == PH_WIDEN ? SPAN_PARTS
-                                          : 1u;
+// ---- the build phases: a launch each ----------------------------------------
+// Block of phase ph: part (block mod parts) of item (block / parts).
+// Descriptors are loaded into scalar registers.
+template <uint32_t PARTS>
+struct PhaseUnit {
+  BuildView v;
+  uint32_t tile;  // the part's number in its mesh
+  __device__ PhaseUnit(const BatchArgs& a, int ph) {
+    // the phase's start, the end of the one before
+    if (blockIdx.x == 0 && threadIdx.x == 0) *clock_stamp(a.ctl, ph) = wall_clock64();
+    const BatchWork w = load_uniform(a.items + a.phase_begin[ph] + blockIdx.x / PARTS);
+    v = load_uniform(&a.meshes[w.mesh].v);
+    tile = w.tile * PARTS + blockIdx.x % PARTS;
+  }
+};
+// The end of what may be the last phase with items (near enough: its last
+// block's).
+__device__ inline void stamp_end(const BatchArgs& a, int ph) {
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *clock_stamp(a.ctl, ph + 1) = wall_clock64();
 }
 
+// Clears the control words before a run; block 0 of the init phase, so that the
+// reset lives in the same captured graph as the run.
+__device__ inline void reset_ctl(uint32_t* ctl) {
+  static_assert(BATCH_CTL_WORDS <= 64, "one wave clears the control words");
+  if (threadIdx.x < BATCH_CTL_WORDS) ctl[threadIdx.x] = 0u;
+  if (threadIdx.x < BATCH_XCDS) ctl[BATCH_XTICKET_BASE + threadIdx.x * BATCH_XTICKET_STRIDE] = 0u;
+}
+__global__ void k_batch_reset(uint32_t* ctl) { reset_ctl(ctl); }
 
-// LDS words of the batch kernel: the build kernel's largest phase (lean sort
-// tile, Morton histograms, refit chunk), the trace kernel's stack.
-constexpr int cmax(int x, int y) { return x > y ? x : y; }
-constexpr int batch_lds_words(bool build, int depth, bool tstack) {
-  return build ? cmax(cmax(cmax(sort_lds_words(SORT_ITEMS_LEAN), SORT_PASSES * 256),
-                           refit_chunk_lds_words<BATCH_REFIT_CHUNK>()),
-                      karras_lds_words<NODE_TILE / KARRAS_PARTS>())
-               : depth * BUILD_BLOCK * (tstack ? 2 : 1);
+// (launched with a block at least, for the reset)
+__global__ __launch_bounds__(BUILD_BLOCK) void k_batch_init(BatchArgs a) {
+  if (blockIdx.x == 0) {
+    reset_ctl(a.ctl);
+    __syncthreads();
+  }
+  if (a.phase_begin[PH_INIT] + blockIdx.x >= a.phase_begin[PH_INIT + 1]) return;
+  const PhaseUnit<1> u(a, PH_INIT);
+  build_init_misc(u.v, threadIdx.x, BUILD_BLOCK);
+}
+constexpr int TRI_BLOCK = 1024;
+__global__ __launch_bounds__(TRI_BLOCK) void k_batch_bounds(BatchArgs a) {
+  __shared__ uint32_t lds[6 * (TRI_BLOCK / 64)];
+  const PhaseUnit<1> u(a, PH_BOUNDS);
+  bounds_tile<TRI_BLOCK>(u.v, u.tile, lds);
+}
+// Also clears the sort's look-back words, a part a tile (in the init phase's
+// one item a mesh they took 0.1 ms of one block).
+__global__ __launch_bounds__(TRI_BLOCK) void k_batch_morton(BatchArgs a) {
+  __shared__ uint32_t lds[SORT_PASSES * 256];
+  const PhaseUnit<1> u(a, PH_MORTON);
+  build_init_status(u.v, u.tile * TRI_BLOCK + threadIdx.x, tiles_of(u.v.n, TRI_TILE) * TRI_BLOCK);
+  morton_tile<TRI_BLOCK>(u.v, u.tile, lds);
+}
+// The tile comes from the mesh's ticket of the pass, so a tile's look-back only
+// waits on tiles whose blocks are already running (a mesh has a block for each
+// of its tiles).
+template <int PASS, int WAVES>
+__global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void
+k_batch_sort(BatchArgs a) {
+  __shared__ uint32_t lds[sort_lds_words(SORT_ITEMS_LEAN)];
+  __shared__ uint32_t s_tile;
+  const PhaseUnit<1> u(a, PH_SORT0 + PASS);
+  if (threadIdx.x == 0) s_tile = atomicAdd(&u.v.B.misc[MISC_TILECTR + PASS], 1u);
+  __syncthreads();
+  onesweep_tile<PASS, SORT_ITEMS_LEAN>(u.v, s_tile, lds);
+}
+constexpr uint32_t KARRAS_PARTS = NODE_TILE / BUILD_BLOCK;  // a node a thread
+__global__ __launch_bounds__(BUILD_BLOCK) void k_batch_karras(BatchArgs a) {
+  __shared__ uint32_t lds[karras_lds_words<BUILD_BLOCK>()];
+  const PhaseUnit<KARRAS_PARTS> u(a, PH_KARRAS);
+  karras_tile<BUILD_BLOCK>(u.v, u.tile, lds);
+}
+// Chunk-union refit, pass 1 (with the chunks' wide records), a block an item.
+constexpr int BATCH_REFIT_CHUNK = BUILD_BLOCK * BATCH_REFIT_CHUNKS;
+__global__ __launch_bounds__(BATCH_REFIT_CHUNK) void k_batch_refit(BatchArgs a) {
+  __shared__ uint32_t lds[refit_chunk_lds_words<BATCH_REFIT_CHUNK>()];
+  const PhaseUnit<1> u(a, PH_REFIT);
+  refit_chunk_tile<BATCH_REFIT_CHUNK>(u.v, u.tile, lds);
+  stamp_end(a, PH_REFIT);
+}
+// Pass 2: the nodes spanning chunks, a wave per 64 nodes; then their wide
+// records.
+__global__ __launch_bounds__(BUILD_BLOCK) void k_batch_span(BatchArgs a) {
+  const PhaseUnit<BATCH_SPAN_TILES> u(a, PH_TOP);
+  refit_span_wave<BATCH_REFIT_CHUNK>(u.v.B, u.v.n, u.tile * BUILD_BLOCK + threadIdx.x);
+}
+__global__ __launch_bounds__(BUILD_BLOCK) void k_batch_widen(BatchArgs a) {
+  const PhaseUnit<BATCH_SPAN_TILES> u(a, PH_WIDEN);
+  const uint32_t i = u.tile * BUILD_BLOCK + threadIdx.x;
+  if (i + 1u < u.v.n && spans_chunks<BATCH_REFIT_CHUNK>(u.v.B, i)) widen_global(u.v.B, i);
+  stamp_end(a, PH_WIDEN);
 }
 
-// Two kernels share this body. KM_BUILD runs the build phases of every mesh
-// (init ... widen) with grid barriers between them; KM_TRACE runs the trace
-// phase alone (ray tiles over built BVHs, no barrier): after KM_BUILD in a
-// batch run (WIDE: walking the 4-wide nodes of the widen phase), or as the
-// continuous-batching step of the serving loop (binary nodes). WAVES waves
-// per SIMD cap the registers: the build phases are written to fit 8 (lean
-// 8-key sort tiles, descriptors loaded per phase); the 4-wide walk fits 8
-// (63 VGPRs) where its LDS stack allows, the binary walk 7-8.
-enum KernelMode { KM_BUILD, KM_TRACE };
-template <int DEPTH, bool TSTACK, int WAVES, KernelMode MODE, bool WIDE, bool WAVE_ITEMS = WIDE>
-__global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_batch(
-    BatchArgs a) {
-  __shared__ uint32_t lds[batch_lds_words(MODE == KM_BUILD, DEPTH, TSTACK)];
+// The trace phase (ray tiles over built BVHs): after the build in a batch run
+// (WIDE: walking the 4-wide nodes of the widen phase), or as the
+// continuous-batching step of the serving loop (its binary or wide nodes).
+// WAVES waves per SIMD cap the registers: the 4-wide walk fits 8 (64 VGPRs)
+// where its LDS stack allows, the binary walk 7-8. WAVE_ITEMS (the batch run):
+// waves take items on their own and never wait for the rest of their block;
+// otherwise (the serving step, whose tiles are sized for a block) a block
+// takes an item and its waves share it.
+template <int DEPTH, bool TSTACK, int WAVES, bool WIDE, bool WAVE_ITEMS = WIDE>
+__global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void
+k_batch_trace(BatchArgs a) {
+  __shared__ uint32_t lds[DEPTH * BUILD_BLOCK * (TSTACK ? 2 : 1)];
   __shared__ uint32_t s_item, s_ctr;
-  uint32_t* const ctl = a.ctl;
-  const BatchWork* const items = a.items;
-  const BatchMeshDev* const meshes = a.meshes;
-  if constexpr (MODE == KM_TRACE) {
-    // WAVE_ITEMS (the batch run): waves take items on their own and never wait
-    // for the rest of their block; otherwise (the serving step, whose tiles are
-    // sized for a block) a block takes an item and its waves share it.
-    if constexpr (WAVE_ITEMS) {
-      ItemSlices src{a, SegItems(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), 0u, 0u, 0u,
-                     BatchWork{}, false, false};
-      if (!src.take(src.held)) return;
-      for (;;) {
-        const BatchMeshDev m = load_uniform(meshes + src.held.mesh);
-        src.mesh = src.held.mesh, src.kind = src.held.tile & BATCH_ANY_BIT, src.nrays = m.nrays;
-        src.first = true, src.have_held = false;
-        trace_mesh<DEPTH, TSTACK, WIDE>(a, m, lds, &src);
-        if (!src.have_held) return;
-      }
-    } else {
-      SegQueue<1> queue(0u);
-      for (;;) {
-        if (threadIdx.x == 0) s_item = queue.take(a);
-        __syncthreads();
-        const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
-        __syncthreads();
-        if (it == NO_ITEM) return;
-        const BatchWork w = load_uniform(items + it);
-        const BatchMeshDev m = load_uniform(meshes + w.mesh);
-        trace_item<DEPTH, TSTACK, WIDE>(a.gstack, a.gdepth, ctl + BATCH_CTL_TRACE_ERR, a.ray_tile,
-                                        a.refill_idle, m, w.tile, lds, &s_ctr);
-      }
-    }
-    return;
-  }
-  // ---- the build phases, block by block, grid barriers between them
-  // blocks the device places after the membership closed take no part
-  const uint32_t ticket = join_grid(ctl, &s_item);
-  if (ticket == ~0u) return;
-  if (ticket == 0u && threadIdx.x == 0)
-    *clock_stamp(ctl, 0) = (unsigned long long)wall_clock64();
-  // The blocks take a phase's parts in turn: part k is block (k mod members)'s,
-  // without a ticket. (A sort tile waits on the tiles before it: every block
-  // takes its own in ascending order.) The blocks of the first phase are not
-  // counted yet: its items go by ticket.
-  uint32_t members = 0;
-  constexpr int last = (int)PH_TRACE;
-  for (int ph = 0; ph < last; ++ph) {
-   {
-    // kernarg words, block-uniform
-    const uint32_t b0 = a.phase_begin[ph], parts = phase_parts(ph);
-    const uint32_t units = (a.phase_begin[ph + 1] - b0) * parts;
-    uint32_t unit = ticket - members;
+  if constexpr (WAVE_ITEMS) {
+    ItemSlices src{a, SegItems(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), 0u, 0u, 0u,
+                   BatchWork{}, false, false};
+    if (!src.take(src.held)) return;
     for (;;) {
-      if (members != 0u) {
-        unit += members;
-      } else {
-        if (threadIdx.x == 0) s_item = next_item(ctl + BATCH_CTL_TICKET + ph, 0u, units);
-        __syncthreads();
-        unit = s_item;
-        __syncthreads();
-      }
-      // block-uniform: keep the item and its mesh descriptor in scalar registers
-      unit = __builtin_amdgcn_readfirstlane(unit);
-      if (unit >= units) break;
-      const uint32_t part = unit % parts;
-      const BatchWork w = load_uniform(items + b0 + unit / parts);
-      const BatchMeshDev* const mp = meshes + w.mesh;
-      // each phase loads the descriptor itself: fields it does not read are
-      // never loaded and hold no scalar registers
-#define VIEW const BuildView v = load_uniform(&mp->v)
-      switch (ph) {
-        case PH_INIT: {
-          VIEW;
-          build_init_misc(v, threadIdx.x, BUILD_BLOCK);
-          break;
-        }
-        case PH_BOUNDS: {
-          VIEW;
-          bounds_tile<BUILD_BLOCK, TRI_TILE / BOUNDS_PARTS>(v, w.tile * BOUNDS_PARTS + part, lds);
-          break;
-        }
-        case PH_MORTON: {
-          VIEW;
-          // the sort's look-back words, a part a tile (in the init phase's one
-          // item a mesh they took 0.1 ms of one block)
-          build_init_status(v, w.tile * BUILD_BLOCK + threadIdx.x,
-                            tiles_of(v.n, TRI_TILE) * BUILD_BLOCK);
-          morton_tile(v, w.tile, lds);
-          break;
-        }
-        case PH_SORT0: {
-          VIEW;
-          onesweep_tile<0, SORT_ITEMS_LEAN>(v, w.tile, lds);
-          break;
-        }
-        case PH_SORT1: {
-          VIEW;
-          onesweep_tile<1, SORT_ITEMS_LEAN>(v, w.tile, lds);
-          break;
-        }
-        case PH_SORT2: {
-          VIEW;
-          onesweep_tile<2, SORT_ITEMS_LEAN>(v, w.tile, lds);
-          break;
-        }
-        case PH_SORT3: {
-          VIEW;
-          onesweep_tile<3, SORT_ITEMS_LEAN>(v, w.tile, lds);
-          break;
-        }
-        case PH_KARRAS: {
-          VIEW;
-          karras_tile<NODE_TILE / KARRAS_PARTS>(v, w.tile * KARRAS_PARTS + part, lds);
-          break;
-        }
-        case PH_REFIT: {  // chunk-union refit, pass 1 (with the chunks' wide records)
-          VIEW;
-          const uint32_t chunk = w.tile * BATCH_REFIT_CHUNKS + part;
-          if (chunk * BATCH_REFIT_CHUNK < v.n) refit_chunk_tile<BATCH_REFIT_CHUNK>(v, chunk, lds);
-          break;
-        }
-        case PH_TOP: {  // pass 2: the nodes spanning chunks, a wave per 64 nodes
-          VIEW;
-          for (uint32_t t = part; t < (uint32_t)BATCH_SPAN_TILES; t += SPAN_PARTS)
-            refit_span_wave<BATCH_REFIT_CHUNK>(
-                v.B, v.n, (w.tile * BATCH_SPAN_TILES + t) * BUILD_BLOCK + threadIdx.x);
-          break;
-        }
-        case PH_WIDEN: {  // wide records of the spanning nodes
-          VIEW;
-          for (uint32_t t = part; t < (uint32_t)BATCH_SPAN_TILES; t += SPAN_PARTS) {
-            const uint32_t i = (w.tile * BATCH_SPAN_TILES + t) * BUILD_BLOCK + threadIdx.x;
-            if (i + 1u < v.n && spans_chunks<BATCH_REFIT_CHUNK>(v.B, i)) widen_global(v.B, i);
-          }
-          break;
-        }
-        default:
-          break;
-      }
-#undef VIEW
-      __syncthreads();
+      const BatchMeshDev m = load_uniform(a.meshes + src.held.mesh);
+      src.mesh = src.held.mesh, src.kind = src.held.tile & BATCH_ANY_BIT, src.nrays = m.nrays;
+      src.first = true, src.have_held = false;
+      trace_mesh<DEPTH, TSTACK, WIDE>(a, m, lds, &src);
+      if (!src.have_held) return;
     }
-   }
-    if (ph + 1 < last) members = grid_barrier(ctl, (uint32_t)(ph + 1), ticket, &s_item);
+  } else {
+    SegQueue<1> queue(0u);
+    for (;;) {
+      if (threadIdx.x == 0) s_item = queue.take(a);
+      __syncthreads();
+      const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
+      __syncthreads();
+      if (it == NO_ITEM) return;
+      const BatchWork w = load_uniform(a.items + it);
+      const BatchMeshDev m = load_uniform(a.meshes + w.mesh);
+      trace_item<DEPTH, TSTACK, WIDE>(a.gstack, a.gdepth, a.ctl + BATCH_CTL_TRACE_ERR, a.ray_tile,
+                                      a.refill_idle, m, w.tile, lds, &s_ctr);
+    }
   }
-  if (threadIdx.x == 0 && members != 0u) {
-    const uint32_t g = ticket % (uint32_t)BATCH_BAR_GROUPS;
-    arrived_last(ctl, (uint32_t)last, members, g, atomicAdd(bar_group(ctl, g), 1u));
-  }
-}
-
-// Clears the queue tickets, the barrier and the error words before a run (a
-// kernel, so that the reset lives in the same captured graph as the run).
-__global__ void k_batch_reset(uint32_t* ctl) {
-  static_assert(BATCH_CTL_WORDS <= 64 && 2 * BATCH_BAR_GROUPS <= 64,
-                "one 64-thread block clears the control and barrier words");
-  // no start stamp yet: the largest value
-  const bool start = threadIdx.x == BATCH_CTL_CLOCK || threadIdx.x == BATCH_CTL_CLOCK + 1;
-  if (threadIdx.x < BATCH_CTL_WORDS) ctl[threadIdx.x] = start ? 0xFFFFFFFFu : 0u;
-  if (threadIdx.x < 2 * BATCH_BAR_GROUPS) *bar_group(ctl, threadIdx.x) = 0u;
-  if (threadIdx.x < BATCH_XCDS) ctl[BATCH_XTICKET_BASE + threadIdx.x * BATCH_BAR_STRIDE] = 0u;
 }
 
 typedef void (*BatchFn)(BatchArgs);
@@ -508,29 +331,29 @@ struct BatchVariant {
   bool tstack;
   BatchFn fn;
 };
-// The build kernel of a batch run, by waves per SIMD (the register cap trades
-// occupancy against spills of the sort phase's look-back window).
-const BatchFn kBuild[] = {k_batch<0, false, 8, KM_BUILD, false>, k_batch<0, false, 7, KM_BUILD, false>,
-                          k_batch<0, false, 6, KM_BUILD, false>, k_batch<0, false, 5, KM_BUILD, false>,
-                          k_batch<0, false, 4, KM_BUILD, false>};
+// The sort passes of a batch build, by waves per SIMD (the register cap trades
+// occupancy against spills of their look-back window).
+#define RQ_SORTS(W) {k_batch_sort<0, W>, k_batch_sort<1, W>, k_batch_sort<2, W>, k_batch_sort<3, W>}
+const BatchFn kSort[][SORT_PASSES] = {RQ_SORTS(8), RQ_SORTS(7), RQ_SORTS(6), RQ_SORTS(5), RQ_SORTS(4)};
+#undef RQ_SORTS
 constexpr int kBuildWaves[] = {8, 7, 6, 5, 4};
-constexpr int kNumBuildVariants = sizeof(kBuild) / sizeof(kBuild[0]);
+constexpr int kNumBuildVariants = sizeof(kBuildWaves) / sizeof(kBuildWaves[0]);
 // Trace kernels of a batch run (4-wide walk): the batch configurations.
 const BatchVariant kBatchVariants[] = {
-    {24, false, k_batch<24, false, 6, KM_TRACE, true>},
-    {16, false, k_batch<16, false, 8, KM_TRACE, true>},
-    {32, false, k_batch<32, false, 4, KM_TRACE, true>},
-    {12, true, k_batch<12, true, 6, KM_TRACE, true>},
-    {28, false, k_batch<28, false, 5, KM_TRACE, true>},
-    {30, false, k_batch<30, false, 5, KM_TRACE, true>}};
+    {24, false, k_batch_trace<24, false, 6, true>},
+    {16, false, k_batch_trace<16, false, 8, true>},
+    {32, false, k_batch_trace<32, false, 4, true>},
+    {12, true, k_batch_trace<12, true, 6, true>},
+    {28, false, k_batch_trace<28, false, 5, true>},
+    {30, false, k_batch_trace<30, false, 5, true>}};
 // Trace kernels of the serving loop: binary walks (0-5), then 4-wide walks
 // with block-shared items (6-7; the slots keep wide nodes).
 const BatchVariant kServeVariants[] = {
-    {16, false, k_batch<16, false, 7, KM_TRACE, false>}, {20, false, k_batch<20, false, 7, KM_TRACE, false>},
-    {8, true, k_batch<8, true, 7, KM_TRACE, false>},     {10, true, k_batch<10, true, 7, KM_TRACE, false>},
-    {16, false, k_batch<16, false, 8, KM_TRACE, false>}, {8, true, k_batch<8, true, 8, KM_TRACE, false>},
-    {16, false, k_batch<16, false, 5, KM_TRACE, true, false>},
-    {16, false, k_batch<16, false, 8, KM_TRACE, true, false>}};
+    {16, false, k_batch_trace<16, false, 7, false>}, {20, false, k_batch_trace<20, false, 7, false>},
+    {8, true, k_batch_trace<8, true, 7, false>},     {10, true, k_batch_trace<10, true, 7, false>},
+    {16, false, k_batch_trace<16, false, 8, false>}, {8, true, k_batch_trace<8, true, 8, false>},
+    {16, false, k_batch_trace<16, false, 5, true, false>},
+    {16, false, k_batch_trace<16, false, 8, true, false>}};
 constexpr int kServeWideFirst = 6;
 constexpr int kNumBatchVariants = sizeof(kBatchVariants) / sizeof(kBatchVariants[0]);
 constexpr int kNumServeVariants = sizeof(kServeVariants) / sizeof(kServeVariants[0]);
@@ -559,18 +382,29 @@ void serve_variant_info(int v, int* depth, int* tstack, int* wide) {
 }
 int batch_num_build_variants() { return kNumBuildVariants; }
 int batch_build_waves(int b) { return kBuildWaves[b]; }
-uint32_t batch_build_grid_blocks(int device, int b) { return grid_blocks(device, kBuild[b]); }
+uint32_t batch_build_grid_blocks(int device, int b) { return grid_blocks(device, kSort[b][0]); }
 uint32_t batch_trace_grid_blocks(int device, int v) {
   return grid_blocks(device, kBatchVariants[v].fn);
 }
 uint32_t serve_grid_blocks(int device, int v) { return grid_blocks(device, kServeVariants[v].fn); }
 
-hipError_t launch_batch(const LaunchCtx& lc, const BatchArgs& a, int build, uint32_t build_grid,
-                        int variant, uint32_t trace_grid) {
-  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, lc.stream, a.ctl);
+hipError_t launch_batch(const LaunchCtx& lc, const BatchArgs& a, int build, int variant,
+                        uint32_t trace_grid) {
   {
     ProfScope ps(lc, "batch_build");
-    hipLaunchKernelGGL(kBuild[build], dim3(build_grid), dim3(BUILD_BLOCK), 0, lc.stream, a);
+    auto phase = [&](int ph, BatchFn fn, uint32_t parts, int block) {
+      const uint32_t items = a.phase_begin[ph + 1] - a.phase_begin[ph];
+      const uint32_t grid = ph == PH_INIT ? std::max(1u, items) : items * parts;
+      if (grid) hipLaunchKernelGGL(fn, dim3(grid), dim3(block), 0, lc.stream, a);
+    };
+    phase(PH_INIT, k_batch_init, 1, BUILD_BLOCK);
+    phase(PH_BOUNDS, k_batch_bounds, 1, TRI_BLOCK);
+    phase(PH_MORTON, k_batch_morton, 1, TRI_BLOCK);
+    for (int p = 0; p < SORT_PASSES; ++p) phase(PH_SORT0 + p, kSort[build][p], 1, BUILD_BLOCK);
+    phase(PH_KARRAS, k_batch_karras, KARRAS_PARTS, BUILD_BLOCK);
+    phase(PH_REFIT, k_batch_refit, 1, BATCH_REFIT_CHUNK);
+    phase(PH_TOP, k_batch_span, BATCH_SPAN_TILES, BUILD_BLOCK);
+    phase(PH_WIDEN, k_batch_widen, BATCH_SPAN_TILES, BUILD_BLOCK);
   }
   {
     ProfScope ps(lc, "batch_trace");

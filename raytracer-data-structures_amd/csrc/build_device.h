@@ -2,8 +2,8 @@
 // sort -> Karras emission -> two-pass refit). Each function is one unit of
 // work for one block of BUILD_BLOCK (256) threads (the triangle passes take
 // the block size as a parameter): the standalone kernels in
-// build_kernels.hip launch one block per unit, the persistent batch kernel in
-// batch_kernels.hip pulls the same units from its work queue. LDS scratch is
+// build_kernels.hip launch one block per unit, the batch kernels in
+// batch_kernels.hip one per unit of every mesh. LDS scratch is
 // passed in so that a kernel calling several phases holds one buffer.
 //
 // Replaces constructLBVHTree (accelerators.h:570-586): its Morton step
@@ -503,11 +503,10 @@ constexpr int karras_lds_words() {
   return TILE + 2 * KARRAS_HALO;
 }
 
-// TILE internal nodes per unit: the batch kernel queues NODE_TILE, the
-// standalone kernel one node per thread (each node is an independent chain of
-// dependent key loads, so more units hide more latency). lds holds
-// karras_lds_words<TILE>() words.
-template <int TILE = NODE_TILE>
+// TILE internal nodes per unit: the kernels take one node per thread (each node
+// is an independent chain of dependent key loads, so more units hide more
+// latency). lds holds karras_lds_words<TILE>() words.
+template <int TILE>
 __device__ inline void karras_tile(const BuildView& v, uint32_t tile, uint32_t* lds) {
   if (v.n < 2) return;
   const int64_t begin = (int64_t)tile * TILE;
@@ -666,9 +665,8 @@ __device__ inline uint32_t leaf_depth(const BuildBuffers& B, uint32_t n, uint32_
 }
 
 // ---- chunk-union refit ------------------------------------------------------------
-// Pass 1, one block of CHUNK threads per chunk of CHUNK leaves (the standalone
-// build: REFIT_CHUNK = 1024; the batch kernel: its 256-thread blocks):
-// each thread writes its leaf record, the block scans the leaf boxes into
+// Pass 1, one block of CHUNK threads per chunk of CHUNK leaves (REFIT_CHUNK =
+// 1024 in the standalone and the batch build): each thread writes its leaf record, the block scans the leaf boxes into
 // per-leaf prefix and suffix unions of the chunk (and the chunk's union), and
 // each leaf climbs while the node's leaf range lies inside the chunk: the
 // second of a node's two arrivals (an arrival counter) unions the sibling's

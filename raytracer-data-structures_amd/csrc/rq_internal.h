@@ -61,9 +61,9 @@ static_assert(sizeof(WideNode) == 64, "wide node record is 64 bytes");
 constexpr float WIDE_Q0 = 1024.0f;
 
 // Radix sort tiling (onesweep): WAVES*64 threads, ITEMS keys per thread.
-// The standalone build sorts 16 keys per thread; the batch kernel, whose
-// register budget is set by traversal, sorts 8 (SORT_ITEMS_LEAN). Look-back
-// status words are allocated for the smaller tile, so either fits.
+// A large standalone build sorts 16 keys per thread; a small one and the batch
+// build, many small ones, sort 8 (SORT_ITEMS_LEAN). Look-back status words are
+// allocated for the smaller tile, so either fits.
 constexpr int SORT_WAVES = 4;
 constexpr int SORT_ITEMS = 16;
 constexpr int SORT_ITEMS_LEAN = 8;
@@ -72,12 +72,10 @@ constexpr int SORT_TILE = SORT_BLOCK * SORT_ITEMS;
 constexpr int SORT_TILE_LEAN = SORT_BLOCK * SORT_ITEMS_LEAN;
 constexpr int SORT_PASSES = 4;  // 30-bit codes, 8-bit digits
 
-// Refit: a block owns REFIT_CHUNK consecutive leaves (the standalone kernel
-// one leaf per thread, the batch kernel four); the top pass runs in one
-// work-group.
+// Refit: a block owns REFIT_CHUNK consecutive leaves, one per thread.
 constexpr int REFIT_CHUNK = 1024;
-// The smallest refit chunk (the batch kernel's 256-thread blocks): the
-// chunk-union buffers hold one union per chunk of this size.
+// The smallest refit chunk: the chunk-union buffers hold one union per chunk
+// of this size.
 constexpr int REFIT_CHUNK_MIN = 256;
 
 // Lookback status word: [31:30] flag, [29:0] count.

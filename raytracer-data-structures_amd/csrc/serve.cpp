@@ -478,7 +478,7 @@ bool launch_step(rq_server* s) {
   const uint32_t grid = std::min(s->grid, std::max(1u, tiles_of(ni, BATCH_XCDS)) * BATCH_XCDS);
   if (e == hipSuccess) e = launch_serve_trace(LaunchCtx{s->s_trace, nullptr}, a, s->variant, grid);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(s->err_host[buf], s->ctl + BATCH_CTL_BARRIER_ERR, 2 * sizeof(uint32_t),
+    e = hipMemcpyAsync(s->err_host[buf], s->ctl + BATCH_CTL_TRACE_ERR, sizeof(uint32_t),
                        hipMemcpyDeviceToHost, s->s_trace);
   if (e == hipSuccess) e = hipEventRecord(st->end, s->s_trace);
   // Each chunk's results go to the caller's (page-locked) host arrays as soon
@@ -546,7 +546,7 @@ void retire_steps(rq_server* s) {
     const hipError_t e = hipEventQuery(st->end);
     if (e == hipErrorNotReady) return;
     const int buf = (int)(st - s->steps);
-    const bool bad = e != hipSuccess || s->err_host[buf][0] || s->err_host[buf][1];
+    const bool bad = e != hipSuccess || s->err_host[buf][0];
     float ms = 0.0f;
     if (e == hipSuccess) (void)hipEventElapsedTime(&ms, st->start, st->end);
     uint64_t rays = 0;
@@ -768,11 +768,11 @@ int rq_server_create(int device, const rq_server_config* cfg_in, rq_server** out
                               hipHostMallocDefault) != hipSuccess ||
                 hipHostMalloc((void**)&s->host_items[b], s->max_items * sizeof(BatchWork),
                               hipHostMallocDefault) != hipSuccess ||
-                hipHostMalloc((void**)&s->err_host[b], 2 * sizeof(uint32_t),
+                hipHostMalloc((void**)&s->err_host[b], sizeof(uint32_t),
                               hipHostMallocDefault) != hipSuccess))
       rc = set_err(c, RQ_E_NOMEM, "pinned staging");
     if (!rc) {
-      s->err_host[b][0] = s->err_host[b][1] = 0;
+      s->err_host[b][0] = 0;
       if (hipEventCreate(&s->steps[b].start) != hipSuccess ||
           hipEventCreate(&s->steps[b].end) != hipSuccess)
         rc = RQ_E_HIP;

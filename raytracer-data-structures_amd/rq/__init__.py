@@ -849,7 +849,7 @@ class Context:
 
 
 class Batch:
-    """rq_batch: many meshes built and traced in one persistent launch.
+    """rq_batch: many meshes built and traced in one run.
 
     items: dicts with keys scene (rq_scene handle), rays (DeviceRays or None),
     hits (dict of DeviceArray: prim required, t/u/v optional; None skips the
@@ -934,7 +934,7 @@ class Batch:
         return w.value
 
     def occupancy(self) -> tuple[int, int]:
-        """rq_batch_occupancy: (blocks that took part in the last run, launch grid)."""
+        """rq_batch_occupancy: (members, grid), the same once the batch has run."""
         m, g = C.c_uint32(), C.c_uint32()
         self.ctx._check(lib().rq_batch_occupancy(self.ctx.h, self.h, C.byref(m), C.byref(g)))
         return m.value, g.value
