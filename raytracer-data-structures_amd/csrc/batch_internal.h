@@ -39,8 +39,8 @@ constexpr int BATCH_XTICKET_BASE = BATCH_XTICKET_STRIDE;
 constexpr int BATCH_CTL_ALLOC_WORDS = BATCH_XTICKET_BASE + BATCH_XCDS * BATCH_XTICKET_STRIDE;
 static_assert(BATCH_CTL_WORDS <= BATCH_XTICKET_BASE, "control words before the tickets");
 constexpr uint32_t BATCH_ANY_BIT = 0x80000000u;            // trace item tile: any-hit query
-// Work items of the refit phases (see batch_kernels.hip): refit chunks of
-// BUILD_BLOCK leaves, BATCH_REFIT_CHUNKS per item; spanning nodes in tiles of
+// Work items of the refit phases (see batch_kernels.hip): BATCH_REFIT_CHUNKS
+// times BUILD_BLOCK leaves an item of the first; spanning nodes in tiles of
 // BUILD_BLOCK, BATCH_SPAN_TILES per item.
 constexpr uint32_t BATCH_REFIT_CHUNKS = 4;
 constexpr uint32_t BATCH_SPAN_TILES = 8;

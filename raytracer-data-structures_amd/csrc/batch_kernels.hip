@@ -264,12 +264,15 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_batch_karras(BatchArgs a) {
   const PhaseUnit<KARRAS_PARTS> u(a, PH_KARRAS);
   karras_tile<BUILD_BLOCK>(u.v, u.tile, lds);
 }
-// Chunk-union refit, pass 1 (with the chunks' wide records), a block an item.
-constexpr int BATCH_REFIT_CHUNK = BUILD_BLOCK * BATCH_REFIT_CHUNKS;
+// Chunk-union refit, pass 1 (with the chunks' wide records), a block a chunk.
+// (48 meshes: 512 leaves a chunk 1815 us, 256 1825.)
+constexpr int BATCH_REFIT_CHUNK = 2 * BUILD_BLOCK;
+constexpr uint32_t REFIT_PARTS = BATCH_REFIT_CHUNKS / 2;
+static_assert(BATCH_REFIT_CHUNK >= REFIT_CHUNK_MIN, "the chunk unions are allocated for this");
 __global__ __launch_bounds__(BATCH_REFIT_CHUNK) void k_batch_refit(BatchArgs a) {
-  __shared__ uint32_t lds[refit_chunk_lds_words<BATCH_REFIT_CHUNK>()];
-  const PhaseUnit<1> u(a, PH_REFIT);
-  refit_chunk_tile<BATCH_REFIT_CHUNK>(u.v, u.tile, lds);
+  __shared__ __align__(8) uint32_t lds[refit_chunk_lds_words<BATCH_REFIT_CHUNK>()];
+  const PhaseUnit<REFIT_PARTS> u(a, PH_REFIT);
+  if (u.tile * BATCH_REFIT_CHUNK < u.v.n) refit_chunk_tile<BATCH_REFIT_CHUNK>(u.v, u.tile, lds);
   stamp_end(a, PH_REFIT);
 }
 // Pass 2: the nodes spanning chunks, a wave per 64 nodes; then their wide
@@ -402,7 +405,7 @@ hipError_t launch_batch(const LaunchCtx& lc, const BatchArgs& a, int build, int 
     phase(PH_MORTON, k_batch_morton, 1, TRI_BLOCK);
     for (int p = 0; p < SORT_PASSES; ++p) phase(PH_SORT0 + p, kSort[build][p], 1, BUILD_BLOCK);
     phase(PH_KARRAS, k_batch_karras, KARRAS_PARTS, BUILD_BLOCK);
-    phase(PH_REFIT, k_batch_refit, 1, BATCH_REFIT_CHUNK);
+    phase(PH_REFIT, k_batch_refit, REFIT_PARTS, BATCH_REFIT_CHUNK);
     phase(PH_TOP, k_batch_span, BATCH_SPAN_TILES, BUILD_BLOCK);
     phase(PH_WIDEN, k_batch_widen, BATCH_SPAN_TILES, BUILD_BLOCK);
   }

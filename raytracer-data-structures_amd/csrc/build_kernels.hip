@@ -61,7 +61,7 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_karras(BuildView v) {
 
 template <int CHUNK>
 __global__ __launch_bounds__(CHUNK) void k_refit_chunk(BuildView v) {
-  __shared__ uint32_t lds[refit_chunk_lds_words<CHUNK>()];
+  __shared__ __align__(8) uint32_t lds[refit_chunk_lds_words<CHUNK>()];
   refit_chunk_tile<CHUNK>(v, blockIdx.x, lds);
 }
 
@@ -84,12 +84,30 @@ __global__ __launch_bounds__(256) void k_widen_span(BuildBuffers B, uint32_t n) 
   if (spans_chunks<CHUNK>(B, i)) widen_global(B, i);
 }
 
-// Leaves per chunk (and threads per block) of the standalone chunk-union
-// refit. 256-leaf chunks (eight blocks per CU instead of two) measured the
-// same for pass 1 on a 1.31 M-triangle mesh (0.139 vs 0.138 ms) and made the
-// spanning-node pass slower (0.035 vs 0.020 ms): the pass moves ~370 bytes
-// per leaf and is bound by them, not by its occupancy.
-constexpr int BUILD_REFIT_CHUNK = REFIT_CHUNK;
+// Leaves per chunk (and threads per block) of the refit, by size. A chunk is a
+// chain of barriers and fetches, so small chunks finish sooner and more of them
+// share a CU, but they leave more spanning nodes, and the topmost span every
+// chunk. Pass 1 + spanning nodes + their wide records, us, at 1024 / 512 / 256:
+// 4 k triangles 30 / 25 / 21, 100 k 40 / 32 / 31, 300 k 67 / 58 / 55, 1 M (soup)
+// 161 / 157 / 159, 1.3 M (sphere) 116 / 109 / 122.
+constexpr uint32_t REFIT_SMALL_MAX = 1u << 19;
+template <int CHUNK>
+void launch_refit(const LaunchCtx& lc, const BuildView& v) {
+  const uint32_t n = v.n, chunks = tiles_of(n, CHUNK);
+  hipStream_t s = lc.stream;
+  {
+    ProfScope ps(lc, "refit");
+    hipLaunchKernelGGL(k_refit_chunk<CHUNK>, dim3(chunks), dim3(CHUNK), 0, s, v);
+  }
+  if (chunks > 1) {
+    ProfScope ps(lc, "refit_top");
+    hipLaunchKernelGGL(k_refit_span<CHUNK>, dim3(tiles_of(n - 1, 256)), dim3(256), 0, s, v.B, n);
+  }
+  if (chunks > 1 && v.B.wide) {
+    ProfScope ps(lc, "widen");
+    hipLaunchKernelGGL(k_widen_span<CHUNK>, dim3(tiles_of(n - 1, 256)), dim3(256), 0, s, v.B, n);
+  }
+}
 
 // Tree height: each block's deepest leaf to B.flags[block] (free once the
 // refit is done), k_height reduces them (a device atomic per wave on one word
@@ -152,20 +170,10 @@ hipError_t launch_build(const LaunchCtx& lc, const float* vx, const float* vy, c
   }
   // chunk-union refit (pass 1 with the chunk-internal wide records, pass 2
   // for the nodes spanning chunks, then their wide records)
-  constexpr int C = BUILD_REFIT_CHUNK;
-  const uint32_t cchunks = tiles_of(n, C);
-  {
-    ProfScope ps(lc, "refit");
-    hipLaunchKernelGGL(k_refit_chunk<C>, dim3(cchunks), dim3(C), 0, s, v);
-  }
-  if (cchunks > 1) {
-    ProfScope ps(lc, "refit_top");
-    hipLaunchKernelGGL(k_refit_span<C>, dim3(tiles_of(n - 1, 256)), dim3(256), 0, s, B, n);
-  }
-  if (cchunks > 1 && B.wide) {
-    ProfScope ps(lc, "widen");
-    hipLaunchKernelGGL(k_widen_span<C>, dim3(tiles_of(n - 1, 256)), dim3(256), 0, s, B, n);
-  }
+  if (n < REFIT_SMALL_MAX)
+    launch_refit<REFIT_CHUNK_MIN>(lc, v);
+  else
+    launch_refit<REFIT_CHUNK>(lc, v);
   return hipGetLastError();
 }
 

@@ -72,10 +72,10 @@ constexpr int SORT_TILE = SORT_BLOCK * SORT_ITEMS;
 constexpr int SORT_TILE_LEAN = SORT_BLOCK * SORT_ITEMS_LEAN;
 constexpr int SORT_PASSES = 4;  // 30-bit codes, 8-bit digits
 
-// Refit: a block owns REFIT_CHUNK consecutive leaves, one per thread.
-constexpr int REFIT_CHUNK = 1024;
-// The smallest refit chunk: the chunk-union buffers hold one union per chunk
-// of this size.
+// Refit: a block owns a chunk of consecutive leaves, one per thread: of
+// REFIT_CHUNK leaves in a large build and in a batch, of REFIT_CHUNK_MIN in a
+// small one. The chunk-union buffers hold one union per REFIT_CHUNK_MIN leaves.
+constexpr int REFIT_CHUNK = 512;
 constexpr int REFIT_CHUNK_MIN = 256;
 
 // Lookback status word: [31:30] flag, [29:0] count.
