@@ -524,6 +524,30 @@ __global__ __launch_bounds__(256) void k_copy16(const uint4* __restrict__ src,
     dst[i] = src[i];
 }
 
+// The image as it is read: its values and their PPM bytes (main.cpp:521-523),
+// min(1, sum / spp) * 255 cut to an integer as the host's conversion does
+// (through 32 signed bits), four a thread. Bound by the link where the outputs
+// are host memory (15 bytes a pixel).
+__global__ __launch_bounds__(256) void k_image_out(const float* img, size_t count, float spp,
+                                                   float* rgb, uint32_t* words) {
+  const size_t w = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (4 * w >= count) return;
+  float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (4 * w + 4 <= count) {
+    f = reinterpret_cast<const float4*>(img)[w];
+  } else {
+    f.x = img[4 * w];
+    if (4 * w + 1 < count) f.y = img[4 * w + 1];
+    if (4 * w + 2 < count) f.z = img[4 * w + 2];
+  }
+  if (rgb) reinterpret_cast<float4*>(rgb)[w] = f;
+  auto byte = [&](float s) {
+    const float x = s / spp;
+    return (uint32_t)(int32_t)((x < 1.0f ? x : 1.0f) * 255) & 255u;
+  };
+  if (words) words[w] = byte(f.x) | byte(f.y) << 8 | byte(f.z) << 16 | byte(f.w) << 24;
+}
+
 }  // namespace
 
 hipError_t launch_copy16(const LaunchCtx& lc, const void* src, void* dst, uint64_t bytes) {
@@ -596,6 +620,14 @@ hipError_t launch_shade_occlusion(const LaunchCtx& lc, const ShadeParams& sp, ui
   ProfScope ps(lc, "shade_occlusion");
   hipLaunchKernelGGL(k_shade_occlusion, dim3(cdiv(npix, 256)), dim3(256), 0, lc.stream, sp, npix,
                      spp, occ, h0, srgb, img);
+  return hipGetLastError();
+}
+
+hipError_t launch_image_out(const LaunchCtx& lc, const float* img, size_t count, uint32_t spp,
+                            float* rgb, uint8_t* bytes) {
+  const size_t words = (count + 3) / 4;
+  hipLaunchKernelGGL(k_image_out, dim3((uint32_t)((words + 255) / 256)), dim3(256), 0, lc.stream,
+                     img, count, (float)spp, rgb, reinterpret_cast<uint32_t*>(bytes));
   return hipGetLastError();
 }
 

@@ -67,6 +67,10 @@ hipError_t launch_count_active(const LaunchCtx& lc, const RaySoA& R, uint64_t n,
 hipError_t launch_shade_occlusion(const LaunchCtx& lc, const ShadeParams& sp, uint32_t npix,
                                   uint32_t spp, const uint8_t* occ, int32_t* h0, float* srgb,
                                   float* img);
+// Copies count image values (sums over spp samples) to rgb, and writes their PPM
+// bytes, either may be null; both with room for a multiple of four.
+hipError_t launch_image_out(const LaunchCtx& lc, const float* img, size_t count, uint32_t spp,
+                            float* rgb, uint8_t* bytes);
 hipError_t launch_shade_final(const LaunchCtx& lc, const SceneView& s, const ShadeParams& sp,
                               uint32_t npix, uint32_t spp, const RaySoA& prim, const RaySoA& bnc,
                               const int32_t* h0, const float* t0, const int32_t* h1,
