@@ -14,6 +14,13 @@ using namespace rq;
 namespace {
 
 constexpr uint32_t HOST_CHUNK = 1u << 20;  // rays per staged launch
+// Up to HOST_DIRECT_MAX rays the kernel reads and writes the pinned buffer itself:
+// two copies less, against fetches over the link (closest hit and any hit, us,
+// copied / direct: one ray 40, 32 / 38, 29; 1024 62, 56 / 57, 49; 4096 73, 60 /
+// 78, 58). From HOST_OVERLAP_MIN on each array is copied over by itself, beside
+// the host's copy of the next one, in and out (307 k rays 700, 430 / 630, 385; 1 M
+// 2400, 1360 / 1830, 1000; but 131 k 330, 236 / 396, 262: a copy costs 15 us).
+constexpr uint32_t HOST_DIRECT_MAX = 2048, HOST_OVERLAP_MIN = 1u << 18;
 constexpr size_t RAY_BYTES = 8 * sizeof(float);
 constexpr size_t HIT_BYTES = sizeof(int32_t) + 3 * sizeof(float);
 
@@ -61,44 +68,63 @@ int host_query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq_h
   const hipStream_t s = (hipStream_t)stream;
   const float* src[8] = {rays->ox, rays->oy, rays->oz, rays->dx,
                          rays->dy, rays->dz, rays->tmin, rays->tmax};
+  const bool direct = n <= HOST_DIRECT_MAX, overlap = n >= HOST_OVERLAP_MIN;
   for (uint32_t i0 = 0; i0 < n; i0 += HOST_CHUNK) {
     const uint32_t m = std::min(HOST_CHUNK, n - i0), ms = round64(m);
     // packed [8][ms] ray arrays, then the outputs
     char* h = static_cast<char*>(c->stage_host);
-    char* d = static_cast<char*>(c->stage_dev);
-    for (int k = 0; k < 8; ++k) std::memcpy(h + (size_t)k * ms * 4, src[k] + i0, (size_t)m * 4);
-    hipError_t e = hipMemcpyAsync(d, h, (size_t)8 * ms * 4, hipMemcpyHostToDevice, s);
+    char* d = direct ? h : static_cast<char*>(c->stage_dev);
+    const size_t arr = (size_t)ms * 4;
+    hipError_t e = hipSuccess;
+    for (int k = 0; k < 8; ++k) {
+      std::memcpy(h + k * arr, src[k] + i0, (size_t)m * 4);
+      if (overlap && e == hipSuccess)
+        e = hipMemcpyAsync(d + k * arr, h + k * arr, arr, hipMemcpyHostToDevice, s);
+    }
+    if (!direct && !overlap) e = hipMemcpyAsync(d, h, 8 * arr, hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return hip_err(c, e, "staging copy in");
     const float* df = reinterpret_cast<const float*>(d);
     const rq_rays dr{df, df + ms, df + 2 * (size_t)ms, df + 3 * (size_t)ms,
                      df + 4 * (size_t)ms, df + 5 * (size_t)ms, df + 6 * (size_t)ms,
                      df + 7 * (size_t)ms};
-    char* dout = d + (size_t)8 * ms * 4;
-    char* hout = h + (size_t)8 * ms * 4;
-    size_t out_bytes = 0;
+    char* dout = d + 8 * arr;
+    char* hout = h + 8 * arr;
+    // the outputs, one behind the other from dout on
+    void* out[4] = {any ? (void*)occ : hits->prim, any ? nullptr : hits->t,
+                    any ? nullptr : hits->u, any ? nullptr : hits->v};
+    const size_t width = any ? 1 : 4;
+    int arrays = 0;
+    for (int k = 0; k < 4; ++k)
+      if (out[k]) arrays = k + 1;
     if (any) {
       rc = rq_any_hit(c, b, &dr, m, reinterpret_cast<uint8_t*>(dout), stream);
-      out_bytes = m;
     } else {
       rq_hits dh{reinterpret_cast<int32_t*>(dout),
-                 hits->t ? reinterpret_cast<float*>(dout + (size_t)ms * 4) : nullptr,
-                 hits->u ? reinterpret_cast<float*>(dout + (size_t)ms * 8) : nullptr,
-                 hits->v ? reinterpret_cast<float*>(dout + (size_t)ms * 12) : nullptr};
+                 hits->t ? reinterpret_cast<float*>(dout + arr) : nullptr,
+                 hits->u ? reinterpret_cast<float*>(dout + 2 * arr) : nullptr,
+                 hits->v ? reinterpret_cast<float*>(dout + 3 * arr) : nullptr};
       rc = rq_closest_hit(c, b, &dr, m, &dh, stream);
-      out_bytes = (size_t)ms * 4 * (hits->v ? 4 : hits->u ? 3 : hits->t ? 2 : 1);
     }
     if (rc) return rc;
-    e = hipMemcpyAsync(hout, dout, out_bytes, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return hip_err(c, e, "staging copy out");
-    if (any) {
-      std::memcpy(occ + i0, hout, m);
-    } else {
-      std::memcpy(hits->prim + i0, hout, (size_t)m * 4);
-      if (hits->t) std::memcpy(hits->t + i0, hout + (size_t)ms * 4, (size_t)m * 4);
-      if (hits->u) std::memcpy(hits->u + i0, hout + (size_t)ms * 8, (size_t)m * 4);
-      if (hits->v) std::memcpy(hits->v + i0, hout + (size_t)ms * 12, (size_t)m * 4);
+    if (!direct && !overlap)
+      e = hipMemcpyAsync(hout, dout, any ? m : arrays * arr, hipMemcpyDeviceToHost, s);
+    for (int k = 0; overlap && k < arrays && e == hipSuccess; ++k) {
+      if (out[k])
+        e = hipMemcpyAsync(hout + k * arr, dout + k * arr, m * width, hipMemcpyDeviceToHost, s);
+      if (k + 1 == arrays || !out[k] || e != hipSuccess) continue;
+      hipEvent_t& ev = c->stage_done[k];
+      if (!ev) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+      if (e == hipSuccess) e = hipEventRecord(ev, s);
     }
+    if (e == hipSuccess && !overlap) e = hipStreamSynchronize(s);
+    for (int k = 0; k < arrays && e == hipSuccess; ++k) {
+      if (!out[k]) continue;
+      if (overlap)
+        e = k + 1 == arrays ? hipStreamSynchronize(s) : hipEventSynchronize(c->stage_done[k]);
+      if (e == hipSuccess)
+        std::memcpy(static_cast<char*>(out[k]) + i0 * width, hout + k * arr, m * width);
+    }
+    if (e != hipSuccess) return hip_err(c, e, "staging copy out");
   }
   return RQ_OK;
 }
@@ -110,6 +136,10 @@ void stage_release(rq_ctx* c) {
   if (c->stage_host) (void)hipHostFree(c->stage_host);
   c->stage_host = nullptr;
   c->stage_dev = nullptr;  // freed with the context's allocations
+  for (hipEvent_t& ev : c->stage_done) {
+    if (ev) (void)hipEventDestroy(ev);
+    ev = nullptr;
+  }
   c->stage_bytes = 0;
 }
 }  // namespace rq

@@ -46,6 +46,7 @@ struct rq_ctx {
   void* stage_host = nullptr;
   void* stage_dev = nullptr;
   size_t stage_bytes = 0;
+  hipEvent_t stage_done[3] = {};  // a staged output array is in the pinned buffer
   // device address of the allocation-free entry's scratch on this device
   // (hipGetSymbolAddress at rq_create)
   unsigned char* scratch = nullptr;
