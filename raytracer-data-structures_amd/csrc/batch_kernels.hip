@@ -57,7 +57,7 @@ __device__ inline T load_uniform(const T* p) {
 template <int DEPTH, bool TSTACK, bool WIDE>
 __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* err,
                                   uint32_t ray_tile, uint32_t refill_idle, const BatchMeshDev& m,
-                                  uint32_t tile, uint32_t* lds, uint32_t* s_ctr) {
+                                  uint32_t tile, uint32_t* lds, uint32_t* s_ctr, SplitSlots* slots) {
   const bool any = (tile & BATCH_ANY_BIT) != 0;
   const uint32_t r0 = (tile & ~BATCH_ANY_BIT) * ray_tile;
   const uint32_t nr = min(ray_tile, m.nrays - r0);
@@ -81,13 +81,13 @@ __device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* er
   ItemRays src{s_ctr, nr};
   if (any) {
     t.occ = m.occ + r0;
-    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE>(t, src, s_node, s_tn);
+    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE, true>(t, src, s_node, s_tn, slots);
   } else {
     t.prim = m.prim + r0;
     t.t = m.t ? m.t + r0 : nullptr;
     t.u = m.u ? m.u + r0 : nullptr;
     t.v = m.v_ ? m.v_ + r0 : nullptr;
-    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE>(t, src, s_node, s_tn);
+    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE, true>(t, src, s_node, s_tn, slots);
   }
   __syncthreads();
 }
@@ -181,13 +181,13 @@ __device__ inline void trace_mesh(const BatchArgs& a, const BatchMeshDev& m, uin
   float* s_tn = reinterpret_cast<float*>(lds + DEPTH * BUILD_BLOCK);
   if (src->kind) {
     t.occ = m.occ;
-    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE>(t, *src, s_node, s_tn);
+    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE, false>(t, *src, s_node, s_tn);
   } else {
     t.prim = m.prim;
     t.t = m.t;
     t.u = m.u;
     t.v = m.v_;
-    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE>(t, *src, s_node, s_tn);
+    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE, false>(t, *src, s_node, s_tn);
   }
 }
 
@@ -313,6 +313,9 @@ k_batch_trace(BatchArgs a) {
       if (!src.have_held) return;
     }
   } else {
+    __shared__ SplitSlots s_split[WIDE ? BUILD_BLOCK / 64 : 1];
+    SplitSlots* const slots =
+        s_split + (WIDE ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0u);
     SegQueue<1> queue(0u);
     for (;;) {
       if (threadIdx.x == 0) s_item = queue.take(a);
@@ -323,7 +326,7 @@ k_batch_trace(BatchArgs a) {
       const BatchWork w = load_uniform(a.items + it);
       const BatchMeshDev m = load_uniform(a.meshes + w.mesh);
       trace_item<DEPTH, TSTACK, WIDE>(a.gstack, a.gdepth, a.ctl + BATCH_CTL_TRACE_ERR, a.ray_tile,
-                                      a.refill_idle, m, w.tile, lds, &s_ctr);
+                                      a.refill_idle, m, w.tile, lds, &s_ctr, slots);
     }
   }
 }

@@ -353,11 +353,11 @@ __device__ inline unsigned long long hit_key(float t, int32_t prim) {
 // vector lanes, which held two registers and cost reads in the loop).
 constexpr int ROWS_SMALL = 0, ROWS_BIG = 1, ROWS_ANY = 2;
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
-          int ROWS, class Src, class Cold>
+          int ROWS, bool SHARE, class Src, class Cold>
 __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src& src,
-                                       int32_t* s_node, float* s_tn, SplitSlots* slots = nullptr) {
+                                       int32_t* s_node, float* s_tn, SplitSlots* slots) {
   // (a tree past 32-bit offsets keeps the walk without it)
-  constexpr bool SPLIT = WIDE && ROWS == ROWS_SMALL;
+  constexpr bool SPLIT = WIDE && SHARE && ROWS != ROWS_BIG;
   static_assert(!(WIDE && COUNT), "counted traversal walks the binary nodes");
   const bool big = ROWS == ROWS_ANY ? a.nprims > WIDE_SMALL_MAX_NODES : ROWS == ROWS_BIG;
   const int tid = threadIdx.x;
@@ -712,12 +712,16 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
 }
 
 // One code path for trees of any size (the batch and serving kernels, whose
-// launches walk many trees and hold their build phases in the same kernel).
+// launches walk many trees). SHARE, idle lanes share the last rays (slots): a
+// serving step's items are 256 rays of a block that waits for its longest one
+// (a burst of 16 requests 1515 -> 1380 us with its copies); a batch run's waves
+// refill from item to item, and the code's presence costs them 3 %.
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
-          class Src>
-__device__ inline void trace_loop(const TraceArgs& a, Src& src, int32_t* s_node, float* s_tn) {
-  trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_ANY>(
-      a, [&] { return &a; }, src, s_node, s_tn);
+          bool SHARE, class Src>
+__device__ inline void trace_loop(const TraceArgs& a, Src& src, int32_t* s_node, float* s_tn,
+                                  SplitSlots* slots = nullptr) {
+  trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_ANY, SHARE>(
+      a, [&] { return &a; }, src, s_node, s_tn, slots);
 }
 // A path per record addressing, chosen once per launch (the query kernels:
 // one tree).
@@ -725,10 +729,10 @@ template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool WIDE, cl
 __device__ inline void trace_loop_split(const TraceArgs& a, const Cold& cold, Src& src,
                                         int32_t* s_node, float* s_tn, SplitSlots* slots) {
   if (WIDE && a.nprims > WIDE_SMALL_MAX_NODES)
-    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE, ROWS_BIG>(
+    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE, ROWS_BIG, false>(
         a, cold, src, s_node, s_tn, slots);
   else
-    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE, ROWS_SMALL>(
+    trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, true, WIDE, ROWS_SMALL, true>(
         a, cold, src, s_node, s_tn, slots);
 }
 

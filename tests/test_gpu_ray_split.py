@@ -74,3 +74,31 @@ def test_split_rays_match_oracle(ctx, O, rq, kind, n):
         ctx.trace_config(*saved)
         ctx.release(b)
         ctx.release(s)
+
+
+# a serving step: tiles of 256 rays, the last one partial, walked to the end
+@pytest.mark.parametrize("kind", ["overlap", "ties", "row"])
+def test_split_rays_in_a_serving_step(ctx, O, rq, kind):
+    mesh, parts = _scene(kind)
+    rays = concat_rays(*parts)
+    srv = rq.Server(0, mesh_slots=2, slot_tris=1 << 13, arena_bytes=64 << 20, max_inflight=8,
+                    step_rays=1 << 16, chunk_rays=1 << 14, ray_tile=1024, hbm_budget=4 << 30)
+    ob = O.OracleBVH(mesh, 1)
+    try:
+        slot = srv.load_mesh(mesh)
+        jobs = []
+        for n in (1, 255, 257, 4099, 40001):
+            part = {k: a[-n:].copy() if n < 300 else a[:n].copy() for k, a in rays.items()}
+            out = (np.empty(n, np.int32), np.empty(n, np.float32), np.empty(n, np.uint8))
+            tk = srv.submit(n, rq.Q_CLOSEST | rq.Q_ANY, mesh=slot, rays=part, prim=out[0],
+                            t=out[1], occ=out[2])
+            jobs.append((part, out, tk))
+        for part, out, tk in jobs:
+            log(f"serving step {kind} n={len(out[0])}")
+            srv.wait(tk)
+            o = ob.closest(part)
+            assert np.array_equal(out[0], o["prim"])
+            assert np.array_equal(_bits(out[1]), _bits(o["t"]))
+            assert np.array_equal(out[2], ob.any(part)["occ"])
+    finally:
+        srv.close()
