@@ -805,7 +805,7 @@ def c4_workload(ctx, count: int = 512):
 
 
 def run_c4(ctx, args) -> int:
-    """512 meshes built and traced (closest + any hit) in one persistent launch
+    """512 meshes built and traced (closest + any hit) in one batch run
     replayed from a hipGraph, against the plain per-request path (per mesh:
     LBVH rebuild, closest-hit launch, any-hit launch, wait) on the same
     device-resident meshes, rays and output buffers."""
@@ -835,7 +835,7 @@ def run_c4(ctx, args) -> int:
         copy_probe(ctx)
         return 0
 
-    # ---- batched: K replays of the captured persistent launch
+    # ---- batched: K replays of the captured run
     ctx.profile(True)
     ctx.profile_reset()
     ctx.sync()
