@@ -130,11 +130,14 @@ __host__ __device__ inline uint32_t trace_chunk(uint32_t n, uint32_t waves,
 // shared, 93 / 64 / 46 at 8 / 4 / 2; 65 k rays, 100 k triangles: 523, 464,
 // 449 / 440 / 426 at 32 / 16 / 8. One ray a wave gains nothing over two: 4 k
 // rays 139 us against 137, 7 k short ones 32 against 28 (a wave costs its
-// start).
+// start). Above 16 a wave neighbouring rays lose more by their wave's issue
+// than the longest of them gains (200 k camera rays, 300 k triangles: 200 us at
+// 32, 173 at 64; uniform ones 67 and 84; 120 k camera rays at 16 108, at 64 150).
+constexpr uint32_t SPREAD_MAX = 16;
 inline uint32_t spread_chunk(uint32_t n, uint32_t waves) {
   uint32_t c = 2;
-  while (c < 64 && (uint64_t)c * waves < n) c <<= 1;
-  return c;
+  while (c <= SPREAD_MAX && (uint64_t)c * waves < n) c <<= 1;
+  return c <= SPREAD_MAX ? c : 64u;
 }
 // Slice schedule of a standalone launch: slices of `chunk` rays over the
 // first three quarters of the stream, then slices of chunk / 4 (at least 64)

@@ -305,6 +305,11 @@ __device__ inline Row row_load(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
 // gain on camera rays is a third less; sharing only from the 4th, 7th or 10th
 // such step on loses 1 to 10 % on every kind of ray.
 constexpr uint32_t SPLIT_IDLE = 48;
+// Visits that a launch's only ray makes by itself first: one that ends within
+// them does not fetch the helpers' code (a call on a sphere of 80 k triangles
+// 27.8 us at 0, 26.4 at 20 or 32; in a soup of 22 k, where helpers pay, 26 / 30 /
+// 33, and 34 without them).
+constexpr uint32_t SINGLE_ALONE = 20;
 constexpr uint32_t SPLIT_SLOTS = 16;  // split rays of a wave at a time
 struct SplitSlots {
   unsigned long long key[SPLIT_SLOTS];  // ~0: no hit; any hit: 0 once there is one
@@ -378,6 +383,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
   // where lanes share), slots used
   int own;
   uint32_t nslots = 0;
+  uint32_t alone = SPLIT && a.nrays == 1u ? SINGLE_ALONE : 0u;
   const Slots ss = (Slots)slots;
 
   auto write_hit = [&](uint32_t of, bool hit, int32_t prim, float t, float u, float v) {
@@ -694,16 +700,24 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
         if (nidle == 64u) break;
         if (!HELP) {
           if (!wave_out && nidle >= a.refill_idle) break;
-          if (SPLIT && nidle >= SPLIT_IDLE) break;
+          if (SPLIT && nidle >= SPLIT_IDLE) {
+            if (alone == 0u) break;
+            --alone;
+          }
         } else if (nidle >= SPLIT_IDLE) {
           share(idle, nidle);
         }
       }
     };
-    walk(std::false_type{});
-    if (SPLIT) {
+    // (a wave with few rays from the start walks the second copy only: a small
+    // launch pays for the code it fetches)
+    auto sharing = [&] {
       const uint32_t nidle = (uint32_t)__popcll(__ballot(!active));
-      if (nidle != 64u && (wave_out || nidle < a.refill_idle)) {
+      return nidle >= SPLIT_IDLE && nidle != 64u && (wave_out || nidle < a.refill_idle);
+    };
+    if (!SPLIT || alone != 0u || !sharing()) walk(std::false_type{});
+    if (SPLIT) {
+      if (sharing()) {
         own = -1;
         walk(std::true_type{});
       }
