@@ -25,6 +25,7 @@ enum BatchPhase {
 // in those L2s; a block drains its own XCD's segment first, then takes from
 // the others.
 constexpr int BATCH_XCDS = 8;
+static_assert(BATCH_XCDS == (int)TRACE_SEGS, "blocks go to the segments in turn (seg_blocks)");
 
 // control words of one batch
 constexpr int BATCH_CTL_TRACE_ERR = 0;  // stack deeper than provided (this run)
