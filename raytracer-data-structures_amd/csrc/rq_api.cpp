@@ -692,7 +692,7 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
   e = launch_trace(launch_ctx(c, stream), a, any, counted, variant);
   if (e != hipSuccess) return hip_err(c, e, "trace launch");
   // the launch moves each of its slot's counters by the segment's number of
-  // slices, or not at all when its waves' first slices cover it (RayStream)
+  // slices, or not at all when its waves' first slices cover it (QuerySlices)
   for (uint32_t q = 0; !own_zero && q < a.segs; ++q) {
     const uint32_t tq = seg_total(q, a.segs, sched.total);
     if (tq > seg_blocks(q, a.segs, a.grid) * ((uint32_t)blk / 64u)) c->counter_base[slot][q] += tq;

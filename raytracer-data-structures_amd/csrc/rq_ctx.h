@@ -88,7 +88,7 @@ void ctx_free(rq_ctx* c, void* p);
 LaunchCtx launch_ctx(rq_ctx* c, void* stream);
 // The next ray-stream counter slot (round robin over COUNTER_SLOTS). A launch
 // passes counter_base[slot] to its kernel and then adds the number of slices
-// its waves take from each counter (RayStream), so the slot's next launch
+// its waves take from each counter (QuerySlices), so the slot's next launch
 // starts from the counters' values after this one.
 uint32_t next_counter_slot(rq_ctx* c);
 // The stack overflow area of launches on `stream`, allocated on a stream's
