@@ -585,7 +585,8 @@ __device__ inline void wide_empty(WideSlots& w, int k) {
 // rounding is below that for an origin within the grid, and relative to the
 // distance (covered by its slack) for one further away. An extent or a
 // coordinate of 2^100 or more (or one that is not finite) makes the step NaN,
-// and the walk reads a NaN plane as a box that reaches everywhere.
+// and the walk reads a NaN plane as a box that reaches everywhere; other steps
+// are at most 2^92, which the walk relies on (steep in trace_device.h).
 __device__ inline void wide_axis(const float* lo, const float* hi, float* base, float* step,
                                  uint32_t* qlo, uint32_t* qhi) {
   const float l = fminf(fminf(lo[0], lo[1]), fminf(lo[2], lo[3]));

@@ -103,7 +103,7 @@ struct ItemRays {
 
 struct RayState {
   float ox, oy, oz, dx, dy, dz;
-  float ix, iy, iz;  // 1/d (the wide walk: of at most 2^100, wide_inv)
+  float ix, iy, iz;  // 1/d
   bool sx, sy, sz;   // sign bit of 1/d: the near plane of that axis is hi
   float tmin;
 };
@@ -138,23 +138,33 @@ __device__ inline bool slab(const float4& lo, const float4& hi, const RayState& 
   return tn <= tf * slack;
 }
 
-// The wide walk's 1/d: finite, so that a plane on the grid is never inf - inf
-// for a ray parallel to an axis. At 2^100 a plane of the grid, which lies
-// outside the exact box by over 2^-10 of a step of at least 2^-60, is still
-// further than 2^30 on its side of an origin on or inside the exact box.
-__device__ inline float wide_inv(float d) {
-  return copysignf(fminf(fabsf(1.0f / d), 0x1p100f), d);
+// Whether a ray is too steep for the wide walk's short form of a plane's distance,
+// (1024 + q) * (step / d) + (base - o) / d: the two parts are some thousand times
+// the distance, and must both be finite and normal for every step a grid can have
+// (2^-60 to 2^92), which holds for 1/d within 2^-60 and 2^20. Steep rays (parallel
+// to an axis, or nearly; 1/d infinite, 0 or NaN) take ((1024 + q) * step +
+// (base - o)) / d instead: 24 more multiplications a visit, and the exact walk's
+// own reading of an infinite 1/d (a plane on the origin gives NaN, "inside"). They
+// have a copy of the loop: a branch inside the one loop holds both forms'
+// registers (48 meshes 1940 us, 1820 with the copy, 1815 without either). Rays
+// along an axis over 1.3 M triangles, 1 M of them: 164 us, the short form 163.
+__device__ inline bool steep(const RayState& r) {
+  const float x = fabsf(r.ix), y = fabsf(r.iy), z = fabsf(r.iz);
+  return !(fmaxf(fmaxf(x, y), z) <= 0x1p20f && fminf(fminf(x, y), z) >= 0x1p-60f);
 }
-// Four planes of a wide node on one axis, a byte each in q: distances
-// (base + (1024 + q) * step - o) / d as (1024 + q) * si + bi with
-// si = step / d and bi = (base - o) / d.
+// Four planes of a wide node on one axis, a byte each in q: (1024 + q) * si + bi,
+// the distances with si = step / d and bi = (base - o) / d; STEEP, with si = step
+// and bi = base - o, times i = 1/d.
 typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
-__device__ inline float4 wide_planes(uint32_t q, float si, float bi) {
+template <bool STEEP>
+__device__ inline float4 wide_planes(uint32_t q, float si, float bi, float i) {
   // 0x6400 | q is the half-precision 1024 + q
   const Half2 a = __builtin_bit_cast(Half2, __builtin_amdgcn_perm(0x64646464u, q, 0x04010400u));
   const Half2 b = __builtin_bit_cast(Half2, __builtin_amdgcn_perm(0x64646464u, q, 0x04030402u));
-  return make_float4(__builtin_fmaf((float)a[0], si, bi), __builtin_fmaf((float)a[1], si, bi),
-                     __builtin_fmaf((float)b[0], si, bi), __builtin_fmaf((float)b[1], si, bi));
+  const float4 p =
+      make_float4(__builtin_fmaf((float)a[0], si, bi), __builtin_fmaf((float)a[1], si, bi),
+                  __builtin_fmaf((float)b[0], si, bi), __builtin_fmaf((float)b[1], si, bi));
+  return STEEP ? make_float4(p.x * i, p.y * i, p.z * i, p.w * i) : p;
 }
 // Slot test of a wide node: the last axis joins the interval [tn, tf] of the
 // others; eps is the relative slack on the far bound.
@@ -231,15 +241,13 @@ __device__ inline bool sphere_hit(const TriRec& S, const RayState& r, float tmax
 // the exact one where the primitive test leaves a doubt.
 __device__ inline bool leaf_box(const float lo[3], const float hi[3], const RayState& r,
                                 float slack) {
-  const float o[3] = {r.ox, r.oy, r.oz}, d[3] = {r.ix, r.iy, r.iz};
+  const float o[3] = {r.ox, r.oy, r.oz}, i[3] = {r.ix, r.iy, r.iz};
   float tn = r.tmin, tf = INFINITY;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    // an axis without direction, the origin on a plane: inside, as 0 * inf
-    const float i = fabsf(d[k]) < 0x1p100f ? d[k] : copysignf(INFINITY, d[k]);
-    const bool s = signbit(i);
-    tn = fmaxf(((s ? hi[k] : lo[k]) - o[k]) * i, tn);
-    tf = fminf(((s ? lo[k] : hi[k]) - o[k]) * i, tf);
+    const bool s = signbit(i[k]);
+    tn = fmaxf(((s ? hi[k] : lo[k]) - o[k]) * i[k], tn);
+    tf = fminf(((s ? lo[k] : hi[k]) - o[k]) * i[k], tf);
   }
   return tn <= tf * slack;
 }
@@ -478,10 +486,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
         r.ox = c->rays.ox[rr], r.oy = c->rays.oy[rr], r.oz = c->rays.oz[rr];
         r.dx = c->rays.dx[rr], r.dy = c->rays.dy[rr], r.dz = c->rays.dz[rr];
         r.tmin = c->rays.tmin[rr], bt = c->rays.tmax[rr];
-        if (WIDE)
-          r.ix = wide_inv(r.dx), r.iy = wide_inv(r.dy), r.iz = wide_inv(r.dz);
-        else
-          r.ix = 1.0f / r.dx, r.iy = 1.0f / r.dy, r.iz = 1.0f / r.dz;
+        r.ix = 1.0f / r.dx, r.iy = 1.0f / r.dy, r.iz = 1.0f / r.dz;
         r.sx = signbit(r.ix), r.sy = signbit(r.iy), r.sz = signbit(r.iz);
         best = -1, bu = 0.0f, bv = 0.0f, vis = 0, tst = 0, sp = 0;
         node = a.nprims == 1 ? ~0 : 0;
@@ -545,9 +550,10 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
     };
     // ---- traverse until enough lanes are idle to be worth a refill, or, HELP,
     // with the idle lanes' help until all are (its own copy of the loop: the
-    // slots' reads stay out of the other one) -------------------------------
-    auto walk = [&](auto split) {
-      constexpr bool HELP = decltype(split)::value;
+    // slots' reads stay out of the other one); a wave with a steep ray takes a
+    // third copy ---------------------------------------------------------------
+    auto walk = [&](auto split, auto any_steep) {
+      constexpr bool HELP = decltype(split)::value, STEEP = decltype(any_steep)::value;
       for (;;) {
         if (HELP && active && own >= 0) {  // what the ray's other lanes found
           const uint32_t hi = (uint32_t)(ss->key[own] >> 32);
@@ -572,22 +578,23 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
           // hold eight registers more
           float t0, t1, t2, t3, f0, f1, f2, f3;
           {
-            const float sx = __uint_as_float(r0[3]) * r.ix, sy = __uint_as_float(r1[0]) * r.iy;
-            const float bx = (__uint_as_float(r0[0]) - r.ox) * r.ix,
-                        by = (__uint_as_float(r0[1]) - r.oy) * r.iy;
-            const float4 nx = wide_planes(r.sx ? r1[3] : r1[2], sx, bx),
-                         fx = wide_planes(r.sx ? r1[2] : r1[3], sx, bx),
-                         ny = wide_planes(r.sy ? r2[1] : r2[0], sy, by),
-                         fy = wide_planes(r.sy ? r2[0] : r2[1], sy, by);
+            float sx = __uint_as_float(r0[3]), bx = __uint_as_float(r0[0]) - r.ox;
+            float sy = __uint_as_float(r1[0]), by = __uint_as_float(r0[1]) - r.oy;
+            if (!STEEP) sx *= r.ix, bx *= r.ix, sy *= r.iy, by *= r.iy;
+            const float4 nx = wide_planes<STEEP>(r.sx ? r1[3] : r1[2], sx, bx, r.ix),
+                         fx = wide_planes<STEEP>(r.sx ? r1[2] : r1[3], sx, bx, r.ix),
+                         ny = wide_planes<STEEP>(r.sy ? r2[1] : r2[0], sy, by, r.iy),
+                         fy = wide_planes<STEEP>(r.sy ? r2[0] : r2[1], sy, by, r.iy);
             t0 = fmaxf(fmaxf(nx.x, ny.x), r.tmin), f0 = fminf(fminf(fx.x, fy.x), bt);
             t1 = fmaxf(fmaxf(nx.y, ny.y), r.tmin), f1 = fminf(fminf(fx.y, fy.y), bt);
             t2 = fmaxf(fmaxf(nx.z, ny.z), r.tmin), f2 = fminf(fminf(fx.z, fy.z), bt);
             t3 = fmaxf(fmaxf(nx.w, ny.w), r.tmin), f3 = fminf(fminf(fx.w, fy.w), bt);
           }
           __builtin_amdgcn_sched_barrier(0);
-          const float sz = __uint_as_float(r1[1]) * r.iz, bz = (__uint_as_float(r0[2]) - r.oz) * r.iz;
-          const float4 nz = wide_planes(r.sz ? r2[3] : r2[2], sz, bz),
-                       fz = wide_planes(r.sz ? r2[2] : r2[3], sz, bz);
+          float sz = __uint_as_float(r1[1]), bz = __uint_as_float(r0[2]) - r.oz;
+          if (!STEEP) sz *= r.iz, bz *= r.iz;
+          const float4 nz = wide_planes<STEEP>(r.sz ? r2[3] : r2[2], sz, bz, r.iz),
+                       fz = wide_planes<STEEP>(r.sz ? r2[2] : r2[3], sz, bz, r.iz);
           const bool h0 = slot_hit(nz.x, fz.x, eps, t0, f0) & (ln.x != 0);
           const bool h1 = slot_hit(nz.y, fz.y, eps, t1, f1) & (ln.y != 0);
           const bool h2 = slot_hit(nz.z, fz.z, eps, t2, f2) & (ln.z != 0);
@@ -715,11 +722,24 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
       const uint32_t nidle = (uint32_t)__popcll(__ballot(!active));
       return nidle >= SPLIT_IDLE && nidle != 64u && (wave_out || nidle < a.refill_idle);
     };
-    if (!SPLIT || alone != 0u || !sharing()) walk(std::false_type{});
+    const bool any_steep = WIDE && __ballot(active && steep(r)) != 0ull;
+    if constexpr (SPLIT) {
+      if (any_steep) {
+        own = -1;
+        walk(std::true_type{}, std::true_type{});
+      }
+      if (alone != 0u || !sharing()) walk(std::false_type{}, std::false_type{});
+    } else {
+      // (which branch is expected places the loops: 48 meshes 1906 us without, 1820 with)
+      if (__builtin_expect(any_steep, 0))
+        walk(std::false_type{}, std::integral_constant<bool, WIDE>{});
+      else
+        walk(std::false_type{}, std::false_type{});
+    }
     if (SPLIT) {
       if (sharing()) {
         own = -1;
-        walk(std::true_type{});
+        walk(std::true_type{}, std::false_type{});
       }
     }
   }
