@@ -238,7 +238,8 @@ __device__ inline bool sphere_hit(const TriRec& S, const RayState& r, float tmax
 // when the triangle is small for its distance (some rays in ten thousand at
 // 10^6 times its size). The walks answer for the rays that hit the box; a wide
 // node's box on the grid is larger than the exact one, so the wide walk tests
-// the exact one where the primitive test leaves a doubt.
+// the exact one where the primitive test leaves a doubt. (A tree of one primitive
+// has no node, and so no box.)
 __device__ inline bool leaf_box(const float lo[3], const float hi[3], const RayState& r,
                                 float slack) {
   const float o[3] = {r.ox, r.oy, r.oz}, i[3] = {r.ix, r.iy, r.iz};
@@ -675,7 +676,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
           float t, u = 0.0f, v = 0.0f;
           bool done = false, hit;
           if (SPHERES && a.sphere) {
-            hit = sphere_hit(T, r, bt, t) && (!WIDE || sphere_box(T, r));
+            hit = sphere_hit(T, r, bt, t) && (!WIDE || a.nprims < 2u || sphere_box(T, r));
           } else {
             hit = mt(T, r, bt, t, u, v);
             if (WIDE && hit && tri_doubt(T, t)) hit = a.nprims < 2u || tri_box(T, r);
