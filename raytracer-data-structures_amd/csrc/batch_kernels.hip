@@ -51,44 +51,77 @@ __device__ inline T load_uniform(const T* p) {
   return t;
 }
 
-// One trace item (a tile of one mesh's rays), shared by the block's waves: a
-// ray counter in LDS hands out chunks of the tile as lanes go idle; the waves
-// meet at a barrier when it is done.
-template <int DEPTH, bool TSTACK, bool WIDE>
-__device__ inline void trace_item(int32_t* gstack, uint32_t gdepth, uint32_t* err,
-                                  uint32_t ray_tile, uint32_t refill_idle, const BatchMeshDev& m,
-                                  uint32_t tile, uint32_t* lds, uint32_t* s_ctr, SplitSlots* slots) {
-  const bool any = (tile & BATCH_ANY_BIT) != 0;
-  const uint32_t r0 = (tile & ~BATCH_ANY_BIT) * ray_tile;
-  const uint32_t nr = min(ray_tile, m.nrays - r0);
+// What a walk over the rays of mesh `mesh` from r0 on needs seldom, read from the
+// kernel's argument memory and the mesh's descriptor each time (the empty asm hides
+// that they never change): as scalars they crowded out the walk's own.
+template <typename T>
+using Constant = __attribute__((address_space(4))) const T*;
+struct ColdArgs : TraceArgs {
+  __device__ const ColdArgs* operator->() const { return this; }
+};
+struct MeshCold {
+  uint32_t mesh, r0;
+  __device__ Constant<BatchArgs> args() const {
+    Constant<BatchArgs> p = (Constant<BatchArgs>)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+  }
+  __device__ ColdArgs operator()() const {
+    const Constant<BatchArgs> p = args();
+    const Constant<BatchMeshDev> m = (Constant<BatchMeshDev>)p->meshes + mesh;
+    ColdArgs c{};
+    c.rays = rq_rays{m->rays.ox + r0, m->rays.oy + r0, m->rays.oz + r0,   m->rays.dx + r0,
+                     m->rays.dy + r0, m->rays.dz + r0, m->rays.tmin + r0, m->rays.tmax + r0};
+    c.prim = m->prim + r0;
+    c.t = m->t ? m->t + r0 : nullptr;
+    c.u = m->u ? m->u + r0 : nullptr;
+    c.v = m->v_ ? m->v_ + r0 : nullptr;
+    c.occ = m->occ + r0;
+    c.gstack = p->gstack;
+    c.gdepth = p->gdepth;
+    c.err = p->ctl + BATCH_CTL_TRACE_ERR;
+    return c;
+  }
+  __device__ LeafBoxes leaf_boxes() const {
+    const Constant<BatchMeshDev> m = (Constant<BatchMeshDev>)args()->meshes + mesh;
+    return LeafBoxes{m->v.B.parent, m->v.B.nodes};
+  }
+};
+// What it needs all the time.
+__device__ inline TraceArgs hot_args(const BatchMeshDev& m, uint32_t nrays, uint32_t refill_idle) {
   TraceArgs t{};
   t.nodes = m.v.B.nodes;
   t.wide = m.v.B.wide;
   t.tris = m.v.B.tris;
   t.nprims = m.v.n;
-  t.rays = rq_rays{m.rays.ox + r0, m.rays.oy + r0, m.rays.oz + r0, m.rays.dx + r0,
-                   m.rays.dy + r0, m.rays.dz + r0, m.rays.tmin + r0, m.rays.tmax + r0};
-  t.nrays = nr;
-  t.gstack = gstack;
-  t.gdepth = gdepth;
-  t.err = err;
+  t.nrays = nrays;
   t.refill_idle = refill_idle;
   t.sphere = 0;  // batch meshes are triangle scenes
+  return t;
+}
+
+// One trace item (a tile of one mesh's rays), shared by the block's waves: a
+// ray counter in LDS hands out chunks of the tile as lanes go idle; the waves
+// meet at a barrier when it is done.
+template <int DEPTH, bool TSTACK, bool WIDE>
+__device__ inline void trace_item(const BatchArgs& a, const BatchWork& w, uint32_t* lds,
+                                  uint32_t* s_ctr, SplitSlots* slots) {
+  const BatchMeshDev m = load_uniform(a.meshes + w.mesh);
+  const uint32_t r0 = (w.tile & ~BATCH_ANY_BIT) * a.ray_tile;
+  const uint32_t nr = min(a.ray_tile, m.nrays - r0);
+  const TraceArgs t = hot_args(m, nr, a.refill_idle);
   if (threadIdx.x == 0) *s_ctr = 0u;
   __syncthreads();
   int32_t* s_node = reinterpret_cast<int32_t*>(lds);
   float* s_tn = reinterpret_cast<float*>(lds + DEPTH * BUILD_BLOCK);
   ItemRays src{s_ctr, nr};
-  if (any) {
-    t.occ = m.occ + r0;
-    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE, true>(t, src, s_node, s_tn, slots);
-  } else {
-    t.prim = m.prim + r0;
-    t.t = m.t ? m.t + r0 : nullptr;
-    t.u = m.u ? m.u + r0 : nullptr;
-    t.v = m.v_ ? m.v_ + r0 : nullptr;
-    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE, true>(t, src, s_node, s_tn, slots);
-  }
+  const MeshCold cold{w.mesh, r0};
+  if (w.tile & BATCH_ANY_BIT)
+    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE, true>(t, cold, src, s_node,
+                                                                          s_tn, slots);
+  else
+    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE, true>(t, cold, src, s_node,
+                                                                            s_tn, slots);
   __syncthreads();
 }
 
@@ -165,30 +198,16 @@ struct ItemSlices {
 template <int DEPTH, bool TSTACK, bool WIDE>
 __device__ inline void trace_mesh(const BatchArgs& a, const BatchMeshDev& m, uint32_t* lds,
                                   ItemSlices* src) {
-  TraceArgs t{};
-  t.nodes = m.v.B.nodes;
-  t.wide = m.v.B.wide;
-  t.tris = m.v.B.tris;
-  t.nprims = m.v.n;
-  t.rays = m.rays;
-  t.nrays = m.nrays;
-  t.gstack = a.gstack;
-  t.gdepth = a.gdepth;
-  t.err = a.ctl + BATCH_CTL_TRACE_ERR;
-  t.refill_idle = a.refill_idle;
-  t.sphere = 0;  // batch meshes are triangle scenes
+  const TraceArgs t = hot_args(m, m.nrays, a.refill_idle);
+  const MeshCold cold{src->mesh, 0u};
   int32_t* s_node = reinterpret_cast<int32_t*>(lds);
   float* s_tn = reinterpret_cast<float*>(lds + DEPTH * BUILD_BLOCK);
-  if (src->kind) {
-    t.occ = m.occ;
-    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE, false>(t, *src, s_node, s_tn);
-  } else {
-    t.prim = m.prim;
-    t.t = m.t;
-    t.u = m.u;
-    t.v = m.v_;
-    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE, false>(t, *src, s_node, s_tn);
-  }
+  if (src->kind)
+    trace_loop<true, false, BUILD_BLOCK, DEPTH, false, false, WIDE, false>(t, cold, *src, s_node,
+                                                                           s_tn);
+  else
+    trace_loop<false, false, BUILD_BLOCK, DEPTH, TSTACK, false, WIDE, false>(t, cold, *src, s_node,
+                                                                             s_tn);
 }
 
 // ---- the build phases: a launch each ----------------------------------------
@@ -324,9 +343,7 @@ k_batch_trace(BatchArgs a) {
       __syncthreads();
       if (it == NO_ITEM) return;
       const BatchWork w = load_uniform(a.items + it);
-      const BatchMeshDev m = load_uniform(a.meshes + w.mesh);
-      trace_item<DEPTH, TSTACK, WIDE>(a.gstack, a.gdepth, a.ctl + BATCH_CTL_TRACE_ERR, a.ray_tile,
-                                      a.refill_idle, m, w.tile, lds, &s_ctr, slots);
+      trace_item<DEPTH, TSTACK, WIDE>(a, w, lds, &s_ctr, slots);
     }
   }
 }

@@ -612,6 +612,7 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
   TraceArgs a{};
   a.nodes = b->B.nodes;
   a.tris = b->B.tris;
+  a.parent = b->B.parent;
   a.nprims = b->n;
   a.rays = *rays;
   a.nrays = n;

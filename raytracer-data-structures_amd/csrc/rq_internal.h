@@ -266,6 +266,7 @@ struct TraceArgs {
   const NodeRec* nodes;
   const WideNode* wide;  // wide variants only
   const TriRec* tris;
+  const int32_t* parent;  // wide variants only: BuildBuffers::parent
   uint32_t nprims;
   rq_rays rays;
   uint32_t nrays;

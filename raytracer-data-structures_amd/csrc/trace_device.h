@@ -119,6 +119,7 @@ constexpr float SLAB_SLACK = 1.000030517578125f;
 // hit with a 2^-9 relative slack keeps every box whose sphere's computed t
 // can still beat the best hit.
 constexpr float SPHERE_SLACK = 1.001953125f;
+constexpr float TRI_ERROR = 0x1p-19f;  // (tri_doubt)
 // Wide walk: a record is loaded at a byte offset node * 64 held in 32 bits (a
 // scalar base plus one vector offset) while the node count stays at or below
 // this; larger trees take 64-bit addresses.
@@ -190,15 +191,16 @@ __device__ inline void cas_hit(bool& ha, int32_t& ca, bool& hb, int32_t& cb) {
 
 // Möller–Trumbore, main.cpp:137-162 (v_0 read as v0), t restricted to
 // (tmin, tmax], tmax the ray's or the best hit so far (the caller tells a tie
-// from an end). Dot products (x*x' + y*y') + z*z', no contraction.
+// from an end). Dot products (x*x' + y*y') + z*z', no contraction. inv is
+// 1 / the determinant.
 __device__ inline bool mt(const TriRec& T, const RayState& r, float tmax, float& t, float& u,
-                          float& v) {
+                          float& v, float& inv) {
   const float px = r.dy * T.e2.z - r.dz * T.e2.y;
   const float py = r.dz * T.e2.x - r.dx * T.e2.z;
   const float pz = r.dx * T.e2.y - r.dy * T.e2.x;
   const float det = (T.e1.x * px + T.e1.y * py) + T.e1.z * pz;
   if (fabsf(det) < 1e-6f) return false;
-  const float inv = 1.0f / det;
+  inv = 1.0f / det;
   const float tx = r.ox - T.v0.x, ty = r.oy - T.v0.y, tz = r.oz - T.v0.z;
   const float uu = ((tx * px + ty * py) + tz * pz) * inv;
   if (uu < 0.0f || uu > 1.0f) return false;
@@ -233,17 +235,16 @@ __device__ inline bool sphere_hit(const TriRec& S, const RayState& r, float tmax
   return true;
 }
 
-// The primitive tests accept a few rays that miss the primitive's box: the
-// sphere test by the cancellation above, the triangle test by its rounding
-// when the triangle is small for its distance (some rays in ten thousand at
-// 10^6 times its size). The walks answer for the rays that hit the box; a wide
-// node's box on the grid is larger than the exact one, so the wide walk tests
-// the exact one where the primitive test leaves a doubt. (A tree of one primitive
-// has no node, and so no box.)
+// The primitive tests accept some rays that miss the primitive's box: the
+// sphere test by the cancellation above, the triangle test by its own rounding.
+// The answers are those for the rays that hit the box; a wide node's box on the
+// grid is larger than the exact one, so the wide walk tests the exact one where
+// the primitive test leaves a doubt. (A tree of one primitive has no node, and so
+// no box.)
 __device__ inline bool leaf_box(const float lo[3], const float hi[3], const RayState& r,
-                                float slack) {
+                                float tmax, float slack) {
   const float o[3] = {r.ox, r.oy, r.oz}, i[3] = {r.ix, r.iy, r.iz};
-  float tn = r.tmin, tf = INFINITY;
+  float tn = r.tmin, tf = tmax;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const bool s = signbit(i[k]);
@@ -252,16 +253,26 @@ __device__ inline bool leaf_box(const float lo[3], const float hi[3], const RayS
   }
   return tn <= tf * slack;
 }
-// A triangle hit at t is doubtful at 2^12 times the triangle's size (the
-// rounding of u and v, about 2^-22 of that ratio, is then a thousandth).
-__device__ inline bool tri_doubt(const TriRec& T, float t) {
+// Whether a triangle hit's rounding may have made it. With m the largest
+// component of the edges, D of the direction, and the distance from the origin to
+// the first vertex at most t D + m, u, v and 1 - u - v are within
+// K D m (t D + 2 m) / det of the exact ones, and t within that times m / D. Where
+// they lie further inside, and t is known to 2^-16, the exact line passes through
+// the triangle, and the slab test of its box accepts that (its slack is 2^-15).
+// K = 2^-19: a search for the largest errors found 12 * 2^-24 for u and v, 17 for
+// 1 - u - v and 26 for t. 2.1 M camera rays take 246 us without this and 251 with it.
+__device__ inline bool tri_doubt(const TriRec& T, const RayState& r, float t, float u, float v,
+                                 float inv) {
   const float m = fmaxf(fmaxf(fmaxf(fabsf(T.e1.x), fabsf(T.e1.y)), fmaxf(fabsf(T.e1.z), fabsf(T.e2.x))),
                         fmaxf(fabsf(T.e2.y), fabsf(T.e2.z)));
-  return t > 0x1p12f * m;
+  const float d = fmaxf(fmaxf(fabsf(r.dx), fabsf(r.dy)), fabsf(r.dz));
+  const float h = (m * TRI_ERROR) * (__builtin_fmaf(t, d, m + m) * fabsf(inv));
+  return !(fminf(fminf(u, v), 1.0f - (u + v)) > h * d && t > (h * 0x1p16f) * m);
 }
-// Its box, from the record (within a rounding of the build's, far less than
-// a doubtful hit's error).
-__device__ inline bool tri_box(const TriRec& T, const RayState& r) {
+// Its box, from the record: each plane within 2^-23 of its vertices' coordinates of
+// the build's. The rays that meet the box with its planes drawn in by more than that
+// meet the build's too; the few others are tested on the box in the leaf's parent.
+__device__ inline bool tri_box(const TriRec& T, const RayState& r, float tmax) {
   const float v[3] = {T.v0.x, T.v0.y, T.v0.z}, e[3] = {T.e1.x, T.e1.y, T.e1.z},
               f[3] = {T.e2.x, T.e2.y, T.e2.z};
   float lo[3], hi[3];
@@ -269,8 +280,23 @@ __device__ inline bool tri_box(const TriRec& T, const RayState& r) {
   for (int k = 0; k < 3; ++k) {
     lo[k] = v[k] + fminf(fminf(e[k], f[k]), 0.0f);
     hi[k] = v[k] + fmaxf(fmaxf(e[k], f[k]), 0.0f);
+    const float in = fmaxf(fabsf(lo[k]), fabsf(hi[k])) * 0x1p-21f;
+    lo[k] += in, hi[k] -= in;
   }
-  return leaf_box(lo, hi, r, SLAB_SLACK);
+  return leaf_box(lo, hi, r, tmax, SLAB_SLACK);
+}
+// The box of leaf k of n as the binary nodes hold it.
+struct LeafBoxes {
+  const int32_t* parent;  // BuildBuffers::parent
+  const NodeRec* nodes;
+};
+__device__ inline bool stored_box(const LeafBoxes& b, uint32_t n, int32_t k, const RayState& r,
+                                  float tmax, float slack) {
+  const uint32_t p = (uint32_t)b.parent[n - 1u + (uint32_t)k];
+  const float4* q = reinterpret_cast<const float4*>(b.nodes + (p >> 1)) + 2u * (p & 1u);
+  const float4 l = q[0], h = q[1];
+  const float lo[3] = {l.x, l.y, l.z}, hi[3] = {h.x, h.y, h.z};
+  return leaf_box(lo, hi, r, tmax, slack);
 }
 // A sphere leaf's box, as the build gives it (leaf_record).
 __device__ inline bool sphere_box(const TriRec& S, const RayState& r) {
@@ -278,7 +304,7 @@ __device__ inline bool sphere_box(const TriRec& S, const RayState& r) {
   float lo[3], hi[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) lo[k] = (c[k] - S.e1.x) + 0.0f, hi[k] = (c[k] + S.e1.x) + 0.0f;
-  return leaf_box(lo, hi, r, SPHERE_SLACK);
+  return leaf_box(lo, hi, r, INFINITY, SPHERE_SLACK);
 }
 
 // The wide records as a raw buffer resource (scalar registers): loads at a
@@ -365,6 +391,7 @@ __device__ inline unsigned long long hit_key(float t, int32_t prim) {
 // query kernels read them again from the kernel's argument memory each time:
 // as hoisted scalars they crowded out the walk's own (33 of them spilled to
 // vector lanes, which held two registers and cost reads in the loop).
+// cold.leaf_boxes() hands out the leaves' exact boxes, for the few doubtful hits.
 constexpr int ROWS_SMALL = 0, ROWS_BIG = 1, ROWS_ANY = 2;
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
           int ROWS, bool SHARE, class Src, class Cold>
@@ -396,7 +423,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
   const Slots ss = (Slots)slots;
 
   auto write_hit = [&](uint32_t of, bool hit, int32_t prim, float t, float u, float v) {
-    const auto* c = cold();
+    const auto c = cold();
     const uint32_t oi = c->out_index ? c->out_index[of] : of;
     if (ANY) {
       c->occ[oi] = hit ? 1 : 0;
@@ -460,6 +487,13 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
     return false;
   };
 
+  // A doubtful hit on triangle T, the leaf `node`: whether the ray meets its box up
+  // to the ray's own end.
+  auto exact_hit = [&](const TriRec& T) -> bool {
+    const float tmax = cold()->rays.tmax[ray];
+    return tri_box(T, r, tmax) || stored_box(cold.leaf_boxes(), a.nprims, ~node, r, tmax, slack);
+  };
+
   for (;;) {
     if (SPLIT && nslots != 0u && __ballot(active) == 0ull) {
       const int lane = lane_now();
@@ -482,7 +516,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
       const uint32_t rank = rank_in(m);
       if (!active && rank < take) {
         const uint32_t rr = cnext + rank;
-        const auto* c = cold();
+        const auto c = cold();
         ray = rr;
         r.ox = c->rays.ox[rr], r.oy = c->rays.oy[rr], r.oz = c->rays.oz[rr];
         r.dx = c->rays.dx[rr], r.dy = c->rays.dy[rr], r.dz = c->rays.dz[rr];
@@ -678,8 +712,10 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
           if (SPHERES && a.sphere) {
             hit = sphere_hit(T, r, bt, t) && (!WIDE || a.nprims < 2u || sphere_box(T, r));
           } else {
-            hit = mt(T, r, bt, t, u, v);
-            if (WIDE && hit && tri_doubt(T, t)) hit = a.nprims < 2u || tri_box(T, r);
+            float inv;
+            hit = mt(T, r, bt, t, u, v, inv);
+            if (WIDE && hit && tri_doubt(T, r, t, u, v, inv) && a.nprims > 1u)
+              hit = exact_hit(T);
           }
           if (hit) {
             const int32_t prim = __float_as_int(T.v0.w);
@@ -752,11 +788,11 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
 // (a burst of 16 requests 1515 -> 1380 us with its copies); a batch run's waves
 // refill from item to item, and the code's presence costs them 3 %.
 template <bool ANY, bool COUNT, int BLOCK, int DEPTH, bool TSTACK, bool SPHERES, bool WIDE,
-          bool SHARE, class Src>
-__device__ inline void trace_loop(const TraceArgs& a, Src& src, int32_t* s_node, float* s_tn,
-                                  SplitSlots* slots = nullptr) {
+          bool SHARE, class Src, class Cold>
+__device__ inline void trace_loop(const TraceArgs& a, const Cold& cold, Src& src, int32_t* s_node,
+                                  float* s_tn, SplitSlots* slots = nullptr) {
   trace_loop_impl<ANY, COUNT, BLOCK, DEPTH, TSTACK, SPHERES, WIDE, ROWS_ANY, SHARE>(
-      a, [&] { return &a; }, src, s_node, s_tn, slots);
+      a, cold, src, s_node, s_tn, slots);
 }
 // A path per record addressing, chosen once per launch (the query kernels:
 // one tree).

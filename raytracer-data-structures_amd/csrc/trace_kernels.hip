@@ -24,6 +24,10 @@ struct KernelArgs {
     asm volatile("" : "+s"(p));
     return p;
   }
+  __device__ LeafBoxes leaf_boxes() const {
+    const ArgsPtr p = (*this)();
+    return LeafBoxes{p->parent, p->nodes};
+  }
 };
 
 // WAVES > 0: registers capped so that this many waves fit a SIMD.
