@@ -133,7 +133,10 @@ int rq_bvh_export(rq_ctx* ctx, const rq_bvh* b, uint32_t* codes, uint32_t* sorte
 /* Download the 4-wide nodes (see rq_trace_variant): for binary internal node
  * i, boxes[i*24 + slot*6 + (lo xyz, hi xyz)] and links[i*4 + slot] (>= 0 wide
  * node, < 0 leaf ~k, 0 unused slot). Every internal node has one; the wide
- * walk reaches the root and the nodes at even depth.
+ * walk reaches the root and the nodes at even depth. The device keeps the boxes
+ * on a byte grid of each node's; the boxes written here are the exact ones, and
+ * RQ_E_DEVICE says that a device box does not hold its exact one, or is more than
+ * two steps of the finest grid larger.
  * RQ_E_UNSUPPORTED for a BVH without wide nodes. */
 int rq_bvh_export_wide(rq_ctx* ctx, const rq_bvh* b, float* boxes, int32_t* links);
 

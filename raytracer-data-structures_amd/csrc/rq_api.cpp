@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "rq_ctx.h"
+#include "wide_check.h"
 
 namespace rq {
 
@@ -541,8 +542,8 @@ int rq_bvh_export_wide(rq_ctx* c, const rq_bvh* b, float* boxes, int32_t* links)
   if (e == hipSuccess) e = hipMemcpy(nodes.data(), b->B.nodes, ni * sizeof(NodeRec), hipMemcpyDeviceToHost);
   if (e != hipSuccess) return hip_err(c, e, "wide export");
   // The records hold the links and the boxes on a grid; the boxes handed out
-  // are the exact ones they stand for (the binary records'), once each
-  // record's box is found to contain its own.
+  // are the exact ones they stand for (the binary records'), once each record's
+  // boxes are found to hold them closely.
   const float inf = std::numeric_limits<float>::infinity();
   for (size_t i = 0; i < ni; ++i) {
     float ex[4][6];
@@ -572,18 +573,18 @@ int rq_bvh_export_wide(rq_ctx* c, const rq_bvh* b, float* boxes, int32_t* links)
     }
     const WideNode& q = w[i];
     const int32_t got[4] = {q.link.x, q.link.y, q.link.z, q.link.w};
-    const double base[3] = {q.base.x, q.base.y, q.base.z}, step[3] = {q.base.w, q.step_y, q.step_z};
-    const uint32_t ql[3] = {q.lox, q.loy, q.loz}, qh[3] = {q.hix, q.hiy, q.hiz};
     for (int s = 0; s < 4; ++s) {
       if (got[s] != want[s])
-        return set_err(c, RQ_E_HIP, "wide node %zu slot %d: link %d, not %d", i, s, got[s], want[s]);
-      for (int x = 0; x < 3 && want[s]; ++x) {
-        const double l = base[x] + (WIDE_Q0 + (ql[x] >> (8 * s) & 255u)) * step[x];
-        const double h = base[x] + (WIDE_Q0 + (qh[x] >> (8 * s) & 255u)) * step[x];
-        if (l > ex[s][x] || h < ex[s][3 + x])  // (a NaN step is a box everywhere)
-          return set_err(c, RQ_E_HIP, "wide node %zu slot %d: its box does not hold the exact one", i, s);
-      }
+        return set_err(c, RQ_E_DEVICE, "wide node %zu slot %d: link %d, not %d", i, s, got[s], want[s]);
       if (boxes) std::memcpy(boxes + 24 * i + 6 * s, ex[s], sizeof ex[s]);
+    }
+    const float base[3] = {q.base.x, q.base.y, q.base.z}, step[3] = {q.base.w, q.step_y, q.step_z};
+    const uint32_t ql[3] = {q.lox, q.loy, q.loz}, qh[3] = {q.hix, q.hiy, q.hiz};
+    for (int x = 0; x < 3; ++x) {
+      const float lo[4] = {ex[0][x], ex[1][x], ex[2][x], ex[3][x]};
+      const float hi[4] = {ex[0][3 + x], ex[1][3 + x], ex[2][3 + x], ex[3][3 + x]};
+      const char* fault = wide_axis_fault(lo, hi, want, base[x], step[x], ql[x], qh[x]);
+      if (fault) return set_err(c, RQ_E_DEVICE, "wide node %zu axis %d: %s", i, x, fault);
     }
     if (links) std::memcpy(links + 4 * i, got, sizeof got);
   }
