@@ -165,6 +165,7 @@ BatchArgs batch_args(const rq_batch* b) {
   int depth, ts;
   batch_variant_info(b->variant, &depth, &ts);
   a.gdepth = TRACE_MAX_STACK_WIDE - depth;  // the batch run walks the 4-wide nodes
+  a.gwords = stack_words(ts);
   a.ray_tile = b->ray_tile;
   a.refill_idle = b->refill;
   return a;
@@ -264,10 +265,10 @@ int rq_batch_create(rq_ctx* c, const rq_batch_item* items, uint32_t count, int m
       b->grid.push_back(batch_trace_grid_blocks(c->device, v));
       int depth, ts;
       batch_variant_info(v, &depth, &ts);
-      gmax = std::max(gmax,
-                      (size_t)b->grid.back() * BUILD_BLOCK * (TRACE_MAX_STACK_WIDE - depth));
+      gmax = std::max(gmax, (size_t)b->grid.back() * BUILD_BLOCK * (TRACE_MAX_STACK_WIDE - depth) *
+                                stack_words(ts));
     }
-    rc = balloc(c, b, gmax * 2 * sizeof(int32_t), (void**)&b->gstack);
+    rc = balloc(c, b, gmax * sizeof(int32_t), (void**)&b->gstack);
   }
   if (!rc) rc = make_work(c, b, b->ray_tile);
   if (!rc) {

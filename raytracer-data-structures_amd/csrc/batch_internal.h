@@ -67,7 +67,7 @@ struct BatchArgs {
   uint32_t trace_seg[BATCH_XCDS + 1];   // trace items of XCD q: [trace_seg[q], trace_seg[q + 1])
   uint32_t* ctl;                        // BATCH_CTL_WORDS
   int32_t* gstack;                      // traversal stack overflow of the persistent grid
-  uint32_t gdepth;
+  uint32_t gdepth, gwords;              // its entries per thread, and their words
   uint32_t ray_tile;
   uint32_t refill_idle;
 };

@@ -79,6 +79,7 @@ struct MeshCold {
     c.occ = m->occ + r0;
     c.gstack = p->gstack;
     c.gdepth = p->gdepth;
+    c.gwords = p->gwords;
     c.err = p->ctl + BATCH_CTL_TRACE_ERR;
     return c;
   }

@@ -229,7 +229,7 @@ int rq_create(rq_ctx** out, int device, size_t budget) {
     int blk, depth, ts;
     trace_variant_info(v, &blk, &depth, &ts);
     gmax = std::max(gmax, (size_t)std::max(c->trace_grid[v], c->trace_grid_any[v]) * blk *
-                              (trace_max_stack(v) - depth));
+                              (trace_max_stack(v) - depth) * stack_words(ts));
   }
   // counter slots (eager, then capture) + one trailing word of traversal error bits
   const size_t cwords = (size_t)(COUNTER_SLOTS + CAPTURE_SLOTS) * SLOT_WORDS;
@@ -238,7 +238,7 @@ int rq_create(rq_ctx** out, int device, size_t budget) {
   if (rc == RQ_OK) {
     c->errword = reinterpret_cast<uint32_t*>(c->counters + cwords);
     hipMemset(c->counters, 0, cbytes);
-    c->gstack_bytes = gmax * 2 * sizeof(int32_t);
+    c->gstack_bytes = gmax * sizeof(int32_t);
     rc = ctx_alloc(c, c->gstack_bytes, (void**)&c->gstack);
   }
   if (rc == RQ_OK) {
@@ -641,8 +641,9 @@ static int query(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t n, rq
   // a counter slot whose start is not tracked here: zeroed in the stream first
   const bool own_zero = captured || count_dev != nullptr;
   a.gdepth = (uint32_t)(trace_max_stack(variant) - depth);
+  a.gwords = stack_words(ts);
   if (noalloc) {
-    const size_t per_block = (size_t)blk * a.gdepth * 2 * sizeof(int32_t);
+    const size_t per_block = (size_t)blk * a.gdepth * a.gwords * sizeof(int32_t);
     const size_t blocks = (NOALLOC_SCRATCH_BYTES - NOALLOC_COUNTER_BYTES) / per_block;
     if (blocks == 0) return set_err(c, RQ_E_UNSUPPORTED, "variant too large for the scratch");
     a.gstack = reinterpret_cast<int32_t*>(c->scratch + NOALLOC_COUNTER_BYTES);

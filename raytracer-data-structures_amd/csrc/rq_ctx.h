@@ -31,7 +31,7 @@ struct rq_ctx {
   uint32_t* errword = nullptr;   // traversal error bits (stack deeper than provided)
   uint32_t counter_seq = 0;
   uint32_t capture_seq = 0;      // next capture slot (after the COUNTER_SLOTS eager ones)
-  // Traversal stack overflow ({node, distance} pairs), indexed by global
+  // Traversal stack overflow (entries of stack_words words), indexed by global
   // thread id: launches that may run at once need separate areas, so each
   // stream gets its own (the default stream's is allocated with the context).
   int32_t* gstack = nullptr;

@@ -87,7 +87,7 @@ constexpr uint32_t MAX_PRIMS = (1u << 30) - 1;
 // Traversal: the LBVH of 30-bit codes is at most 63 levels deep (prefix
 // lengths 2..63 along a path), so 64 stack entries per lane always suffice;
 // kernel variants keep 12..32 of them in LDS and the rest in a global
-// overflow area ([depth][thread] pairs of {node, entry distance}).
+// overflow area ([depth][thread] entries of stack_words words).
 constexpr int TRACE_MAX_STACK = 64;
 // Wide traversal keeps up to 3 entries per wide ancestor, and a path of at
 // most 64 binary levels has at most 32 wide ones.
@@ -277,6 +277,7 @@ struct TraceArgs {
   uint32_t* tests;
   int32_t* gstack;
   uint32_t gdepth;      // overflow entries per thread
+  uint32_t gwords;      // words of an entry (stack_words of the variant)
   // ray-stream counters of this launch's slot (one per segment, never reset)
   // and their values when this launch starts
   unsigned long long* counter;
@@ -303,6 +304,10 @@ int trace_num_variants();
 void trace_variant_info(int v, int* block, int* depth, int* tstack, int* wide = nullptr,
                         int* closest_waves = nullptr, int* any_waves = nullptr);
 int trace_max_stack(int variant);  // total stack entries per lane (LDS + overflow)
+// 32-bit words of a stack entry in the overflow area: the node, and its entry
+// distance where a variant's entries carry one. (With two words for all, eight waves
+// per SIMD made the area 336 MB a stream; so it is 236.)
+constexpr uint32_t stack_words(bool tstack) { return tstack ? 2u : 1u; }
 uint32_t trace_grid_blocks(int device, int variant, bool any);
 hipError_t launch_copy16(const LaunchCtx& lc, const void* src, void* dst, uint64_t bytes);
 // Zeroes a slot's ray-stream counters with a kernel (a memset node would not

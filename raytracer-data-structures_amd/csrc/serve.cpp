@@ -177,7 +177,7 @@ struct rq_server {
   size_t max_items = 0;
   uint32_t* ctl = nullptr;
   int32_t* gstack = nullptr;
-  uint32_t gdepth = 0, grid = 0;
+  uint32_t gdepth = 0, gwords = 0, grid = 0;
   // trace kernel of the steps (serve_variant_info): the 4-wide walk, LDS
   // stack depth 16, 8 waves per SIMD (at 6, against the binary walk, serving 64
   // meshes of 10k-2M triangles at 2000 requests/s: p50 1.40 -> 1.15 ms,
@@ -467,6 +467,7 @@ bool launch_step(rq_server* s) {
   a.ctl = s->ctl;
   a.gstack = s->gstack;
   a.gdepth = s->gdepth;
+  a.gwords = s->gwords;
   a.ray_tile = tile;
   a.refill_idle = 16;
   hipError_t e = hipMemcpyAsync(s->dev_meshes[buf], md, ne * sizeof(BatchMeshDev),
@@ -785,7 +786,8 @@ int rq_server_create(int device, const rq_server_config* cfg_in, rq_server** out
     serve_variant_info(s->variant, &depth, &ts, &wide);
     s->grid = serve_grid_blocks(device, s->variant);
     s->gdepth = (wide ? TRACE_MAX_STACK_WIDE : TRACE_MAX_STACK) - depth;
-    rc = ctx_alloc(c, (size_t)s->grid * BUILD_BLOCK * s->gdepth * 2 * sizeof(int32_t),
+    s->gwords = stack_words(ts);
+    rc = ctx_alloc(c, (size_t)s->grid * BUILD_BLOCK * s->gdepth * s->gwords * sizeof(int32_t),
                    (void**)&s->gstack);
   }
   for (hipStream_t* st : {&s->s_prep, &s->s_trace, &s->s_out})

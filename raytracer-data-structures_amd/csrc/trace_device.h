@@ -450,7 +450,9 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
   };
   // Entry `at` (DEPTH or deeper) of thread t's stack in the overflow area.
   auto spilled = [&](int at, int t) -> int32_t* {
-    return cold()->gstack + 2 * ((size_t)(at - DEPTH) * (gridDim.x * BLOCK) + blockIdx.x * BLOCK + t);
+    const auto c = cold();
+    return c->gstack +
+           c->gwords * ((size_t)(at - DEPTH) * (gridDim.x * BLOCK) + blockIdx.x * BLOCK + t);
   };
   auto push = [&](int32_t c, float tn) {
     if (sp < DEPTH) {

@@ -47,7 +47,7 @@ void k_trace(TraceArgs a) {
 // Device scratch of the allocation-free closest-hit entry
 // (rq_closest_hit_noalloc): the launch's ray-stream counters in the first
 // NOALLOC_COUNTER_BYTES, then the traversal stack overflow area
-// ([depth][thread] pairs). One copy per device, held from module load until
+// ([depth][thread] entries). One copy per device, held from module load until
 // the process ends; its address comes from hipGetSymbolAddress
 // (noalloc_scratch_address), never from the array's name in host code. Calls
 // that overlap on one device share it and race.
