@@ -38,10 +38,9 @@ struct rq_renderer {
   float2* lit1 = nullptr;  // per sample: a diffuse second hit's L.N and Phong term
   float* srgb = nullptr;
   float* img = nullptr;
-  // the image as it is read: a small one whole in pinned memory (values, then
-  // PPM bytes), else the bytes on the device; both null where there was no room
+  // a small image as it is read, in pinned memory (values, then PPM bytes); null
+  // where there was no room
   float* stage = nullptr;
-  uint8_t* ppm = nullptr;
   double* jit = nullptr;
   uint32_t* counters = nullptr;
   // the primary hits' shadow rays are traced on `side` while the bounce rays
@@ -226,7 +225,6 @@ int rq_renderer_create(rq_ctx* c, const rq_render_params* p, rq_renderer** out) 
     r->stage = nullptr;
     (void)hipGetLastError();
   }
-  if (!r->stage) (void)ralloc(c, r, round4(count), (void**)&r->ppm);
   *out = r;
   return RQ_OK;
 }
@@ -364,20 +362,12 @@ int rq_render_read_image(rq_ctx* c, rq_renderer* r, float* rgb, uint8_t* ppm) {
     if (e == hipSuccess && ppm) std::memcpy(ppm, b, count);
     return e == hipSuccess ? RQ_OK : hip_err(c, e, "image read");
   }
-  if (ppm && r->ppm) e = launch_image_out(lc, r->img, count, r->p.spp, nullptr, r->ppm);
+  // (the bytes are made in t0, 4 bytes a sample, which only a frame's own kernels read:
+  // no memory of the budget for them)
+  uint8_t* const b = reinterpret_cast<uint8_t*>(r->t0);
+  if (ppm) e = launch_image_out(lc, r->img, count, r->p.spp, nullptr, b);
   if (e == hipSuccess && rgb) e = hipMemcpy(rgb, r->img, count * 4, hipMemcpyDeviceToHost);
-  if (e == hipSuccess && ppm && r->ppm) {
-    e = hipMemcpy(ppm, r->ppm, count, hipMemcpyDeviceToHost);
-  } else if (e == hipSuccess && ppm) {  // no room for them on the device
-    std::vector<float> img;
-    if (!rgb) {
-      img.resize(count);
-      e = hipMemcpy(img.data(), r->img, count * 4, hipMemcpyDeviceToHost);
-    }
-    const float* f = rgb ? rgb : img.data();
-    for (size_t k = 0; e == hipSuccess && k < count; ++k)
-      ppm[k] = (uint8_t)(std::min(float(1), f[k] / r->p.spp) * 255);
-  }
+  if (e == hipSuccess && ppm) e = hipMemcpy(ppm, b, count, hipMemcpyDeviceToHost);
   return e == hipSuccess ? RQ_OK : hip_err(c, e, "image read");
 }
 
