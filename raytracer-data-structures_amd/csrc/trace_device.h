@@ -411,7 +411,8 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
   bool wave_out = false;         // there are no more slices for this wave
   uint32_t ray = 0;
   int32_t node = 0, best = -1;
-  int sp = 0;
+  int sp = 0;  // stack entries; PENDING: the lane's result is not written yet
+  constexpr int PENDING = -1;
   float bt = 0.0f, bu = 0.0f, bv = 0.0f;
   uint32_t vis = 0, tst = 0;
 
@@ -438,15 +439,26 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
       c->tests[oi] = tst;
     }
   };
-  // The lane's ray, or its part of a split ray, is walked to the end.
+  // The lane's ray, or its part of a split ray, is walked to the end. The result
+  // stays in the lane until the lane is needed again: written where each ray ended, it
+  // took a wave a read of the output pointers and stores of its own for each length of
+  // ray (300 k camera rays over 80 triangles 24.1 -> 22.7 us closest and 24.5 -> 23.3 any
+  // hit, 2.1 M over 1.3 M 252 -> 244, 16.8 M uniform ones over 5.2 M 1446 -> 1360). The
+  // stack's height marks it: as a lane mask it made scalars spill, and all was lost.
   auto finish = [&](auto split) {
     if (!decltype(split)::value) {
-      write_hit(ray, best >= 0, best, bt, bu, bv);
+      sp = PENDING;
     } else {
-      if (own < 0) write_hit(ray, best >= 0, best, bt, bu, bv);
+      sp = own < 0 ? PENDING : 0;
       own = -1;
     }
     active = false;
+  };
+  auto flush = [&] {
+    if (sp == PENDING) {
+      write_hit(ray, best >= 0, best, bt, bu, bv);
+      sp = 0;
+    }
   };
   // Entry `at` (DEPTH or deeper) of thread t's stack in the overflow area.
   auto spilled = [&](int at, int t) -> int32_t* {
@@ -497,6 +509,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
   };
 
   for (;;) {
+    flush();
     if (SPLIT && nslots != 0u && __ballot(active) == 0ull) {
       const int lane = lane_now();
       if (lane < (int)nslots) {
@@ -527,8 +540,8 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
         r.sx = signbit(r.ix), r.sy = signbit(r.iy), r.sz = signbit(r.iz);
         best = -1, bu = 0.0f, bv = 0.0f, vis = 0, tst = 0, sp = 0;
         node = a.nprims == 1 ? ~0 : 0;
-        active = true;
-        if (!(r.tmin < bt) || a.nprims == 0) finish(std::false_type{});
+        active = r.tmin < bt && a.nprims != 0;
+        if (!active) write_hit(rr, false, -1, 0.0f, 0.0f, 0.0f);
       }
       cnext += take;
       m = __ballot(!active);
@@ -566,6 +579,7 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
       const int from = __builtin_amdgcn_ds_bpermute((int)(rank - k * givers) * 4, table);
       const int gsp = __shfl(sp, from, 64);
       const bool help = !active && (int)k < gsp;
+      flush();
       auto take = [&](auto& x) {
         const auto y = __shfl(x, from, 64);
         if (help) x = y;
