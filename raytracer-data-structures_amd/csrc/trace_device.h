@@ -345,6 +345,12 @@ constexpr uint32_t SPLIT_IDLE = 48;
 // 27.8 us at 0, 26.4 at 20 or 32; in a soup of 22 k, where helpers pay, 26 / 30 /
 // 33, and 34 without them).
 constexpr uint32_t SINGLE_ALONE = 20;
+// Full waves (64 rays a slice) over fewer primitives than this walk without help: few
+// of their rays are long enough to pay for the helpers' code (300 k camera rays with and
+// without, any hit and closest, us: 80 triangles 23.2 / 21.2 and 22.7 / 22.7, 320 29.3 /
+// 30.0 and 31.1 / 30.5, 1 M of them 50.3 / 49.1 and 51.9 / 51.8, soup of 300 16.1 / 15.7
+// and 16.7 / 16.4; past it, soup of 4000 54.0 / 54.7, a sphere of 5120 61.6 / 65.9).
+constexpr uint32_t SHARE_MIN_PRIMS = 512;
 constexpr uint32_t SPLIT_SLOTS = 16;  // split rays of a wave at a time
 struct SplitSlots {
   unsigned long long key[SPLIT_SLOTS];  // ~0: no hit; any hit: 0 once there is one
@@ -420,7 +426,10 @@ __device__ inline void trace_loop_impl(const TraceArgs& a, const Cold& cold, Src
   // where lanes share), slots used
   int own;
   uint32_t nslots = 0;
-  uint32_t alone = SPLIT && a.nrays == 1u ? SINGLE_ALONE : 0u;
+  // steps that the wave makes without help when it could have some
+  uint32_t alone = 0u;
+  if (SPLIT && a.nrays == 1u) alone = SINGLE_ALONE;
+  if (SPLIT && a.nprims < SHARE_MIN_PRIMS && a.chunk >= 64u) alone = ~0u;
   const Slots ss = (Slots)slots;
 
   auto write_hit = [&](uint32_t of, bool hit, int32_t prim, float t, float u, float v) {
