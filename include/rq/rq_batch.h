@@ -84,9 +84,10 @@ int rq_batch_phase_ms(rq_ctx* ctx, rq_batch* b, double* ms, int cap);
 /* Synchronises and reports the error bits of the last run: 2 = a ray needed a
  * deeper stack than provided, 4 = a mesh build reported an error. */
 int rq_batch_errors(rq_ctx* ctx, rq_batch* b, uint32_t* bits);
-/* Synchronises and reports the blocks of the build's sort kernels that the
- * device holds at a time (grid), and as members the same once the batch has
- * run: every run takes its whole grid, however busy the device. */
+/* Synchronises and reports the trace blocks of the last run: its launch grid,
+ * and as members those that started, counted on the device (0 before a run).
+ * They are equal however busy the device is: blocks that are placed late find
+ * the items that are left. */
 int rq_batch_occupancy(rq_ctx* ctx, rq_batch* b, uint32_t* members, uint32_t* grid);
 
 #ifdef __cplusplus

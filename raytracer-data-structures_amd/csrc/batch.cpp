@@ -30,8 +30,7 @@ struct rq_batch {
   int32_t* gstack = nullptr;
   uint32_t gdepth = 0;
   int build = 3;                       // sort kernels: 5 waves per SIMD (batch_build_waves)
-  std::vector<uint32_t> build_grid;    // their blocks on the device at a time
-  bool ran = false;
+  uint32_t run_grid = 0;               // trace blocks of the last run (0: none yet)
   std::vector<uint32_t> grid;          // the trace kernel's, per configuration
   // the autotuned choice on 512 mixed meshes (1k-500k triangles, incoherent
   // rays): trace configuration 1 (LDS depth 16), 512-ray items, refill at 16
@@ -171,6 +170,13 @@ BatchArgs batch_args(const rq_batch* b) {
   return a;
 }
 
+// Trace blocks of a run: no more than there are items for their waves.
+uint32_t trace_grid(const rq_batch* b) {
+  const uint32_t items = b->trace_seg[BATCH_XCDS] - b->trace_seg[0];
+  return std::min(b->grid[b->variant],
+                  std::max(1u, tiles_of(items, BATCH_XCDS * BUILD_BLOCK / 64)) * BATCH_XCDS);
+}
+
 int launch(rq_ctx* c, rq_batch* b, hipStream_t s, bool profile) {
   if (b->built_ray_tile != b->ray_tile) {
     int rc = make_work(c, b, b->ray_tile);
@@ -178,12 +184,9 @@ int launch(rq_ctx* c, rq_batch* b, hipStream_t s, bool profile) {
   }
   LaunchCtx lc = launch_ctx(c, s);
   if (!profile) lc.prof = nullptr;
-  // no more trace blocks than there are items for their waves
-  const uint32_t items = b->trace_seg[BATCH_XCDS] - b->trace_seg[0];
-  const uint32_t grid = std::min(b->grid[b->variant],
-                                 std::max(1u, tiles_of(items, BATCH_XCDS * BUILD_BLOCK / 64)) * BATCH_XCDS);
+  const uint32_t grid = trace_grid(b);
   hipError_t e = launch_batch(lc, batch_args(b), b->build, b->variant, grid);
-  b->ran = b->ran || e == hipSuccess;
+  if (e == hipSuccess) b->run_grid = grid;
   return e == hipSuccess ? RQ_OK : hip_err(c, e, "batch launch");
 }
 
@@ -259,8 +262,6 @@ int rq_batch_create(rq_ctx* c, const rq_batch_item* items, uint32_t count, int m
   }
   if (!rc) {
     size_t gmax = 0;
-    for (int k = 0; k < batch_num_build_variants(); ++k)
-      b->build_grid.push_back(batch_build_grid_blocks(c->device, k));
     for (int v = 0; v < batch_num_variants(); ++v) {
       b->grid.push_back(batch_trace_grid_blocks(c->device, v));
       int depth, ts;
@@ -487,10 +488,17 @@ int rq_batch_get_build_waves(rq_ctx* c, const rq_batch* b, int* waves) {
 
 int rq_batch_occupancy(rq_ctx* c, rq_batch* b, uint32_t* members, uint32_t* grid) {
   if (!c || !b || !members || !grid) return RQ_E_INVALID;
-  const hipError_t e = hipDeviceSynchronize();
+  hipError_t e = hipDeviceSynchronize();
+  uint32_t n = 0;
+  for (int q = 0; q < BATCH_XCDS && e == hipSuccess; ++q) {
+    uint32_t k = 0;
+    e = hipMemcpy(&k, b->ctl + BATCH_XTICKET_BASE + q * BATCH_XTICKET_STRIDE + BATCH_XBLOCKS,
+                  sizeof k, hipMemcpyDeviceToHost);
+    n += k;
+  }
   if (e != hipSuccess) return hip_err(c, e, "batch occupancy");
-  *grid = b->build_grid[b->build];
-  *members = b->ran ? *grid : 0u;  // no launch depends on which blocks are placed
+  *grid = b->run_grid ? b->run_grid : trace_grid(b);
+  *members = n;
   return RQ_OK;
 }
 

@@ -39,6 +39,8 @@ constexpr int BATCH_XTICKET_STRIDE = 1024;  // words
 constexpr int BATCH_XTICKET_BASE = BATCH_XTICKET_STRIDE;
 constexpr int BATCH_CTL_ALLOC_WORDS = BATCH_XTICKET_BASE + BATCH_XCDS * BATCH_XTICKET_STRIDE;
 static_assert(BATCH_CTL_WORDS <= BATCH_XTICKET_BASE, "control words before the tickets");
+// A segment's page also counts the trace blocks that started on it, on another line.
+constexpr int BATCH_XBLOCKS = 64;
 constexpr uint32_t BATCH_ANY_BIT = 0x80000000u;            // trace item tile: any-hit query
 // Work items of the refit phases (see batch_kernels.hip): BATCH_REFIT_CHUNKS
 // times BUILD_BLOCK leaves an item of the first; spanning nodes in tiles of
@@ -78,7 +80,6 @@ void batch_variant_info(int v, int* depth, int* tstack);
 // The build's sort kernels by waves per SIMD (8, 7, 6, 5, 4).
 int batch_num_build_variants();
 int batch_build_waves(int build);
-uint32_t batch_build_grid_blocks(int device, int build);
 uint32_t batch_trace_grid_blocks(int device, int v);
 // The serving loop's trace kernels (binary walk over its slots).
 int serve_num_variants();

@@ -237,7 +237,10 @@ __device__ inline void stamp_end(const BatchArgs& a, int ph) {
 __device__ inline void reset_ctl(uint32_t* ctl) {
   static_assert(BATCH_CTL_WORDS <= 64, "one wave clears the control words");
   if (threadIdx.x < BATCH_CTL_WORDS) ctl[threadIdx.x] = 0u;
-  if (threadIdx.x < BATCH_XCDS) ctl[BATCH_XTICKET_BASE + threadIdx.x * BATCH_XTICKET_STRIDE] = 0u;
+  if (threadIdx.x < BATCH_XCDS) {
+    uint32_t* x = ctl + BATCH_XTICKET_BASE + threadIdx.x * BATCH_XTICKET_STRIDE;
+    x[0] = x[BATCH_XBLOCKS] = 0u;
+  }
 }
 __global__ void k_batch_reset(uint32_t* ctl) { reset_ctl(ctl); }
 
@@ -321,6 +324,9 @@ __global__ __launch_bounds__(BUILD_BLOCK) __attribute__((amdgpu_waves_per_eu(WAV
 k_batch_trace(BatchArgs a) {
   __shared__ uint32_t lds[DEPTH * BUILD_BLOCK * (TSTACK ? 2 : 1)];
   __shared__ uint32_t s_item, s_ctr;
+  if (threadIdx.x == 0)
+    atomicAdd(a.ctl + BATCH_XTICKET_BASE + blockIdx.x % BATCH_XCDS * BATCH_XTICKET_STRIDE +
+                  BATCH_XBLOCKS, 1u);
   if constexpr (WAVE_ITEMS) {
     ItemSlices src{a, SegItems(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), 0u, 0u, 0u,
                    BatchWork{}, false, false};
@@ -406,7 +412,6 @@ void serve_variant_info(int v, int* depth, int* tstack, int* wide) {
 }
 int batch_num_build_variants() { return kNumBuildVariants; }
 int batch_build_waves(int b) { return kBuildWaves[b]; }
-uint32_t batch_build_grid_blocks(int device, int b) { return grid_blocks(device, kSort[b][0]); }
 uint32_t batch_trace_grid_blocks(int device, int v) {
   return grid_blocks(device, kBatchVariants[v].fn);
 }

@@ -934,7 +934,7 @@ class Batch:
         return w.value
 
     def occupancy(self) -> tuple[int, int]:
-        """rq_batch_occupancy: (members, grid), the same once the batch has run."""
+        """rq_batch_occupancy: (trace blocks that started in the last run, its grid)."""
         m, g = C.c_uint32(), C.c_uint32()
         self.ctx._check(lib().rq_batch_occupancy(self.ctx.h, self.h, C.byref(m), C.byref(g)))
         return m.value, g.value
