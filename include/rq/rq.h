@@ -259,7 +259,8 @@ int rq_trace_refill_get(rq_ctx* ctx, uint32_t* closest_refill, uint32_t* any_ref
  * atomics, smaller ones keep the rays in flight closer together. */
 int rq_trace_slice_set(rq_ctx* ctx, uint32_t closest_slice, uint32_t any_slice);
 int rq_trace_slice_get(rq_ctx* ctx, uint32_t* closest_slice, uint32_t* any_slice);
-/* Times every variant (and refill threshold 16/48/56/64 idle lanes) on the given
+/* Times every variant (of those that run the same kernel, as 14 and 17 do, the
+ * first) at every refill threshold (16/48/56/64 idle lanes) on the given
  * device rays (default stream, `repeats` launches each after one warm-up), then
  * slice sizes 256/512/2048 against the default 1024 for the best of them, keeps
  * the fastest for that query kind (variant, refill, slice) in the context and

@@ -842,6 +842,7 @@ int rq_autotune_trace(rq_ctx* c, const rq_bvh* b, const rq_rays* rays, uint32_t 
     trace_variant_info(v, &blk, &depth, &ts, &wide);
     if (any && ts) continue;  // entry distances only help closest hit
     if (wide && !b->B.wide) continue;
+    if (trace_first_variant(v, any) != v) continue;  // timed already
     for (uint32_t rf : refills) {
       c->closest_variant = v, c->any_variant = v, c->refill_closest = c->refill_any = rf;
       c->slice_closest = c->slice_any = bs;

@@ -304,6 +304,9 @@ int trace_num_variants();
 void trace_variant_info(int v, int* block, int* depth, int* tstack, int* wide = nullptr,
                         int* closest_waves = nullptr, int* any_waves = nullptr);
 int trace_max_stack(int variant);  // total stack entries per lane (LDS + overflow)
+// The first variant that runs the same kernel for that kind of query (of those whose
+// entries carry distances, and of the others).
+int trace_first_variant(int variant, bool any);
 // 32-bit words of a stack entry in the overflow area: the node, and its entry
 // distance where a variant's entries carry one. (With two words for all, eight waves
 // per SIMD made the area 336 MB a stream; so it is 236.)

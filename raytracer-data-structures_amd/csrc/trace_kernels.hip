@@ -127,6 +127,14 @@ void trace_variant_info(int v, int* block, int* depth, int* tstack, int* wide,
 
 int trace_max_stack(int v) { return kVariants[v].wide ? TRACE_MAX_STACK_WIDE : TRACE_MAX_STACK; }
 
+int trace_first_variant(int v, bool any) {
+  for (int f = 0; f < v; ++f) {
+    const Variant &a = kVariants[f], &b = kVariants[v];
+    if (a.tstack == b.tstack && (any ? a.any == b.any : a.closest == b.closest)) return f;
+  }
+  return v;
+}
+
 uint32_t trace_grid_blocks(int device, int v, bool any) {
   int cus = 0, per = 0;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
