@@ -169,7 +169,7 @@ def cfg_arg(t) -> str | None:
 # ------------------------------------------------------- rocprofv3 counters
 COPY_PROBE_BYTES = 1 << 30
 KERNEL_SYMBOL = {"trace_closest": "k_trace<false, false", "trace_any": "k_trace<true, false",
-                 "batch_build": "KernelMode)0", "batch_trace": "KernelMode)1"}
+                 "batch_build": "k_batch_", "batch_trace": "k_batch_trace<"}
 COPY_SYMBOL = "k_copy16"
 # Three passes: HBM bytes read, HBM bytes written, and the issue / cache counters
 # (at most 4 TCC, 8 SQ and 2 GRBM counters per pass).
@@ -239,9 +239,14 @@ def _pmc_run(counters: str, config: str, extra: list) -> dict | None:
 
 
 def _pick(per_kernel: dict, sym: str):
-    """The mean of the most-dispatched kernel whose name contains sym."""
-    hits = [(n, v) for k, (v, n) in per_kernel.items() if sym in k]
-    return max(hits)[1] if hits else None
+    """The mean of the most-dispatched kernel whose name contains sym; for a batch's
+    build the sum over its phases' kernels (each is dispatched once a run)."""
+    build = sym == KERNEL_SYMBOL["batch_build"]
+    hits = [(n, v) for k, (v, n) in per_kernel.items()
+            if sym in k and not (build and KERNEL_SYMBOL["batch_trace"] in k)]
+    if not hits:
+        return None
+    return sum(v for _, v in hits) if build else max(hits)[1]
 
 
 def measure_pmc(config: str, kernels, trace_cfg: str | None) -> dict:
