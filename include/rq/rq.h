@@ -254,9 +254,10 @@ int rq_trace_refill_set(rq_ctx* ctx, uint32_t closest_refill, uint32_t any_refil
 int rq_trace_refill_get(rq_ctx* ctx, uint32_t* closest_refill, uint32_t* any_refill);
 /* Largest wave slice per query kind: the persistent waves take rays from the
  * launch's ray stream in slices of this many (a power of two, 64..4096;
- * default 1024), halved for launches too small to give every wave two, and a
- * quarter as many over the stream's last quarter. Larger slices cost fewer
- * atomics, smaller ones keep the rays in flight closer together. */
+ * default 1024), halved (to 64 at least) until every wave gets eight, and a
+ * quarter as many over the stream's last quarter; a launch too small to give
+ * every wave 64 rays gives each 2 to 16. Larger slices cost fewer atomics,
+ * smaller ones keep the rays in flight closer together. */
 int rq_trace_slice_set(rq_ctx* ctx, uint32_t closest_slice, uint32_t any_slice);
 int rq_trace_slice_get(rq_ctx* ctx, uint32_t* closest_slice, uint32_t* any_slice);
 /* Times every variant (of those that run the same kernel, as 14 and 17 do, the

@@ -145,12 +145,12 @@ __device__ inline void centroids(const BuildView& v, uint32_t t, uint32_t end, f
 }
 
 // ---- phase 1: centroid bounds of one tile (SCENE_AABB map) ------------------------
-template <int BLOCK = BUILD_BLOCK, int TILE = TRI_TILE>
+template <int BLOCK = BUILD_BLOCK>
 __device__ inline void bounds_tile(const BuildView& v, uint32_t tile, uint32_t* lds) {
   constexpr int W = BLOCK / 64;  // waves; lds holds 6 * W words
   uint32_t lo[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, hi[3] = {0u, 0u, 0u};
-  const uint32_t end = min((tile + 1) * (uint32_t)TILE, v.n);
-  for (uint32_t t = tile * TILE + threadIdx.x; t < end; t += CENTROIDS * BLOCK) {
+  const uint32_t end = min((tile + 1) * (uint32_t)TRI_TILE, v.n);
+  for (uint32_t t = tile * TRI_TILE + threadIdx.x; t < end; t += CENTROIDS * BLOCK) {
     float3 c[CENTROIDS];
     centroids<BLOCK>(v, t, end, c);  // (a clamped index repeats one: no harm)
 #pragma unroll

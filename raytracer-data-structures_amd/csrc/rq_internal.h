@@ -126,7 +126,7 @@ __host__ __device__ inline uint32_t trace_chunk(uint32_t n, uint32_t waves,
 // Rays per wave of a launch too small to give every wave 64 (`waves`: the
 // waves the chip holds): two, or the power of two above that at which all have
 // a wave; the idle lanes share the rays' walks (SplitSlots in trace_device.h).
-// 64: full waves. 16 k rays, 500 spheres: 295 us at 64 a wave, 255 of them
+// 64: full waves. 16 k rays, 35,947 spheres: 295 us at 64 a wave, 255 of them
 // shared, 93 / 64 / 46 at 8 / 4 / 2; 65 k rays, 1.3 M triangles: 523, 464,
 // 449 / 440 / 426 at 32 / 16 / 8. One ray a wave gains nothing over two: 4 k
 // rays 139 us against 137, 7 k short ones 32 against 28 (a wave costs its
